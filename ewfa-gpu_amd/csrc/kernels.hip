@@ -151,16 +151,77 @@ __device__ __forceinline__ void stage_overlapped(uint64_t* S, const uint64_t* g,
     }
 }
 
+// Adds n to a work counter and returns its old value; with an `end`, a counter
+// that has passed it is only read (one thread's call).
+constexpr uint32_t NO_LOOK = 0xFFFFFFFFu;
+__device__ __forceinline__ uint32_t counter_take(uint32_t* counter, uint32_t n, uint32_t end) {
+    if (end != NO_LOOK) {
+        const uint32_t now = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (now >= end) return now;
+    }
+    return atomicAdd(counter, n);
+}
+
 // A wave's next work item from a counter: lane 0 adds n, every lane gets the
 // old value.  The wave barrier joins the lanes' paths first: without it the
 // compiler may thread a branch on the lane elsewhere in the caller's loop
 // (`if (lane == 0) store`) past the add, into a loop of lanes 1..63 alone
 // that reads the counter's value from a lane that never adds.
-__device__ __forceinline__ uint32_t wave_take(uint32_t* counter, uint32_t n, int lane) {
+__device__ __forceinline__ uint32_t wave_take(uint32_t* counter, uint32_t n, int lane, uint32_t end = NO_LOOK) {
     __builtin_amdgcn_wave_barrier();
     uint32_t b = 0;
-    if (lane == 0) b = atomicAdd(counter, n);
+    if (lane == 0) b = counter_take(counter, n, end);
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+}
+
+// Items per queue pull: the policy's grab while every block gets at least two
+// pulls of it, fewer when the list is short, so that 10,000 pairs under a
+// grab of 16 spread over the whole grid instead of 625 blocks of 16 in turn
+// (150 bp pairs: 149 -> 36 us with the counters' changes in for_shares).
+__device__ __forceinline__ uint32_t grab_for(uint32_t most, uint32_t count) {
+    return max(min(most, count / (2u * gridDim.x)), 1u);
+}
+
+// The same where a block's first items are its own (for_shares): a list of
+// at most two items per block is all first items.
+__device__ __forceinline__ uint32_t grab_own(uint32_t most, uint32_t count) {
+    const uint32_t own = max(gridDim.x / (uint32_t)XCDS, 1u);  // blocks of a share
+    const uint32_t per = (count / (uint32_t)XCDS + own) / own;
+    return per <= 2u ? per : grab_for(most, count);
+}
+
+// The list of `count` items in XCDS contiguous shares: a block works its own
+// XCD's share first, then helps the others in turn, so neighbouring pairs
+// (whose descriptors and packed words share cache lines) mostly go through
+// one XCD's L2.  take(q, end) hands out the next items of share q; with
+// an end (a share of another XCD, most likely used up), the counter is read
+// before it is added to (every block asks the seven other shares at its end: 8,192
+// blocks adding to 8 counters were 80 us of such a launch).
+// OWN_FIRST (passes of short items): each block's first `grab` items of its
+// share are its own without a counter, and a share that its own blocks' first
+// items cover is never asked for, so a list of at most grid x grab items
+// takes no atomic at all.  Passes of long items go without: a block that finds
+// its CU late, behind another pass, would start its item late.
+template <bool OWN_FIRST, typename Take, typename Run>
+__device__ __forceinline__ void for_shares(uint32_t count, uint32_t grab, const Take& take, const Run& run) {
+    const uint32_t home = blockIdx.x % (uint32_t)XCDS;
+    for (uint32_t r = 0; r < (uint32_t)XCDS; ++r) {
+        const uint32_t q = (home + r) % (uint32_t)XCDS;
+        const uint32_t lo = (uint32_t)(((uint64_t)count * q) / XCDS);
+        const uint32_t hi = (uint32_t)(((uint64_t)count * (q + 1)) / XCDS);
+        const uint32_t len = hi - lo;
+        // items of the share that its own blocks (q, q + XCDS, ...) take
+        // unasked (grab is at most 2 or count / (2 x grid), so the products
+        // stay within 32 bits)
+        const uint32_t first =
+            OWN_FIRST ? min((gridDim.x + (uint32_t)XCDS - 1u - q) / (uint32_t)XCDS * grab, len) : 0u;
+        const auto next = [&]() { return first < len ? first + take(q, r ? len - first : NO_LOOK) : len; };
+        uint32_t got = OWN_FIRST && r == 0 ? blockIdx.x / (uint32_t)XCDS * grab : next();
+        while (got < len) {
+            run(lo + got, min(lo + got + grab, hi));
+            got = next();
+        }
+    }
 }
 
 // Synchronisation of the threads working on one pair.
@@ -1371,28 +1432,17 @@ __global__ __launch_bounds__(64, NC <= 3 ? 8 : 6) void align_reg_kernel(AlignArg
             pidx = nidx;
         }
     };
+    const uint32_t grab = grab_own(a.grab, count);
     if (a.xqueue) {
-        // the list in XCDS contiguous shares, share q handed out by counter
-        // q: a block takes its own XCD's share first, then helps the others
-        // in turn, so neighbouring pairs (whose descriptors and packed words
-        // share cache lines) mostly go through one XCD's L2
-        const uint32_t home = blockIdx.x % (uint32_t)XCDS;
-        for (uint32_t r = 0; r < (uint32_t)XCDS; ++r) {
-            const uint32_t q = (home + r) % (uint32_t)XCDS;
-            const uint32_t lo = (uint32_t)(((uint64_t)count * q) / XCDS);
-            const uint32_t hi = (uint32_t)(((uint64_t)count * (q + 1)) / XCDS);
-            for (;;) {
-                const uint32_t got = wave_take(a.xqueue + q * XQ_STRIDE, a.grab, lane);
-                if (got >= hi - lo) break;
-                run(lo + got, min(lo + got + a.grab, hi));
-            }
-        }
+        for_shares<true>(count, grab, [&](uint32_t q, uint32_t end) {
+            return wave_take(a.xqueue + q * XQ_STRIDE, grab, lane, end);
+        }, run);
         return;
     }
     for (;;) {
-        const uint32_t base = wave_take(a.queue, a.grab, lane);
+        const uint32_t base = wave_take(a.queue, grab, lane);
         if (base >= count) break;
-        run(base, min(base + a.grab, count));
+        run(base, min(base + grab, count));
     }
 }
 
@@ -1416,12 +1466,13 @@ __global__ __launch_bounds__(64 * G) void align_kernel(AlignArgs a, int persiste
         return;
     }
     if (count == 0) return;  // as in align_reg_kernel
+    const uint32_t grab = grab_for(a.grab, count);
     // `grab` items from a work counter, the value seen by the whole group
-    const auto take = [&](uint32_t* counter) -> uint32_t {
+    const auto take = [&](uint32_t* counter, uint32_t end) -> uint32_t {
         if constexpr (G == 1) {
-            return wave_take(counter, a.grab, tid);
+            return wave_take(counter, grab, tid, end);
         } else {
-            if (tid == 0) s_base = atomicAdd(counter, a.grab);
+            if (tid == 0) s_base = counter_take(counter, grab, end);
             __syncthreads();
             const uint32_t b = s_base;
             __syncthreads();
@@ -1434,24 +1485,16 @@ __global__ __launch_bounds__(64 * G) void align_kernel(AlignArgs a, int persiste
             group_sync<G>();  // the slot is reused by the next pair
         }
     };
-    if (a.xqueue) {  // per-XCD shares, as in align_reg_kernel
-        const uint32_t home = blockIdx.x % (uint32_t)XCDS;
-        for (uint32_t r = 0; r < (uint32_t)XCDS; ++r) {
-            const uint32_t q = (home + r) % (uint32_t)XCDS;
-            const uint32_t lo = (uint32_t)(((uint64_t)count * q) / XCDS);
-            const uint32_t hi = (uint32_t)(((uint64_t)count * (q + 1)) / XCDS);
-            for (;;) {
-                const uint32_t got = take(a.xqueue + q * XQ_STRIDE);
-                if (got >= hi - lo) break;
-                run(lo + got, min(lo + got + a.grab, hi));
-            }
-        }
+    if (a.xqueue) {
+        for_shares<false>(count, grab, [&](uint32_t q, uint32_t end) {
+            return take(a.xqueue + q * XQ_STRIDE, end);
+        }, run);
         return;
     }
     for (;;) {
-        const uint32_t base = take(a.queue);
+        const uint32_t base = take(a.queue, NO_LOOK);
         if (base >= count) break;
-        run(base, min(base + a.grab, count));
+        run(base, min(base + grab, count));
     }
 }
 
