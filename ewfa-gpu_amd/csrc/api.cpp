@@ -102,16 +102,14 @@ struct ewfa_ctx {
     float align_ms = 0.f, emit_ms = 0.f;
     bool timing = false;
     // graph cache for the persistent path
-    hipGraphExec_t graph = nullptr, graph2 = nullptr;  // graph2: emit part when timed
+    hipGraphExec_t graph = nullptr;  // the plan up to its published counts
     struct Key {
         const void *words, *pairs, *results, *cigars, *ops;
         size_t n;
         uint32_t max_len;
-        bool timing;
         bool operator==(const Key& o) const {
             return words == o.words && pairs == o.pairs && results == o.results &&
-                   cigars == o.cigars && ops == o.ops && n == o.n && max_len == o.max_len &&
-                   timing == o.timing;
+                   cigars == o.cigars && ops == o.ops && n == o.n && max_len == o.max_len;
         }
     } graph_key{};
     bool use_graph = true;
@@ -462,6 +460,17 @@ void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t n, Chain& 
 
 int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
     pl = Plan{};
+    if (n <= (uint32_t)c->num_cus && max_len > c->policy.buckets.front().len_hi) {
+        // at most a pair per CU: the call lasts as long as its longest pair,
+        // so all go through that pair's pass, without bucketing and the fork
+        // over streams (60 pairs of 100..2,000 bp: 175 -> 130 us)
+        pl.nb = 1;
+        pl.blen[0] = max_len;
+        CHK(pass_from_bucket(c, c->policy.bucket_for(max_len), max_len, n, pl.pass[0]));
+        plan_chain(c, max_len, pl.pass[0].dcap, n, pl.chain);
+        assign_slots(pl);
+        return EWFA_OK;
+    }
     for (const ewfa::BucketPolicy& b : c->policy.buckets) {
         if (pl.nb == ewfa::MAX_BUCKETS) break;
         pl.table.hi[pl.nb] = b.len_hi;
@@ -719,6 +728,7 @@ int enqueue_main(ewfa_ctx* c, const Pass& p, const uint64_t* words, const ewfa_p
 // first), the emit per bucket, and the deferred count's copy to the host.
 // The deferral chain of a plan, then the marking of pairs no pass could
 // resolve.
+// n bounds the deferred pairs.
 int enqueue_chain(ewfa_ctx* c, const Chain& ch, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t n,
                   uint32_t max_len, ewfa_result_t* results, int8_t* cigars, hipStream_t s) {
     const ewfa::Scratch sx = scratch_of(c);
@@ -727,7 +737,8 @@ int enqueue_chain(ewfa_ctx* c, const Chain& ch, const uint64_t* words, const ewf
     const int ctr[2] = {CTRL_DEFER_A, CTRL_DEFER_B};
     int cur = 0;
     for (int k = 0; k < ch.np; ++k) {
-        const Pass& p = ch.pass[k];
+        Pass p = ch.pass[k];
+        p.grid = std::min(p.grid, n);
         // the pass's queue head, the count of the list it defers into and
         // its bounds' work counter start at zero (one launch)
         HIPCHK(ewfa::launch_clear_words(
@@ -760,8 +771,11 @@ int enqueue_chain(ewfa_ctx* c, const Chain& ch, const uint64_t* words, const ewf
 }
 
 // phase: PLAN_ALL, or PLAN_ALIGN (bucketing, the bucket passes and the emits
-// of the block buckets) then PLAN_EMIT (the fused passes' fallback emit and
-// the deferral chain) as two graphs timed between their launches.
+// of the block buckets), after which a call that waits for its results reads
+// whether anything is left for PLAN_EMIT (the fused passes' fallback emit and
+// the deferral chain): most calls defer nothing, and the chain's empty
+// launches (2 to 17 of them, about 4.5 us each) were up to half of a small
+// call.
 enum { PLAN_ALL = 3, PLAN_ALIGN = 1, PLAN_EMIT = 2 };
 
 // The streams (and join events) a plan's bucket passes fan out over beyond
@@ -784,7 +798,7 @@ int ensure_aux(ewfa_ctx* c, int F) {
 
 int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t n,
                  uint32_t max_len, ewfa_result_t* results, int8_t* cigars, hipStream_t s, bool timing,
-                 int phase = PLAN_ALL) {
+                 int phase = PLAN_ALL, uint32_t fallbacks = 0xFFFFFFFFu, uint32_t deferred = 0xFFFFFFFFu) {
     const ewfa::Scratch sx = scratch_of(c);
     uint32_t* ctrl = sx.ctrl;
     uint32_t* lists = sx.buckets;
@@ -856,8 +870,11 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
         }
         if (timing) HIPCHK(hipEventRecord(c->ev_a1, s));
     }
+    if (phase == PLAN_ALIGN)
+        HIPCHK(ewfa::launch_publish_counts(ctrl + CTRL_DEFER_A, ctrl + CTRL_FALLBACK, c->host_ctrl + CTRL_DEFER_A,
+                                           c->host_ctrl + CTRL_FALLBACK, s));
     if (!(phase & PLAN_EMIT)) return EWFA_OK;
-    if (fused) {
+    if (fused && fallbacks > 0) {
         // paths with a match run of 255 bases or more go through the emit kernel
         ewfa::EmitArgs e{};
         e.words = words;
@@ -867,11 +884,12 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
         e.ops_stride = ewfa::ops_words(max_len + 1);
         e.cigars = cigars;
         e.list = sx.list_fb;
-        e.count = n;
+        e.count = std::min(n, fallbacks);
         e.count_ptr = ctrl + CTRL_FALLBACK;
-        CHK(emit_list(c, e, n, max_len, s));
+        CHK(emit_list(c, e, e.count, max_len, s));
     }
-    CHK(enqueue_chain(c, pl.chain, words, pairs, n, max_len, results, cigars, s));
+    if (deferred > 0)
+        CHK(enqueue_chain(c, pl.chain, words, pairs, std::min(n, deferred), max_len, results, cigars, s));
     if (timing) HIPCHK(hipEventRecord(c->ev_e1, s));
     return EWFA_OK;
 }
@@ -1432,7 +1450,6 @@ int ewfa_destroy(ewfa_ctx_t* c) {
     for (hipEvent_t e : c->ev_words) (void)hipEventDestroy(e);
     release_retired(c);
     if (c->graph) (void)hipGraphExecDestroy(c->graph);
-    if (c->graph2) (void)hipGraphExecDestroy(c->graph2);
     for (hipEvent_t e : {c->ev_in, c->ev_a0, c->ev_a1, c->ev_e1, c->ev_fork})
         if (e) (void)hipEventDestroy(e);
     for (int i = 0; i < ewfa_ctx::MAX_FANOUT - 1; ++i) {
@@ -1585,65 +1602,54 @@ int ewfa_align_device(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t*
         CHK(reserve_plan(c, pl, n));
         CHK(ensure_aux(c, pl.fanout));  // not while a graph is being captured
         const bool timing = c->timing;
-        ewfa_ctx::Key key{d_words, d_pairs, d_results, d_cigars, ops_base(c), n, max_len, timing};
-        if (c->use_graph) {
-            // with timing: two graphs (align, emit) with events between them
-            const int nparts = timing ? 2 : 1;
-            const uint64_t gen = c->buffer_gen;
-            if (!(c->graph && c->graph_key == key && c->graph_policy_gen == c->policy_gen &&
-                  c->graph_buffer_gen == gen)) {
-                for (hipGraphExec_t* ge : {&c->graph, &c->graph2})
-                    if (*ge) {
-                        (void)hipGraphExecDestroy(*ge);
-                        *ge = nullptr;
-                    }
-                for (int part = 0; part < nparts; ++part) {
-                    const int phase = timing ? (part == 0 ? PLAN_ALIGN : PLAN_EMIT) : PLAN_ALL;
-                    hipGraph_t g = nullptr;
-                    HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                    int rc = enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s,
-                                          false, phase);
-                    hipError_t ce = hipStreamEndCapture(s, &g);
-                    if (rc != EWFA_OK) {
-                        if (g) (void)hipGraphDestroy(g);
-                        return rc;
-                    }
-                    if (ce != hipSuccess) return fail(EWFA_ERR_HIP, "graph capture: %s", hipGetErrorString(ce));
-                    hipGraphExec_t* ge = part == 0 ? &c->graph : &c->graph2;
-                    hipError_t ie = hipGraphInstantiate(ge, g, nullptr, nullptr, 0);
-                    (void)hipGraphDestroy(g);
-                    if (ie != hipSuccess) {
-                        *ge = nullptr;
-                        return fail(EWFA_ERR_HIP, "graph instantiate: %s", hipGetErrorString(ie));
-                    }
-                }
-                c->graph_key = key;
-                c->graph_policy_gen = c->policy_gen;
-                c->graph_buffer_gen = gen;
+        ewfa_ctx::Key key{d_words, d_pairs, d_results, d_cigars, ops_base(c), n, max_len};
+        const uint64_t gen = c->buffer_gen;
+        // a single pass is three launches: enqueued as they are they take less
+        // than a replay (one pair 43 -> 36 us), and new buffers or another
+        // count need no capture (100 us and more)
+        const bool use_graph = c->use_graph && pl.nb > 1;
+        if (use_graph && !(c->graph && c->graph_key == key && c->graph_policy_gen == c->policy_gen &&
+                              c->graph_buffer_gen == gen)) {
+            if (c->graph) (void)hipGraphExecDestroy(c->graph);
+            c->graph = nullptr;
+            hipGraph_t g = nullptr;
+            HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+            int rc = enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s, false,
+                                  PLAN_ALIGN);
+            hipError_t ce = hipStreamEndCapture(s, &g);
+            if (rc != EWFA_OK) {
+                if (g) (void)hipGraphDestroy(g);
+                return rc;
             }
-            if (timing) {
-                HIPCHK(hipEventRecord(c->ev_a0, s));
-                HIPCHK(hipGraphLaunch(c->graph, s));
-                HIPCHK(hipEventRecord(c->ev_a1, s));
-                HIPCHK(hipGraphLaunch(c->graph2, s));
-                HIPCHK(hipEventRecord(c->ev_e1, s));
-            } else {
-                HIPCHK(hipGraphLaunch(c->graph, s));
+            if (ce != hipSuccess) return fail(EWFA_ERR_HIP, "graph capture: %s", hipGetErrorString(ce));
+            hipError_t ie = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(g);
+            if (ie != hipSuccess) {
+                c->graph = nullptr;
+                return fail(EWFA_ERR_HIP, "graph instantiate: %s", hipGetErrorString(ie));
             }
-            HIPCHK(hipStreamSynchronize(s));
-            if (timing) {
-                float ms = 0.f;
-                if (hipEventElapsedTime(&ms, c->ev_a0, c->ev_a1) == hipSuccess) c->align_ms = ms;
-                if (hipEventElapsedTime(&ms, c->ev_a1, c->ev_e1) == hipSuccess) c->emit_ms = ms;
-            }
-        } else {
-            CHK(enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s, timing));
-            HIPCHK(hipStreamSynchronize(s));
-            if (timing) {
-                float ms = 0.f;
-                if (hipEventElapsedTime(&ms, c->ev_a0, c->ev_a1) == hipSuccess) c->align_ms = ms;
-                if (hipEventElapsedTime(&ms, c->ev_a1, c->ev_e1) == hipSuccess) c->emit_ms = ms;
-            }
+            c->graph_key = key;
+            c->graph_policy_gen = c->policy_gen;
+            c->graph_buffer_gen = gen;
+        }
+        if (timing) HIPCHK(hipEventRecord(c->ev_a0, s));
+        if (use_graph)
+            HIPCHK(hipGraphLaunch(c->graph, s));
+        else
+            CHK(enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s, false,
+                             PLAN_ALIGN));
+        if (timing) HIPCHK(hipEventRecord(c->ev_a1, s));
+        HIPCHK(hipStreamSynchronize(s));
+        const uint32_t deferred = c->host_ctrl[CTRL_DEFER_A], fallbacks = c->host_ctrl[CTRL_FALLBACK];
+        if (deferred || fallbacks)
+            CHK(enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s, false, PLAN_EMIT,
+                             fallbacks, deferred));
+        if (timing) HIPCHK(hipEventRecord(c->ev_e1, s));
+        if (deferred || fallbacks || timing) HIPCHK(hipStreamSynchronize(s));
+        if (timing) {
+            float ms = 0.f;
+            if (hipEventElapsedTime(&ms, c->ev_a0, c->ev_a1) == hipSuccess) c->align_ms = ms;
+            if (hipEventElapsedTime(&ms, c->ev_a1, c->ev_e1) == hipSuccess) c->emit_ms = ms;
         }
         return EWFA_OK;
     }

@@ -2180,6 +2180,16 @@ __global__ __launch_bounds__(64) void clear_words_kernel(uint32_t* p, uint64_t m
     if ((mask >> i) & 1u) p[i] = 0u;
 }
 
+// The deferred and fallback counts of a plan's bucket passes into host
+// memory, for the call to see whether anything is left to enqueue.
+__global__ __launch_bounds__(64) void publish_counts_kernel(const uint32_t* defer, const uint32_t* fallback,
+                                                            uint32_t* host_defer, uint32_t* host_fallback) {
+    if (threadIdx.x == 0) {
+        *host_defer = *defer;
+        *host_fallback = *fallback;
+    }
+}
+
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, uint32_t value, size_t n) {
     const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
     if (i < n) p[i] = value;
@@ -2401,6 +2411,13 @@ hipError_t launch_compact(const ewfa_pair_t* pairs, const ewfa_result_t* results
 hipError_t launch_clear_words(uint32_t* p, uint64_t mask, hipStream_t stream) {
     if (mask == 0) return hipSuccess;
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(64), 0, stream, p, mask);
+    return hipGetLastError();
+}
+
+hipError_t launch_publish_counts(const uint32_t* defer, const uint32_t* fallback, uint32_t* host_defer,
+                                 uint32_t* host_fallback, hipStream_t stream) {
+    hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(64), 0, stream, defer, fallback, host_defer,
+                       host_fallback);
     return hipGetLastError();
 }
 
