@@ -673,6 +673,9 @@ int emit_list(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max
 }
 
 int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, bool staged, hipStream_t s) {
+    // few pairs: a wave each, whose walk takes a tenth of a lane's (a lane's
+    // steps wait for memory; large lists hide that over many pairs)
+    if (staged && items <= (uint32_t)c->num_cus * 4u) return emit_list(c, e, items, max_len, s);
     const int sw = seq_words_for(max_len);
     if (staged && sw <= ewfa::EMIT_LDS_MAX_SW)
         HIPCHK(ewfa::launch_emit_lds(e, items, sw, s));
