@@ -76,7 +76,14 @@ enum : int {
     CTRL_BCOUNT = 16,   // pairs per bucket (MAX_BUCKETS)
     CTRL_BOUNDQ = 24,   // work counters of the bucket passes' distance bounds (MAX_BUCKETS)
     CTRL_XQ = 64,       // per-XCD work counters of the bucket passes (MAX_BUCKETS x XCDS, strided)
-    CTRL_WORDS = CTRL_XQ + ewfa::MAX_BUCKETS * ewfa::XCDS * ewfa::XQ_STRIDE
+    // per bucket: the bit-parallel sort's bins and cursors, the classes' places,
+    // the count of pairs left to the wavefront and the pass's work counter
+    CTRL_BP = CTRL_XQ + ewfa::MAX_BUCKETS * ewfa::XCDS * ewfa::XQ_STRIDE,
+    BP_SEG = 2 * ewfa::BP_BINS,
+    BP_REST = BP_SEG + ewfa::BP_CLASSES + 1,
+    BP_QUEUE = BP_REST + 1,
+    BP_CTRL = (BP_QUEUE + 32) & ~31,
+    CTRL_WORDS = CTRL_BP + ewfa::MAX_BUCKETS * BP_CTRL
 };
 
 }  // namespace
@@ -98,6 +105,7 @@ struct ewfa_ctx {
     int num_cus = 0;
     size_t lds_max = 0;
     DevBuf ops, bt, ctrl, list_a, list_b, buckets, runs, list_fb, bound, gslot, order;
+    DevBuf bp_list, bp_rest, bp_slots;  // bit-parallel passes
     uint32_t* host_ctrl = nullptr;  // pinned mirror of the control words
     float align_ms = 0.f, emit_ms = 0.f;
     bool timing = false;
@@ -216,6 +224,9 @@ struct Pass {
     int gslot;          // 1: the block's slot (sequence copies, offsets) in HBM
     size_t gslot_bytes; // bytes of one such slot
     size_t gslot_off;   // byte offset of the pass's HBM slots
+    // the bit-parallel pass ahead of a bounded bucket pass (0 blocks: none)
+    uint32_t bp_grid;
+    size_t bp_slot_bytes, bp_off;
 };
 
 // Passes whose wavefront LDS cannot hold keep their slots in HBM.  Their
@@ -289,6 +300,24 @@ void choose_band_cap(ewfa_ctx* c, Pass& p) {
     p.band_cap = std::min(cap, p.dcap);
 }
 
+// Bytes of slots a bit-parallel pass may hold: at 50 kbp (4.1 MB a slot) three
+// waves per SIMD.
+constexpr size_t BP_BUDGET = (size_t)12 << 30;
+
+// The bit-parallel pass of a bucket pass with bounds: it takes the pairs for
+// which it is the cheaper way (bp_class_of).  Not under a distance cap, whose
+// output is the wavefront's at the capped level.
+void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
+    p.bp_grid = 0;
+    p.bp_slot_bytes = 0;
+    if (p.reg || p.gslot || p.bt_lds || p.off16 || p.dcap < BOUND_MIN_DCAP || c->opts.max_distance > 0) return;
+    if (p.seq_words > ewfa::BOUND_MAX_SEQ_WORDS) return;
+    p.bp_slot_bytes = ewfa::bp_tok_bytes() + ewfa::bp_rec_bytes(blen);
+    const uint64_t room = std::max<size_t>(BP_BUDGET / p.bp_slot_bytes, 1);
+    const uint64_t most = (uint64_t)std::max(ewfa::bp_blocks_per_cu(), 1) * (uint64_t)c->num_cus;
+    p.bp_grid = (uint32_t)std::min<uint64_t>({room, most, std::max<uint32_t>(items, 1u)});
+}
+
 int finish_pass(ewfa_ctx* c, Pass& p, uint32_t items) {
     if (p.gslot) {
         // slot in HBM, no dynamic LDS; blocks bounded by occupancy and memory
@@ -357,6 +386,7 @@ int pass_from_bucket(ewfa_ctx* c, const ewfa::BucketPolicy& b, uint32_t blen, ui
     }
     choose_off16(p, blen);
     choose_band_cap(c, p);
+    choose_bp(c, p, blen, items);
     return finish_pass(c, p, items);
 }
 
@@ -402,6 +432,7 @@ struct Plan {
     int fanout = 1;
     size_t bt_bytes = 0, runs_bytes = 0;  // regions the plan's slots need
     size_t gslot_bytes = 0;               // HBM slots of the passes beyond LDS
+    size_t bp_bytes = 0;                  // slots of the bit-parallel passes
 };
 
 // Bytes of one block's slot in the backtrace region (block passes with the
@@ -434,6 +465,13 @@ void assign_slots(Plan& pl) {
         bt = std::max(bt, slot_bytes(p) * p.grid);
         if (p.gslot) gs = std::max(gs, p.gslot_bytes * p.grid);
     }
+    size_t bp = 0;
+    for (int b = 0; b < pl.nb; ++b) {
+        Pass& p = pl.pass[b];
+        p.bp_off = pl.fanout > 1 ? bp : 0;
+        bp = std::max(bp, p.bp_off + p.bp_slot_bytes * p.bp_grid);
+    }
+    pl.bp_bytes = bp;
     pl.bt_bytes = bt;
     pl.runs_bytes = runs;
     pl.gslot_bytes = gs;
@@ -585,6 +623,11 @@ int reserve_plan(ewfa_ctx* c, const Plan& pl, size_t n) {
     CHK(c->gslot.reserve(c, pl.gslot_bytes));
     if (pl.nb > 1) CHK(c->buckets.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
     CHK(c->bound.reserve(c, std::max<size_t>(n, 1) * 4));
+    if (pl.bp_bytes) {
+        CHK(c->bp_slots.reserve(c, pl.bp_bytes));
+        CHK(c->bp_list.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
+        CHK(c->bp_rest.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
+    }
     bool narrow = false;
     for (int b = 0; b < pl.nb; ++b) narrow = narrow || pl.pass[b].band_cap > 0;
     if (narrow) CHK(c->order.reserve(c, (size_t)std::max(pl.nb, 1) * std::max<size_t>(n, 1) * 4));
@@ -814,6 +857,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
     for (int b = 0; b < pl.nb; ++b) fused = fused || pl.pass[b].reg;
     if (phase & PLAN_ALIGN) {
         HIPCHK(ewfa::launch_fill_u32(ctrl, 0u, CTRL_XQ + (size_t)pl.nb * ewfa::XCDS * ewfa::XQ_STRIDE, s));
+        if (pl.bp_bytes) HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_BP, 0u, (size_t)pl.nb * BP_CTRL, s));
         if (bucketed) HIPCHK(ewfa::launch_bucketize(pairs, n, pl.table, lists, ctrl + CTRL_BCOUNT, s));
         if (timing) HIPCHK(hipEventRecord(c->ev_a0, s));
         if (F > 1) {
@@ -844,6 +888,35 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 a.fallback_count = ctrl + CTRL_FALLBACK;
             }
             CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
+            if (p.bp_grid && a.bound) {
+                // the bit-parallel pass takes its pairs, the rest stay
+                uint32_t* ctl = ctrl + CTRL_BP + (size_t)b * BP_CTRL;
+                ewfa::BpArgs x{};
+                x.words = words;
+                x.pairs = pairs;
+                x.results = results;
+                x.cigars = cigars;
+                x.max_len = pl.blen[b];
+                x.bound = a.bound;
+                x.bins = ctl;
+                x.cursors = ctl + ewfa::BP_BINS;
+                x.seg = ctl + BP_SEG;
+                x.list_out = c->bp_list.as<uint32_t>() + (size_t)b * n;
+                x.list = x.list_out;
+                x.rest = c->bp_rest.as<uint32_t>() + (size_t)b * n;
+                x.rest_count = ctl + BP_REST;
+                x.queue = ctl + BP_QUEUE;
+                x.defer_list = sx.list_a;
+                x.defer_count = ctrl + CTRL_DEFER_A;
+                x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;
+                x.slot_bytes = p.bp_slot_bytes;
+                x.tok_bytes = ewfa::bp_tok_bytes();
+                HIPCHK(ewfa::launch_bp_sort(x, a.list, a.count_ptr, n, q));
+                HIPCHK(ewfa::launch_bp(x, p.bp_grid, q));
+                a.list = x.rest;
+                a.count_ptr = x.rest_count;
+            }
+            const uint32_t* const emit_items = a.list;
             if (p.band_cap > 0 && a.bound && sx.order) {
                 // the pass takes its pairs by decreasing bound, share by share
                 uint32_t* ord = sx.order + (size_t)b * n;
@@ -861,9 +934,9 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 e.ops = ops_base(c);
                 e.ops_stride = ewfa::ops_words(max_len + 1);
                 e.cigars = cigars;
-                e.list = bucketed ? lists + (size_t)b * n : nullptr;
+                e.list = emit_items;
                 e.count = n;
-                e.count_ptr = bucketed ? ctrl + CTRL_BCOUNT + b : nullptr;
+                e.count_ptr = a.count_ptr;
                 CHK(emit(c, e, n, pl.blen[b], true, q));
             }
         }
@@ -1219,6 +1292,7 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
             break;
         }
     pl.fanout = 1;
+    for (int b = 0; b < pl.nb; ++b) pl.pass[b].bp_grid = 0;  // nor for bit-parallel slots
     assign_slots(pl);
     // per-pair buffers first, then one region for the passes' slots
     const auto r256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -1464,7 +1538,7 @@ int ewfa_destroy(ewfa_ctx_t* c) {
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     for (DevBuf* b : {&c->ops, &c->bt, &c->ctrl, &c->list_a, &c->list_b, &c->buckets, &c->runs, &c->list_fb, &c->bound,
-                      &c->gslot, &c->order, &c->h_words, &c->h_pairs, &c->h_results, &c->h_cigars, &c->dense, &c->scan})
+                      &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results, &c->h_cigars, &c->dense, &c->scan})
         b->release();
     if (c->host_ctrl) (void)hipHostFree(c->host_ctrl);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
@@ -1551,7 +1625,7 @@ int ewfa_context_memory(ewfa_ctx_t* c, size_t* bytes) {
     if (!c || !bytes) return fail(EWFA_ERR_ARG, "null argument");
     size_t b = 0;
     for (const DevBuf* d : {&c->ops, &c->bt, &c->ctrl, &c->list_a, &c->list_b, &c->buckets, &c->runs,
-                            &c->list_fb, &c->bound, &c->gslot, &c->order, &c->h_words, &c->h_pairs, &c->h_results,
+                            &c->list_fb, &c->bound, &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results,
                             &c->h_cigars, &c->dense, &c->scan})
         b += d->bytes;
     *bytes = b + c->retired_bytes;

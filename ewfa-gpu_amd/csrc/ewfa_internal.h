@@ -169,6 +169,64 @@ inline int reg_chunks_for(int dcap) {
 }
 
 
+// ---- bit-parallel passes (bitpar.hip) ----
+// Classes of pairs by the words of 32 diagonals their band holds, widest first.
+constexpr int BP_CLASSES = 6;
+__host__ __device__ inline int bp_words(int c) { return c == 0 ? 256 : c == 1 ? 192 : c == 2 ? 128 : c == 3 ? 64 : c == 4 ? 32 : 16; }
+// Pairs that share a wave, and a column's wave instructions per pair.
+__host__ __device__ inline uint32_t bp_pairs_per_wave(int c) { return c <= 3 ? 1u : c == 4 ? 2u : 4u; }
+__host__ __device__ inline float bp_column_cost(int c) {
+    return c == 0 ? 60.f : c == 1 ? 47.f : c == 2 ? 34.f : c == 3 ? 20.f : c == 4 ? 13.f : 6.5f;
+}
+constexpr int BP_LEN_BINS = 32;
+constexpr int BP_BINS = (BP_CLASSES + 1) * BP_LEN_BINS;
+
+// The band of N words for a pair of target diagonal tk: at column block j (columns
+// 32j..32j+31) it holds row words j + S .. j + S + N - 1, i.e. at every column the
+// diagonals -32b .. 32a with a = -S, b = N - 1 - a.  Returns the most edits L
+// whose every path it holds (floor((L+tk)/2) <= 32a, floor((L-tk)/2) <= 32b), -1
+// when it does not reach tk.
+__host__ __device__ inline int bp_band(int N, int tk, int& S) {
+    int a = ((N - 1) * 64 + 2 * tk + 64) >> 7;
+    a = a < 0 ? 0 : a > N - 1 ? N - 1 : a;
+    const int b = N - 1 - a;
+    const int up = 64 * a + 1 - tk, down = 64 * b + 1 + tk;
+    const int L = up < down ? up : down;
+    S = -a;
+    return L >= (tk < 0 ? -tk : tk) ? L : -1;
+}
+
+struct BpArgs {
+    const uint64_t* words;
+    const ewfa_pair_t* pairs;
+    ewfa_result_t* results;
+    int8_t* cigars;
+    uint32_t max_len;
+    const uint32_t* bound;    // per pair
+    uint32_t* bins;           // BP_BINS counts and BP_BINS cursors, zero at first
+    uint32_t* cursors;
+    uint32_t* seg;            // BP_CLASSES + 1 places in list
+    uint32_t* list_out;       // the sorted list, as written
+    const uint32_t* list;     // ... and as read
+    uint32_t* rest;           // pairs left to the wavefront, and their count
+    uint32_t* rest_count;
+    uint32_t* queue;          // work counter of the pass
+    uint32_t* defer_list;
+    uint32_t* defer_count;
+    uint8_t* slots;           // per block: tok_bytes of tokens, then the records
+    size_t slot_bytes, tok_bytes;
+};
+
+// Token bytes and record bytes of a slot for texts up to max_len bases.
+inline size_t bp_tok_bytes() { return 4u * (size_t)(64 * 256 + 128); }
+inline size_t bp_rec_bytes(uint32_t max_len) { return (size_t)(max_len / 32u + 1u) * 64u * 5u * 8u; }
+// Sorts a list's pairs by class (list null: the identity; count from *count_ptr
+// when not null).
+hipError_t launch_bp_sort(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
+                          hipStream_t stream);
+hipError_t launch_bp(const BpArgs& a, uint32_t grid, hipStream_t stream);
+int bp_blocks_per_cu();
+
 // Bytes of a pair's CIGAR region the emit kernel wrote: whole dwords from
 // cigar_off up to and including the terminator (or up to cigar_cap when the
 // stream filled or overflowed it); none when the emit did not run.

@@ -27,6 +27,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "device.h"
 #include "ewfa_internal.h"
 
 namespace ewfa {
@@ -36,14 +37,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // Word 3 of a raw byte buffer resource on gfx9 parts (32-bit data format, so
 // untyped accesses are in range; bounds checked against the record count).
 constexpr int BUF_DWORD3 = 0x00020000;
-
-// x with lane `lane` set to the uniform value v (v_writelane, whatever the
-// exec mask).  The lane select goes through M0: one instruction reads one
-// scalar register besides M0.
-__device__ __forceinline__ int writelane_i32(int x, int v, int lane) {
-    asm("v_writelane_b32 %0, %1, m0" : "+v"(x) : "s"(v), "{m0}"(lane));
-    return x;
-}
 
 // x with lane L (a constant) set to the uniform value v.
 template <int L>
@@ -151,29 +144,6 @@ __device__ __forceinline__ void stage_overlapped(uint64_t* S, const uint64_t* g,
     }
 }
 
-// Adds n to a work counter and returns its old value; with an `end`, a counter
-// that has passed it is only read (one thread's call).
-constexpr uint32_t NO_LOOK = 0xFFFFFFFFu;
-__device__ __forceinline__ uint32_t counter_take(uint32_t* counter, uint32_t n, uint32_t end) {
-    if (end != NO_LOOK) {
-        const uint32_t now = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (now >= end) return now;
-    }
-    return atomicAdd(counter, n);
-}
-
-// A wave's next work item from a counter: lane 0 adds n, every lane gets the
-// old value.  The wave barrier joins the lanes' paths first: without it the
-// compiler may thread a branch on the lane elsewhere in the caller's loop
-// (`if (lane == 0) store`) past the add, into a loop of lanes 1..63 alone
-// that reads the counter's value from a lane that never adds.
-__device__ __forceinline__ uint32_t wave_take(uint32_t* counter, uint32_t n, int lane, uint32_t end = NO_LOOK) {
-    __builtin_amdgcn_wave_barrier();
-    uint32_t b = 0;
-    if (lane == 0) b = counter_take(counter, n, end);
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
-}
-
 // Items per queue pull: the policy's grab while every block gets at least two
 // pulls of it, fewer when the list is short, so that 10,000 pairs under a
 // grab of 16 spread over the whole grid instead of 625 blocks of 16 in turn
@@ -224,18 +194,6 @@ __device__ __forceinline__ void for_shares(uint32_t count, uint32_t grab, const 
     }
 }
 
-// Synchronisation of the threads working on one pair.
-template <int G>
-__device__ __forceinline__ void group_sync() {
-    if constexpr (G == 1) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-        __syncthreads();
-    }
-}
-
 // ---------------------------------------------------------------------------
 // one pair
 
@@ -252,19 +210,6 @@ __device__ __forceinline__ int slot_bt_word(int seq_words, int dcap) {
 // top, i.e. in at most three consecutive 64-diagonal chunks.  The walk then
 // takes each op bit out of lane j with readlane (scalar work), from LDS or
 // HBM alike.
-// Inclusive prefix sum over the 64 lanes with DPP only: row shifts by 1, 2,
-// 4 and 8 within each row of 16 lanes, then lane 15 and lane 31 broadcast
-// into the rows above.  Every lane of the wave must take part.
-__device__ __forceinline__ int wave_incl_scan_i32(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
-    return x;
-}
-
 // Maximum of x over the 64 lanes (every lane takes part; x >= -1), by the
 // same DPP steps, read from lane 63.
 __device__ __forceinline__ int wave_max_i32(int x) {
