@@ -304,14 +304,25 @@ void choose_band_cap(ewfa_ctx* c, Pass& p) {
 // waves per SIMD.
 constexpr size_t BP_BUDGET = (size_t)12 << 30;
 
-// The bit-parallel pass of a bucket pass with bounds: it takes the pairs for
+// Pairs from which a list's distance bounds are searched a lane per pair
+// (bp_bound_kernel), below that a wave per pair: a lane's search lasts as long
+// as its pair's columns (0.4 ms at 5 kbp) whatever the count, which a small
+// call waits for.
+constexpr uint32_t LANE_BOUND_MIN = 8192;
+constexpr uint32_t BP_MIN_LEN = 2500;
+
+// The bit-parallel pass ahead of a block bucket pass: it takes the pairs for
 // which it is the cheaper way (bp_class_of).  Not under a distance cap, whose
 // output is the wavefront's at the capped level.
 void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     p.bp_grid = 0;
     p.bp_slot_bytes = 0;
-    if (p.reg || p.gslot || p.bt_lds || p.off16 || p.dcap < BOUND_MIN_DCAP || c->opts.max_distance > 0) return;
+    if (p.reg || p.gslot || p.bt_lds || c->opts.max_distance > 0) return;
     if (p.seq_words > ewfa::BOUND_MAX_SEQ_WORDS) return;
+    // passes without bounds of their own: only where the bounds are cheap, and
+    // from BP_MIN_LEN on (pairs of 1,200..2,500 bp at 1..10% edits lose more to
+    // the two passes ahead than they gain)
+    if (p.dcap < BOUND_MIN_DCAP && (items < LANE_BOUND_MIN || blen <= BP_MIN_LEN)) return;
     p.bp_slot_bytes = ewfa::bp_tok_bytes() + ewfa::bp_rec_bytes(blen);
     const uint64_t room = std::max<size_t>(BP_BUDGET / p.bp_slot_bytes, 1);
     const uint64_t most = (uint64_t)std::max(ewfa::bp_blocks_per_cu(), 1) * (uint64_t)c->num_cus;
@@ -887,8 +898,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 a.fallback_list = sx.list_fb;
                 a.fallback_count = ctrl + CTRL_FALLBACK;
             }
-            CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
-            if (p.bp_grid && a.bound) {
+            if (p.bp_grid) {
                 // the bit-parallel pass takes its pairs, the rest stay
                 uint32_t* ctl = ctrl + CTRL_BP + (size_t)b * BP_CTRL;
                 ewfa::BpArgs x{};
@@ -897,7 +907,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.results = results;
                 x.cigars = cigars;
                 x.max_len = pl.blen[b];
-                x.bound = a.bound;
+                x.bound = sx.bound;
                 x.bins = ctl;
                 x.cursors = ctl + ewfa::BP_BINS;
                 x.seg = ctl + BP_SEG;
@@ -911,10 +921,18 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;
                 x.slot_bytes = p.bp_slot_bytes;
                 x.tok_bytes = ewfa::bp_tok_bytes();
+                if (n >= LANE_BOUND_MIN) {
+                    HIPCHK(ewfa::launch_bp_bound(x, sx.bound, a.list, a.count_ptr, n, (uint32_t)c->num_cus * 16u, q));
+                    a.bound = p.dcap < BOUND_MIN_DCAP ? nullptr : sx.bound;
+                } else {
+                    CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
+                }
                 HIPCHK(ewfa::launch_bp_sort(x, a.list, a.count_ptr, n, q));
                 HIPCHK(ewfa::launch_bp(x, p.bp_grid, q));
                 a.list = x.rest;
                 a.count_ptr = x.rest_count;
+            } else {
+                CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
             }
             const uint32_t* const emit_items = a.list;
             if (p.band_cap > 0 && a.bound && sx.order) {

@@ -506,6 +506,135 @@ __global__ __launch_bounds__(64, 4) void bp_kernel(BpArgs a) {
     }
 }
 
+// ---- distance bounds ------------------------------------------------------------
+// An upper bound on each pair's distance from a window of 64 diagonals that
+// follows the path: the same table, one pair per lane, the window's vertical
+// deltas in a 64-bit word that moves down a row a column (so only the diagonal
+// term shifts).  Every 32 columns the window moves by up to BAND_MOVE rows
+// towards the edge with the smaller value.  Rows that enter it count +1 a row
+// from the ones it holds, so every value is that of a real alignment.
+// One lane per pair costs a sixth of the wave per pair of bound_kernel (a level
+// there keeps 64 lanes for some 5 cells that matter) but takes tlen columns of
+// about 80 ns however few pairs there are: it is for large lists.
+
+namespace {
+
+constexpr int BAND_MOVE = 12;
+
+struct LaneBand {
+    uint64_t vp, vn;
+    int sc;  // value of the row above the window's first
+    int r0;  // the window's first row (from 0) at the next column
+};
+
+// One column: p0, p1 the window's pattern planes, c0, c1 the text base's masks;
+// returns bit 0 of the diagonal-delta-0 vector (of the first row).
+__device__ __forceinline__ uint32_t band_column(LaneBand& b, uint64_t p0, uint64_t p1, uint64_t c0, uint64_t c1) {
+    const uint64_t eq = ~(p0 ^ c0) & ~(p1 ^ c1);
+    const uint64_t xh = (((eq & b.vp) + b.vp) ^ b.vp) | eq;
+    const uint64_t ph = b.vn | ~(xh | b.vp);
+    const uint64_t mh = b.vp & xh;
+    const uint64_t d0 = (uint64_t)((uint32_t)xh | (uint32_t)b.vn);
+    const uint64_t xv = (eq | b.vn) >> 1;
+    b.vp = mh | ~(xv | ph);
+    b.vn = ph & xv;
+    return (uint32_t)d0;
+}
+
+__device__ __forceinline__ uint64_t sign_mask(uint32_t planes, int i) {
+    const int m = (int)(planes << (31 - i)) >> 31;
+    return (uint64_t)(int64_t)m;
+}
+
+__device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen, int tlen) {
+    const int nwp = (plen + 31) >> 5;
+    LaneBand b{~0ull << 32, ~0ull >> 32, 32, -32};
+    uint32_t a[4], c[4];  // pattern planes from row r0 & ~31
+    const auto load = [&]() {
+        const int w = b.r0 >> 5;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) planes_of(gp[min(max(w + x, 0), nwp)], a[x], c[x]);
+        // ... moved so that bit 0 is row r0: 96 rows
+        const uint32_t sh = (uint32_t)b.r0 & 31u;
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            a[x] = __builtin_amdgcn_alignbit(a[x + 1], a[x], sh);
+            c[x] = __builtin_amdgcn_alignbit(c[x + 1], c[x], sh);
+        }
+    };
+    const auto window = [&](const uint32_t (&v)[4], int i) -> uint64_t {
+        return (uint64_t)__builtin_amdgcn_alignbit(v[1], v[0], (uint32_t)i) |
+               ((uint64_t)__builtin_amdgcn_alignbit(v[2], v[1], (uint32_t)i) << 32);
+    };
+    const int full = tlen >> 5;
+    for (int j = 0; j < full; ++j) {
+        uint32_t t0, t1;
+        load();
+        planes_of(gt[j], t0, t1);
+        uint32_t z = 0;
+#pragma unroll 16
+        for (int i = 0; i < 32; ++i) {
+            const uint32_t d0 = band_column(b, window(a, i), window(c, i), sign_mask(t0, i), sign_mask(t1, i));
+            z = __builtin_amdgcn_alignbit(d0, z, 1);
+        }
+        b.sc += 32 - __popc(z);
+        b.r0 += 32;
+        // bottom edge's value less the top edge's, halved: rows to move up
+        const int diff = __popcll(b.vp) - __popcll(b.vn);
+        const int up = min(max(diff / 2, -BAND_MOVE), BAND_MOVE);
+        if (up > 0) {
+            b.vp <<= up;
+            b.vn = (b.vn << up) | ((1ull << up) - 1ull);
+            b.sc += up;
+        } else if (up < 0) {
+            const uint64_t m = (1ull << -up) - 1ull;
+            b.sc += __popcll(b.vp & m) - __popcll(b.vn & m);
+            b.vp = (b.vp >> -up) | ~(~0ull >> -up);
+            b.vn >>= -up;
+        }
+        b.r0 -= up;
+    }
+    const int rest = tlen & 31;
+    if (rest) {
+        uint32_t t0, t1;
+        load();
+        planes_of(gt[full], t0, t1);
+        for (int i = 0; i < rest; ++i)
+            b.sc += 1 - (int)(band_column(b, window(a, i), window(c, i), sign_mask(t0, i), sign_mask(t1, i)) & 1u);
+        b.r0 += rest;
+    }
+    // row plen - 1 of the last column
+    const int idx = plen - b.r0;
+    if (idx <= 0) return (uint32_t)(b.sc - idx);
+    const uint64_t m = idx >= 64 ? ~0ull : (1ull << idx) - 1ull;
+    return (uint32_t)(b.sc + __popcll(b.vp & m) - __popcll(b.vn & m) + max(idx - 64, 0));
+}
+
+}  // namespace
+
+__global__ __launch_bounds__(64, 4) void bp_bound_kernel(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
+                                                         uint32_t* bound, const uint32_t* list,
+                                                         const uint32_t* count_ptr, uint32_t count) {
+    const uint32_t n = count_ptr ? *count_ptr : count;
+    for (uint32_t item = blockIdx.x * 64u + threadIdx.x; item < n; item += gridDim.x * 64u) {
+        const uint32_t pidx = list ? list[item] : item;
+        const ewfa_pair_t pr = pairs[pidx];
+        uint32_t u = BOUND_NONE;
+        if (pr.plen <= max_len && pr.tlen <= max_len)
+            u = lane_bound(words + pr.pattern_off, words + pr.text_off, (int)pr.plen, (int)pr.tlen);
+        bound[pidx] = u;
+    }
+}
+
+hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* list, const uint32_t* count_ptr,
+                           uint32_t count, uint32_t max_grid, hipStream_t stream) {
+    if (count == 0) return hipSuccess;
+    const uint32_t blocks = (count + 63u) / 64u;
+    hipLaunchKernelGGL(bp_bound_kernel, dim3(blocks < max_grid ? blocks : max_grid), dim3(64), 0, stream, a.words,
+                       a.pairs, a.max_len, bound, list, count_ptr, count);
+    return hipGetLastError();
+}
+
 // ---- which pairs come here -----------------------------------------------------
 
 namespace {
@@ -520,13 +649,21 @@ __device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& p
     for (int c = BP_CLASSES - 1; c >= 0; --c) {
         int S;
         if (bp_band(bp_words(c), tk, S) >= (int)u) {
-            // wave instructions of either way
-            const float wfa = 0.22f * (float)u * (float)u + 40.0f * (float)u;
+            // wave instructions of either way (the wavefront's weights fitted
+            // to calls: 500,000 pairs of 100..10,000 bp at 1..10% edits took 25.1,
+            // 20.6, 20.1 and 20.7 ms with 0.22, 0.5, 1 and 2 per u * u)
+            const float wfa = 0.6f * (float)u * (float)u + 100.0f * (float)u;
             const float bp = (float)pr.tlen * (bp_column_cost(c) + 4.0f) + 25.0f * (float)u;
             return wfa < bp ? BP_CLASSES : c;
         }
     }
-    return BP_CLASSES;
+    // A bound beyond the widest band mostly comes of a window that lost the
+    // path at a long gap (values then grow at the rate of unrelated sequences,
+    // several times that of 10..15% edits): the distance is likely within the
+    // band, and a pair whose is not has wasted little next to the wavefront
+    // passes it goes on to.
+    int S;
+    return bp_band(bp_words(0), tk, S) >= 0 ? 0 : BP_CLASSES;
 }
 
 // Bin of a pair in the sort: its class, then its length, longest first.

@@ -220,6 +220,9 @@ struct BpArgs {
 // Token bytes and record bytes of a slot for texts up to max_len bases.
 inline size_t bp_tok_bytes() { return 4u * (size_t)(64 * 256 + 128); }
 inline size_t bp_rec_bytes(uint32_t max_len) { return (size_t)(max_len / 32u + 1u) * 64u * 5u * 8u; }
+// Upper bounds on the distances of a list's pairs, a lane each.
+hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* list, const uint32_t* count_ptr,
+                           uint32_t count, uint32_t max_grid, hipStream_t stream);
 // Sorts a list's pairs by class (list null: the identity; count from *count_ptr
 // when not null).
 hipError_t launch_bp_sort(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
