@@ -82,7 +82,7 @@ enum : int {
     BP_SEG = 2 * ewfa::BP_BINS,
     BP_REST = BP_SEG + ewfa::BP_CLASSES + 1,
     BP_QUEUE = BP_REST + 1,
-    BP_CTRL = (BP_QUEUE + 32) & ~31,
+    BP_CTRL = (BP_QUEUE + 2 + 31) & ~31,
     CTRL_WORDS = CTRL_BP + ewfa::MAX_BUCKETS * BP_CTRL
 };
 
@@ -225,7 +225,8 @@ struct Pass {
     size_t gslot_bytes; // bytes of one such slot
     size_t gslot_off;   // byte offset of the pass's HBM slots
     // the bit-parallel pass ahead of a bounded bucket pass (0 blocks: none)
-    uint32_t bp_grid;
+    uint32_t bp_grid, bp_part[3];  // the most, and by part (BP_ALL, ..)
+    int bp_spread;
     size_t bp_slot_bytes, bp_off;
 };
 
@@ -302,7 +303,7 @@ void choose_band_cap(ewfa_ctx* c, Pass& p) {
 
 // Bytes of slots a bit-parallel pass may hold: at 50 kbp (4.1 MB a slot) three
 // waves per SIMD.
-constexpr size_t BP_BUDGET = (size_t)12 << 30;
+constexpr size_t BP_BUDGET = (size_t)20 << 30;
 
 // Pairs from which a list's distance bounds are searched a lane per pair
 // (bp_bound_kernel), below that a wave per pair: a lane's search lasts as long
@@ -310,6 +311,10 @@ constexpr size_t BP_BUDGET = (size_t)12 << 30;
 // call waits for.
 constexpr uint32_t LANE_BOUND_MIN = 8192;
 constexpr uint32_t BP_MIN_LEN = 2500;
+// Lists below this get twice the lanes per pair: eight pairs a wave would leave
+// SIMDs with less than two waves (15,001 pairs of 3..7 kbp: 4.0 -> 3.5 ms; 500,000
+// pairs of up to 10 kbp 17.5 -> 20.8 ms, so large lists keep the narrow groups).
+constexpr uint32_t BP_SPREAD_BELOW = 32768;
 
 // The bit-parallel pass ahead of a block bucket pass: it takes the pairs for
 // which it is the cheaper way (bp_class_of).  Not under a distance cap, whose
@@ -323,10 +328,17 @@ void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     // from BP_MIN_LEN on (pairs of 1,200..2,500 bp at 1..10% edits lose more to
     // the two passes ahead than they gain)
     if (p.dcap < BOUND_MIN_DCAP && (items < LANE_BOUND_MIN || blen <= BP_MIN_LEN)) return;
+    p.bp_spread = items < BP_SPREAD_BELOW ? 1 : 0;
     p.bp_slot_bytes = ewfa::bp_tok_bytes() + ewfa::bp_rec_bytes(blen);
     const uint64_t room = std::max<size_t>(BP_BUDGET / p.bp_slot_bytes, 1);
-    const uint64_t most = (uint64_t)std::max(ewfa::bp_blocks_per_cu(), 1) * (uint64_t)c->num_cus;
-    p.bp_grid = (uint32_t)std::min<uint64_t>({room, most, std::max<uint32_t>(items, 1u)});
+    const bool apart = p.dcap >= BOUND_MIN_DCAP;
+    for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW}) {
+        p.bp_part[part] = 0;
+        if (apart == (part == ewfa::BP_ALL)) continue;
+        const uint64_t most = (uint64_t)std::max(ewfa::bp_blocks_per_cu(part), 1) * (uint64_t)c->num_cus;
+        p.bp_part[part] = (uint32_t)std::min<uint64_t>({room, most, std::max<uint32_t>(items, 1u)});
+        p.bp_grid = std::max(p.bp_grid, p.bp_part[part]);
+    }
 }
 
 int finish_pass(ewfa_ctx* c, Pass& p, uint32_t items) {
@@ -916,6 +928,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.rest = c->bp_rest.as<uint32_t>() + (size_t)b * n;
                 x.rest_count = ctl + BP_REST;
                 x.queue = ctl + BP_QUEUE;
+                x.spread = p.bp_spread;
                 x.defer_list = sx.list_a;
                 x.defer_count = ctrl + CTRL_DEFER_A;
                 x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;
@@ -928,7 +941,8 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                     CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
                 }
                 HIPCHK(ewfa::launch_bp_sort(x, a.list, a.count_ptr, n, q));
-                HIPCHK(ewfa::launch_bp(x, p.bp_grid, q));
+                for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW})
+                    HIPCHK(ewfa::launch_bp(x, part, p.bp_part[part], q));
                 a.list = x.rest;
                 a.count_ptr = x.rest_count;
             } else {

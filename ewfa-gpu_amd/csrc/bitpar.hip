@@ -59,36 +59,64 @@ __device__ __forceinline__ void planes_of(uint64_t w, uint32_t& a, uint32_t& b) 
 // first lane.
 template <int GL>
 __device__ __forceinline__ uint32_t from_above(uint32_t x, int lane) {
-    if constexpr (GL == 16) {  // row_shr:1
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);
-    } else {  // wave_shr:1
-        const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x138, 0xF, 0xF, true);
-        if constexpr (GL == 32) return lane == 32 ? 0u : y;
-        return y;
-    }
+    // row_shr:1 within rows of 16 lanes, else wave_shr:1
+    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, GL <= 16 ? 0x111 : 0x138, 0xF, 0xF, true);
+    if constexpr (GL == 64 || GL == 16) return y;
+    return y & ((lane & (GL - 1)) ? ~0u : 0u);
 }
 
 // A lane's value from the lane after it in its group; a group's last lane
 // gets `bottom`.
 template <int GL>
 __device__ __forceinline__ uint32_t from_below(uint32_t x, uint32_t bottom, int lane) {
-    if constexpr (GL == 16) {  // row_shl:1
-        return (uint32_t)__builtin_amdgcn_update_dpp((int)bottom, (int)x, 0x101, 0xF, 0xF, false);
-    } else {  // wave_shl:1
-        const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp((int)bottom, (int)x, 0x130, 0xF, 0xF, false);
-        if constexpr (GL == 32) return lane == 31 ? bottom : y;
-        return y;
+    // row_shl:1 or wave_shl:1
+    const uint32_t y =
+        (uint32_t)__builtin_amdgcn_update_dpp((int)bottom, (int)x, GL <= 16 ? 0x101 : 0x130, 0xF, 0xF, false);
+    if constexpr (GL == 64 || GL == 16) return y;
+    return (lane & (GL - 1)) == GL - 1 ? bottom : y;
+}
+
+// A lane's value from lane x (uniform) of its group.
+template <int GL>
+__device__ __forceinline__ uint32_t from_group(uint32_t v, int x, int lane) {
+    if constexpr (GL == 64) return (uint32_t)__builtin_amdgcn_readlane((int)v, x);
+    return (uint32_t)__builtin_amdgcn_ds_bpermute(((lane & ~(GL - 1)) + x) << 2, (int)v);
+}
+
+// Inclusive sum, minimum and maximum over a group.
+template <int GL>
+__device__ __forceinline__ int group_incl_sum(int v, int lane) {
+#pragma unroll
+    for (int d = 1; d < GL; d <<= 1) {
+        const int t = __builtin_amdgcn_ds_bpermute((lane - d) << 2, v);
+        if ((lane & (GL - 1)) >= d) v += t;
     }
+    return v;
+}
+template <int GL>
+__device__ __forceinline__ int group_max(int v, int lane) {
+#pragma unroll
+    for (int d = 1; d < GL; d <<= 1) v = max(v, (int)__builtin_amdgcn_ds_bpermute((lane ^ d) << 2, v));
+    return v;
 }
 
 struct BpPair {
     const uint64_t* gp;  // packed words
     const uint64_t* gt;
-    int plen, tlen, nwp, nwt;
-    int S, L;            // band: words j + S .. j + S + N - 1 at column block j
+    int plen, tlen, nwp, nwt, tk;
+    int L;               // the most edits looked for
+    int S;               // band: words j + S .. at column block j
 };
 
-__device__ __forceinline__ BpPair bp_load(const BpArgs& a, const ewfa_pair_t& pr, int N) {
+// The band's widths over the column blocks: segment k of `n` starts at block
+// from[k], with w[k] words a lane, its records from row at[k] on (a row: 64
+// lanes of Pv, Mv, then 64 lanes of the horizontal deltas below the word).
+// Uniform over the wave; S[k] is each pair's own.
+struct BpSegs {
+    int n, from[4], w[4], at[4], S[4];
+};
+
+__device__ __forceinline__ BpPair bp_load(const BpArgs& a, uint32_t pidx, const ewfa_pair_t& pr, int N) {
     BpPair p;
     p.gp = a.words + pr.pattern_off;
     p.gt = a.words + pr.text_off;
@@ -96,7 +124,8 @@ __device__ __forceinline__ BpPair bp_load(const BpArgs& a, const ewfa_pair_t& pr
     p.tlen = (int)pr.tlen;
     p.nwp = (p.plen + 31) >> 5;
     p.nwt = (p.tlen + 31) >> 5;
-    p.L = bp_band(N, p.tlen - p.plen, p.S);
+    p.tk = p.tlen - p.plen;
+    p.L = min(bp_band(N, p.tk, p.S), (int)min(a.bound[pidx], 0x7FFFFFFFu));
     return p;
 }
 
@@ -142,12 +171,12 @@ __device__ __forceinline__ void add_carry(uint32_t (&s)[W], uint64_t cin) {
 
 // One column of the band: W words per lane, GL lanes per pair, every lane of
 // the wave taking part.  c0, c1: the text base's bits as masks.  nhp, hm gather
-// the horizontal deltas below the lane's last row (nhp: those that are not +1).
-// 18 vector instructions at W = 1, 12 to 14 per word more.
+// the horizontal deltas below each word (nhp: those that are not +1).  19
+// vector instructions at W = 1, 14 to 16 per word more.
 template <int GL, int W>
 __device__ __forceinline__ void bp_column(uint32_t (&Pv)[W], uint32_t (&Mv)[W], const uint32_t (&P0)[W],
-                                          const uint32_t (&P1)[W], uint32_t c0, uint32_t c1, uint32_t& nhp,
-                                          uint32_t& hm, int lane) {
+                                          const uint32_t (&P1)[W], uint32_t c0, uint32_t c1,
+                                          uint32_t (&nhp)[W], uint32_t (&hm)[W], int lane) {
     uint32_t Eq[W], x[W], s[W];
 #pragma unroll
     for (int w = 0; w < W; ++w) {
@@ -172,8 +201,11 @@ __device__ __forceinline__ void bp_column(uint32_t (&Pv)[W], uint32_t (&Mv)[W], 
         nPh[w] = ~Mv[w] & (Xh | Pv[w]);
         Mh[w] = Pv[w] & Xh;
     }
-    nhp = __builtin_amdgcn_alignbit(nhp, nPh[W - 1], 31);
-    hm = __builtin_amdgcn_alignbit(hm, Mh[W - 1], 31);
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        nhp[w] = __builtin_amdgcn_alignbit(nhp[w], nPh[w], 31);
+        hm[w] = __builtin_amdgcn_alignbit(hm[w], Mh[w], 31);
+    }
     const uint32_t pd = from_above<GL>(nPh[W - 1], lane);  // +1 above the band's first row
     const uint32_t md = from_above<GL>(Mh[W - 1], lane);
 #pragma unroll
@@ -186,184 +218,316 @@ __device__ __forceinline__ void bp_column(uint32_t (&Pv)[W], uint32_t (&Mv)[W], 
     }
 }
 
-// The table's deltas of 64/GL pairs (p: the lane's own), column block by column
-// block of 32.  rec gets, per block, every lane's vertical deltas at its start
-// (W uint2 of Pv, Mv) and the horizontal deltas below its last row over the
-// block (a uint2, column i at bit 31 - i): 64 * (W + 1) uint2.
+// One segment of the table's deltas of 64/GL pairs (p: the lane's own), from
+// column block j on in blocks of 32 columns: until nblk, or until no pair of
+// the wave needs more than `fewer` words a lane (looked at every BP_LOOK blocks;
+// then the band moves to the words still needed and `w` says how many words a
+// lane they take).  Records every block's deltas (BpSegs) at rec.
+//
+// What a pair still needs: a cell (v, h) of value D on diagonal k is on a path of
+// at most L edits only if D + |k - tk| <= L, and such a path stays on diagonals
+// min(k, tk) - s/2 .. max(k, tk) + s/2 from there on, s = L - D - |k - tk|.  Values
+// are looked at where words meet; a cell up to 16 rows away has s at most 32
+// larger, which the range takes in.  A band that started U wide narrows to
+// nothing about linearly, so half of the table is never computed.
+constexpr int BP_LOOK = 8;
+
+// A narrowed band's words pass from one segment to the next in LDS, 4 planes of
+// n_prev words a group, this band's from `first` on (n_prev 0: the first segment).
 template <int GL, int W>
-__device__ __forceinline__ void bp_forward(const BpPair& p, int nblk, uint2* rec, int lane) {
+__device__ __forceinline__ int bp_segment(BpPair& p, int j, int nblk, int& n_prev, int& first, int& sc, uint2*& rec,
+                                          int& w_next, uint32_t* lds, int lane) {
     constexpr int N = GL * W;
     const int gl = lane & (GL - 1);
-    uint32_t Pv[W], Mv[W], P0[W], P1[W];
+    uint32_t vp[W], vm[W], q0[W], q1[W];
+    if (n_prev) {
+        const uint32_t* G = lds + (lane / GL) * (4 * n_prev) + first + gl * W;
+        group_sync<1>();
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-        // rows above the first (negative words) count down to it, so that row
-        // 0 holds h in every column whatever their bases
-        const int A = p.S + gl * W + w;
-        Pv[w] = A < 0 ? 0u : ~0u;
-        Mv[w] = A < 0 ? ~0u : 0u;
-        planes_of(p.gp[min(max(A, 0), p.nwp)], P0[w], P1[w]);
-    }
-    for (int jb = 0; jb < nblk; jb += GL) {
-        // the next GL blocks' text planes and the pattern planes that enter
-        // the band with them, one per lane
-        uint32_t f0, f1, e0, e1;
-        planes_of(p.gt[min(jb + gl, p.nwt)], f0, f1);
-        planes_of(p.gp[min(max(jb + gl + p.S + N - 1, 0), p.nwp)], e0, e1);
-        const int nx = min(GL, nblk - jb);
-        for (int x = 0; x < nx; ++x) {
-            uint32_t T0, T1, q0, q1;
-            if constexpr (GL == 64) {
-                T0 = (uint32_t)__builtin_amdgcn_readlane((int)f0, x);
-                T1 = (uint32_t)__builtin_amdgcn_readlane((int)f1, x);
-                q0 = (uint32_t)__builtin_amdgcn_readlane((int)e0, x);
-                q1 = (uint32_t)__builtin_amdgcn_readlane((int)e1, x);
-            } else {
-                const int at = ((lane & ~(GL - 1)) + x) << 2;
-                T0 = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)f0);
-                T1 = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)f1);
-                q0 = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)e0);
-                q1 = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)e1);
-            }
-            if (jb + x > 0) {  // the band moves down a word
-                const uint32_t nPv = from_below<GL>(Pv[0], ~0u, lane);
-                const uint32_t nMv = from_below<GL>(Mv[0], 0u, lane);
-                const uint32_t n0 = from_below<GL>(P0[0], q0, lane);
-                const uint32_t n1 = from_below<GL>(P1[0], q1, lane);
-#pragma unroll
-                for (int w = 0; w + 1 < W; ++w) {
-                    Pv[w] = Pv[w + 1];
-                    Mv[w] = Mv[w + 1];
-                    P0[w] = P0[w + 1];
-                    P1[w] = P1[w + 1];
-                }
-                Pv[W - 1] = nPv;
-                Mv[W - 1] = nMv;
-                P0[W - 1] = n0;
-                P1[W - 1] = n1;
-            }
-#pragma unroll
-            for (int w = 0; w < W; ++w) rec[w * 64 + lane] = make_uint2(Pv[w], Mv[w]);
-            uint32_t nhp = 0, hm = 0;
-            for (int i8 = 0; i8 < 32; i8 += 8) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint32_t c0 = (uint32_t)((int)(T0 << (31 - i)) >> 31);
-                    const uint32_t c1 = (uint32_t)((int)(T1 << (31 - i)) >> 31);
-                    bp_column<GL, W>(Pv, Mv, P0, P1, c0, c1, nhp, hm, lane);
-                }
-                T0 >>= 8;
-                T1 >>= 8;
-            }
-            rec[W * 64 + lane] = make_uint2(~nhp, hm);
-            rec += 64 * (W + 1);
+        for (int w = 0; w < W; ++w) {
+            vp[w] = G[w];
+            vm[w] = G[n_prev + w];
+            q0[w] = G[2 * n_prev + w];
+            q1[w] = G[3 * n_prev + w];
         }
+        group_sync<1>();
+    } else {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            // rows above the first (negative words) count down to it, so that
+            // row 0 holds h in every column whatever their bases
+            const int A = p.S + gl * W + w;
+            vp[w] = A < 0 ? 0u : ~0u;
+            vm[w] = A < 0 ? ~0u : 0u;
+            planes_of(p.gp[min(max(A, 0), p.nwp)], q0[w], q1[w]);
+        }
+    }
+    int x = GL;  // feeder place
+    uint32_t f0 = 0, f1 = 0, e0 = 0, e1 = 0;
+    const int j0 = j;
+    w_next = W;
+    for (; j < nblk; ++j) {
+        if (x == GL) {
+            // the next GL blocks' text planes and the pattern planes that enter
+            // the band with them, one per lane
+            planes_of(p.gt[min(j + gl, p.nwt)], f0, f1);
+            planes_of(p.gp[min(max(j + gl + p.S + N - 1, 0), p.nwp)], e0, e1);
+            x = 0;
+        }
+        if (j > j0) {  // the band moves down a word
+            sc += 32 + __popc(vp[0]) - __popc(vm[0]);  // (a group's first lane: the value above its band)
+            const uint32_t b0 = from_below<GL>(vp[0], ~0u, lane);
+            const uint32_t b1 = from_below<GL>(vm[0], 0u, lane);
+            const uint32_t b2 = from_below<GL>(q0[0], from_group<GL>(e0, x, lane), lane);
+            const uint32_t b3 = from_below<GL>(q1[0], from_group<GL>(e1, x, lane), lane);
+#pragma unroll
+            for (int w = 0; w + 1 < W; ++w) {
+                vp[w] = vp[w + 1];
+                vm[w] = vm[w + 1];
+                q0[w] = q0[w + 1];
+                q1[w] = q1[w + 1];
+            }
+            vp[W - 1] = b0;
+            vm[W - 1] = b1;
+            q0[W - 1] = b2;
+            q1[W - 1] = b3;
+            if (W > 1 && ((j - j0) % BP_LOOK) == 0) {
+                // values where words meet, and the diagonals still in reach
+                int tot = 0;
+#pragma unroll
+                for (int w = 0; w < W; ++w) tot += __popc(vp[w]) - __popc(vm[w]);
+                int D = (int)from_group<GL>((uint32_t)sc, 0, lane) + group_incl_sum<GL>(tot, lane) - tot;
+                int lo = 1 << 28, hi = -(1 << 28);  // first and last diagonals
+                const auto look = [&](int k, int d) {
+                    const int sl = p.L - d - abs(k - p.tk);
+                    if (sl + 32 >= 0) {
+                        const int ext = ((sl + 1) >> 1) + 32;
+                        lo = min(lo, min(k, p.tk) - ext);
+                        hi = max(hi, max(k, p.tk) + ext);
+                    }
+                };
+                if (gl == 0) look(-32 * p.S, D);
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    D += __popc(vp[w]) - __popc(vm[w]);
+                    look(-32 * (p.S + gl * W + w + 1), D);
+                }
+                hi = group_max<GL>(hi, lane);
+                lo = -group_max<GL>(-lo, lane);
+                // word i holds diagonals -32(S+i)-31 .. -32(S+i)+31
+                const int ia = min(max(((-hi) >> 5) - p.S, 0), N);
+                const int ib = max(min(((31 - lo) >> 5) + 1 - p.S, N), 0);
+                const int need = max(ib - ia, 1);
+                const int wn = (need + GL - 1) / GL;
+                // the wave's pairs go on together: the most any needs
+                int most = 1;
+#pragma unroll
+                for (int v = W; v >= 2; --v)
+                    if (most == 1 && __builtin_amdgcn_ballot_w64(wn >= v && j < p.nwt)) most = v;
+                if (most < W) {
+                    w_next = most;
+                    first = min(ia, N - GL * most);
+                    n_prev = N;
+                    uint32_t* G = lds + (lane / GL) * (4 * N);
+                    group_sync<1>();
+#pragma unroll
+                    for (int w = 0; w < W; ++w) {
+                        const int at = gl * W + w;
+                        G[at] = vp[w];
+                        G[N + at] = vm[w];
+                        G[2 * N + at] = q0[w];
+                        G[3 * N + at] = q1[w];
+                    }
+                    group_sync<1>();
+                    int drop = 0;  // deltas of the words dropped at the top
+                    for (int i = gl; i < first; i += GL) drop += __popc(G[i]) - __popc(G[N + i]);
+                    drop = group_incl_sum<GL>(drop, lane);
+                    sc += (int)from_group<GL>((uint32_t)drop, GL - 1, lane);
+                    p.S += first;
+                    return j;
+                }
+            }
+        }
+        uint32_t T0 = from_group<GL>(f0, x, lane), T1 = from_group<GL>(f1, x, lane);
+        ++x;
+#pragma unroll
+        for (int w = 0; w < W; ++w) rec[w * 128 + lane] = make_uint2(vp[w], vm[w]);
+        uint32_t nhp[W], hm[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) nhp[w] = hm[w] = 0;
+        for (int i8 = 0; i8 < 32; i8 += 8) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t c0 = (uint32_t)((int)(T0 << (31 - i)) >> 31);
+                const uint32_t c1 = (uint32_t)((int)(T1 << (31 - i)) >> 31);
+                bp_column<GL, W>(vp, vm, q0, q1, c0, c1, nhp, hm, lane);
+            }
+            T0 >>= 8;
+            T1 >>= 8;
+        }
+#pragma unroll
+        for (int w = 0; w < W; ++w) rec[w * 128 + 64 + lane] = make_uint2(~nhp[w], hm[w]);
+        rec += W * 128;
+    }
+    return j;
+}
+
+// The whole table: segments of decreasing width.
+template <int GL>
+__device__ __forceinline__ void bp_forward(BpPair p, int W, int nblk, uint2* rec, BpSegs& sg, uint32_t* lds,
+                                           int lane) {
+    int sc = -32 * p.S, j = 0, w = W, n_prev = 0, first = 0;
+    const uint2* const rec0 = rec;
+    sg.n = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        sg.from[k] = 0x7FFFFFFF;
+        sg.w[k] = 1;
+        sg.at[k] = 0;
+        sg.S[k] = 0;
+        if (j >= nblk) continue;
+        sg.from[k] = j;
+        sg.w[k] = w;
+        sg.at[k] = (int)((rec - rec0) >> 7);
+        sg.S[k] = p.S;
+        sg.n = k + 1;
+        int wn = w;
+        if (w == 4) j = bp_segment<GL, 4>(p, j, nblk, n_prev, first, sc, rec, wn, lds, lane);
+        else if (w == 3) j = bp_segment<GL, 3>(p, j, nblk, n_prev, first, sc, rec, wn, lds, lane);
+        else if (w == 2) j = bp_segment<GL, 2>(p, j, nblk, n_prev, first, sc, rec, wn, lds, lane);
+        else j = bp_segment<GL, 1>(p, j, nblk, n_prev, first, sc, rec, wn, lds, lane);
+        w = wn;
     }
 }
 
 // ---- traceback ---------------------------------------------------------------
-// The path is walked back over tiles of 32 rows x 32 columns whose op codes are
-// computed again from the recorded deltas, TRACE_TILES at a time, a lane each:
-// TRACE_WORDS row words around the path's diagonal over TRACE_BLOCKS column
-// blocks.  The codes (two bits a cell, equal to OP_*, 0 for a match) go to LDS,
-// where the whole wave looks along the diagonal at once: lane i at the cell i
-// steps back, so a match run of up to 64 bases and the op that ends it are one
-// ballot.
-constexpr int TRACE_WORDS = 4, TRACE_BLOCKS = 8, TRACE_TILES = TRACE_WORDS * TRACE_BLOCKS;
-constexpr int TILE_STRIDE = 33;  // uint2 per tile: a column each, and one that spreads the banks
+// The paths are walked back over tiles of 32 rows x 32 columns whose op codes
+// are computed again from the recorded deltas, a lane a tile: TW row words
+// around the path's diagonal over TB column blocks.  The codes (two bits a cell,
+// equal to OP_*, 0 for a match) go to LDS, where lanes look along the diagonal at
+// once, each at a cell so many steps back, so a match run and the op that ends
+// it are one step.
+// Bands of 16 lanes and less (bp_walk): the wave's groups walk side by side, a
+// group over its own GL tiles, and take new tiles together.
+// Wider bands (bp_walk_wave): one pair after the other, the whole wave looking 64
+// cells back and the walk itself in scalar registers.
+template <int GL>
+struct TraceShape {
+    static constexpr int TW = GL >= 32 ? 4 : 2, TB = GL >= 32 ? 8 : GL / TW, RL = 16;
+    static constexpr int TILES = GL >= 32 ? TW * TB : 64;  // of the wave
+};
+constexpr int TILE_WORDS = 32;  // uint2 per tile, column c of tile t at c ^ (t & 31)
 
-template <int W>
-__device__ __forceinline__ void trace_tile(const BpPair& p, const uint2* rec, int lane0, int J, int l, int w,
-                                           uint2* out) {
-    const uint2* rj = rec + (size_t)J * (64 * (W + 1));
-    uint32_t pv[W], mv[W], p0[W], p1[W], T0, T1;
-#pragma unroll
-    for (int x = 0; x < W; ++x) {
-        const uint2 d = rj[x * 64 + lane0 + l];
-        pv[x] = d.x;
-        mv[x] = d.y;
-        planes_of(p.gp[min(max(J + p.S + l * W + x, 0), p.nwp)], p0[x], p1[x]);
-    }
-    uint2 h = make_uint2(~0u, 0u);
-    if (l > 0) h = rj[W * 64 + lane0 + l - 1];
-    planes_of(p.gt[min(J, p.nwt)], T0, T1);
+// Codes of one tile: pv, mv the word's deltas before the block, h the
+// horizontal deltas above it, p0, p1 and T0, T1 the pattern's and text's planes.
+__device__ __forceinline__ void trace_tile(uint32_t pv, uint32_t mv, uint2 h, uint32_t p0, uint32_t p1, uint32_t T0,
+                                           uint32_t T1, uint2* out, int swz) {
 #pragma unroll 4
     for (int i = 0; i < 32; ++i) {
         const uint32_t c0 = (uint32_t)((int)(T0 << (31 - i)) >> 31);
         const uint32_t c1 = (uint32_t)((int)(T1 << (31 - i)) >> 31);
-        uint32_t ip = (h.x >> (31 - i)) & 1u, im = (h.y >> (31 - i)) & 1u;
-        uint32_t hi = 0, lo = 0;
-#pragma unroll
-        for (int x = 0; x < W; ++x) {
-            const uint32_t E = ~(p0[x] ^ c0) & ~(p1[x] ^ c1);
-            const uint32_t Xv = E | mv[x];
-            const uint32_t Eq = E | im;
-            const uint32_t Xh = (((Eq & pv[x]) + pv[x]) ^ pv[x]) | Eq;
-            const uint32_t Ph = mv[x] | ~(Xh | pv[x]), Mh = pv[x] & Xh;
-            const uint32_t D0 = Xh | mv[x];  // diagonal delta 0
-            const uint32_t ps = (Ph << 1) | ip, ms = (Mh << 1) | im;
-            ip = Ph >> 31;
-            im = Mh >> 31;
-            pv[x] = ms | ~(Xv | ps);
-            mv[x] = ps & Xv;
-            // DEL 3: vertical +1; else SUB 2: diagonal +1; else INS 1: horizontal +1
-            const uint32_t h1 = pv[x] | ~D0;
-            const uint32_t l1 = pv[x] | (Ph & ~h1);
-            hi = x == w ? h1 : hi;
-            lo = x == w ? l1 : lo;
-        }
-        out[i] = make_uint2(hi, lo);
+        const uint32_t E = ~(p0 ^ c0) & ~(p1 ^ c1);
+        const uint32_t Xv = E | mv;
+        const uint32_t Eq = E | (h.y >> 31);
+        const uint32_t Xh = (((Eq & pv) + pv) ^ pv) | Eq;
+        const uint32_t Ph = mv | ~(Xh | pv), Mh = pv & Xh;
+        const uint32_t D0 = Xh | mv;  // diagonal delta 0
+        const uint32_t ps = (Ph << 1) | (h.x >> 31), ms = (Mh << 1) | (h.y >> 31);
+        h.x <<= 1;
+        h.y <<= 1;
+        pv = ms | ~(Xv | ps);
+        mv = ps & Xv;
+        // DEL 3: vertical +1; else SUB 2: diagonal +1; else INS 1: horizontal +1
+        const uint32_t hi = pv | ~D0;
+        out[i ^ swz] = make_uint2(hi, pv | (Ph & ~hi));
     }
 }
 
 // Bytes of a run of r matches in the stream.
 __device__ __forceinline__ int run_bytes(int r) { return (r + 126) / 127; }
 
-// The path of pair `pidx` (records in lanes lane0 .. of rec) as tokens
-// (run << 2 | op), last op first, then its CIGAR stream and result.
-template <int GL, int W>
-__device__ __forceinline__ void bp_finish(const BpArgs& a, uint32_t pidx, const ewfa_pair_t& pr, const BpPair& p,
-                                          int lane0, const uint2* rec, uint32_t* tok, uint2* tiles, int lane) {
-    constexpr int N = GL * W;
-    ewfa_result_t* res = a.results + pidx;
+// A group's bits of a wave mask.
+template <int GL>
+__device__ __forceinline__ uint64_t group_bits(uint64_t m, int lane) {
+    if constexpr (GL == 64) return m;
+    const uint32_t half = lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
+    if constexpr (GL == 32) return half;
+    return (half >> (lane & 31 & ~(GL - 1))) & ((1u << GL) - 1u);
+}
+
+// The tile (block J, word idx of the band there) into `out`; S, w, at: the band of
+// J's segment; lane0: the group's first lane.
+__device__ __forceinline__ void bp_tile(const BpPair& p, const uint2* rec, int J, int idx, int S, int w, int at,
+                                        int lane0, uint2* out, int swz) {
+    const int l = (int)((unsigned)idx / (unsigned)w), x = idx - l * w;
+    const uint2 d = rec[(size_t)(at + x) * 128 + lane0 + l];
+    uint2 h = make_uint2(~0u, 0u);  // +1 above the band
+    if (idx > 0) h = rec[(size_t)(at + (x ? x - 1 : w - 1)) * 128 + 64 + lane0 + (x ? l : l - 1)];
+    uint32_t p0, p1, T0, T1;
+    planes_of(p.gp[min(max(J + S + idx, 0), p.nwp)], p0, p1);
+    planes_of(p.gt[min(J, p.nwt)], T0, T1);
+    trace_tile(d.x, d.y, h, p0, p1, T0, T1, out, swz);
+}
+
+// The segment of block J: its band's first word S, words a lane w and J's first
+// record row `at`.
+__device__ __forceinline__ void bp_segment_of(const BpSegs& sg, int J, int& S, int& w, int& at) {
+    w = sg.w[0];
+    S = sg.S[0];
+    at = sg.at[0] + (J - sg.from[0]) * w;
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+        if (J >= sg.from[k]) {
+            w = sg.w[k];
+            S = sg.S[k];
+            at = sg.at[k] + (J - sg.from[k]) * w;
+        }
+}
+
+// The path of one pair, p and sg uniform, as bp_walk gives it.
+template <int GL>
+__device__ __forceinline__ int bp_walk_wave(const BpPair& p, const BpSegs& sg, int lane0, const uint2* rec,
+                                            uint32_t* tok, uint2* tiles, int& run, int lane) {
+    typedef TraceShape<GL> T;
     int rho = p.plen - 1, gam = p.tlen - 1;  // the cell's row and column, from 0
-    int run = 0, cnt = 0, tokv = 0;
-    bool lost = p.L < 0;
+    int cnt = 0, tokv = 0;
+    run = 0;
     const auto push = [&](int op) {
         tokv = writelane_i32(tokv, (run << 2) | op, cnt & 63);
         run = 0;
         ++cnt;
         if ((cnt & 63) == 0) tok[cnt - 64 + lane] = (uint32_t)tokv;
     };
+    if (p.L < 0) return -1;
     int j0 = 0, base = 0;
+    uint64_t tm = 0;  // tiles that lie in the band
     bool have = false;
-    while (rho >= 0 && gam >= 0 && !lost) {
+    while (rho >= 0 && gam >= 0) {
         const bool fresh = !have;
         if (!have) {
             j0 = gam >> 5;
             base = (rho - gam - 32) >> 5;  // the path's diagonal in the middle words
-            const int t = lane & (TRACE_TILES - 1);
-            const int J = j0 - t / TRACE_WORDS;
-            const int idx = base + t % TRACE_WORDS - p.S;  // word of the band
+            const int t = lane & (T::TILES - 1);
+            const int J = j0 - t / T::TW;
+            int S, w, at;
+            bp_segment_of(sg, J, S, w, at);
+            const int idx = base + t % T::TW - S;
+            const bool in = J >= 0 && idx >= 0 && idx < GL * w;
+            tm = __builtin_amdgcn_ballot_w64(in);
             group_sync<1>();
-            if (lane < TRACE_TILES && J >= 0 && idx >= 0 && idx < N)
-                trace_tile<W>(p, rec, lane0, J, idx / W, idx % W, tiles + t * TILE_STRIDE);
+            if (in && lane < T::TILES) bp_tile(p, rec, J, idx, S, w, at, lane0, tiles + t * TILE_WORDS, t & 31);
             group_sync<1>();
             have = true;
         }
         const int r = rho - lane, g = gam - lane;
-        const int J = g >> 5, q = j0 - J, u = (r >> 5) - J - base;
-        const bool in = r >= 0 && g >= 0 && q < TRACE_BLOCKS && (unsigned)u < (unsigned)TRACE_WORDS &&
-                        (unsigned)(base + u - p.S) < (unsigned)N;
-        const uint2 cc = tiles[in ? (q * TRACE_WORDS + u) * TILE_STRIDE + (g & 31) : 0];
+        const int Jc = g >> 5, q = j0 - Jc, u = (r >> 5) - Jc - base, t = q * T::TW + u;
+        const bool in = r >= 0 && g >= 0 && q < T::TB && (unsigned)u < (unsigned)T::TW && ((tm >> (t & 63)) & 1u);
+        const uint2 cc = tiles[in ? t * TILE_WORDS + ((g & 31) ^ (t & 31)) : 0];
         const uint64_t hib = __builtin_amdgcn_ballot_w64(in && ((cc.x >> (r & 31)) & 1u));
         const uint64_t lob = __builtin_amdgcn_ballot_w64(in && ((cc.y >> (r & 31)) & 1u));
         const uint64_t out = __builtin_amdgcn_ballot_w64(!in);
         const uint64_t stop = hib | lob | out;
-        if (fresh && (out & 1ull)) {  // outside the band: no path within L edits
-            lost = true;
-            break;
-        }
+        if (fresh && (out & 1ull)) return -1;  // outside the band: more than L edits
         int pos = 0;
         for (;;) {
             const uint64_t rem = pos < 64 ? stop >> pos : 0ull;
@@ -382,10 +546,7 @@ __device__ __forceinline__ void bp_finish(const BpArgs& a, uint32_t pidx, const 
                 break;
             }
             const int op = (int)((hib >> f) & 1ull) * 2 + (int)((lob >> f) & 1ull);
-            if (cnt >= p.L) {
-                lost = true;
-                break;
-            }
+            if (cnt >= p.L) return -1;
             push(op);
             if (op == OP_SUB) {  // the same diagonal goes on
                 pos = f + 1;
@@ -397,23 +558,114 @@ __device__ __forceinline__ void bp_finish(const BpArgs& a, uint32_t pidx, const 
         }
     }
     const int left = rho >= 0 ? rho + 1 : gam + 1;  // rows or columns before the other's first
-    if (lost || cnt + left > p.L) {
+    if (cnt + left > p.L) return -1;
+    for (int i = 0; i < left; ++i) push(rho >= 0 ? OP_DEL : OP_INS);
+    if (cnt & 63) tok[(cnt & ~63) + lane] = (uint32_t)tokv;
+    return cnt;
+}
+
+// The path of the lane's pair as tokens (run << 2 | op), last op first, at tok.
+// Returns the edits (-1: more than p.L) and in `run` the matches before the
+// first op.
+template <int GL>
+__device__ __forceinline__ int bp_walk(const BpPair& p, bool mine, const BpSegs& sg, const uint2* rec, uint32_t* tok,
+                                       uint2* tiles, int& run, int lane) {
+    typedef TraceShape<GL> T;
+    const int gl = lane & (GL - 1), g0 = lane & ~(GL - 1);
+    int rho = p.plen - 1, gam = p.tlen - 1;  // the cell's row and column, from 0
+    int cnt = 0;
+    bool lost = p.L < 0;
+    run = 0;
+    uint2* const my = tiles + lane * TILE_WORDS;
+    for (;;) {
+        bool go = mine && !lost && rho >= 0 && gam >= 0;
+        if (!__builtin_amdgcn_ballot_w64(go)) break;
+        // tiles: words base, base + 1 (relative to the block) of blocks j0,
+        // j0 - 1, ..
+        const int j0 = gam >> 5;
+        const int base = (rho - gam) >> 5;
+        const int J = j0 - gl / T::TW;
+        int S, w, at;
+        bp_segment_of(sg, J, S, w, at);
+        const int idx = base + gl % T::TW - S;  // word of the band
+        const bool have = go && J >= 0 && idx >= 0 && idx < GL * w;
+        const uint64_t tm = group_bits<GL>(__builtin_amdgcn_ballot_w64(have), lane);
+        group_sync<1>();
+        if (have) bp_tile(p, rec, J, idx, S, w, at, g0, my, lane & 31);
+        group_sync<1>();
+        bool fresh = true;
+        while (__builtin_amdgcn_ballot_w64(go)) {
+            uint64_t hb = 0, lb = 0, ob = 0;  // by cells back: op bits, outside the tiles
+#pragma unroll
+            for (int c = 0; c < T::RL; c += GL) {
+                const int r = rho - gl - c, g = gam - gl - c;
+                const int Jc = g >> 5, q = j0 - Jc, u = (r >> 5) - Jc - base, t = q * T::TW + u;
+                const bool in = r >= 0 && g >= 0 && q < T::TB && (unsigned)u < (unsigned)T::TW && ((tm >> (t & 63)) & 1u);
+                const uint2 cc = tiles[in ? (g0 + t) * TILE_WORDS + ((g & 31) ^ ((g0 + t) & 31)) : 0];
+                hb |= group_bits<GL>(__builtin_amdgcn_ballot_w64(in && ((cc.x >> (r & 31)) & 1u)), lane) << c;
+                lb |= group_bits<GL>(__builtin_amdgcn_ballot_w64(in && ((cc.y >> (r & 31)) & 1u)), lane) << c;
+                ob |= group_bits<GL>(__builtin_amdgcn_ballot_w64(!in), lane) << c;
+            }
+            if (go) {
+                const uint64_t stop = hb | lb | ob;
+                const int f = stop ? (int)__builtin_ctzll(stop) : T::RL;
+                run += f;
+                rho -= f;
+                gam -= f;
+                if (stop) {
+                    if ((ob >> f) & 1u) {
+                        // on to new tiles, unless the path left the band: then
+                        // it has more than L edits
+                        lost = lost || (fresh && f == 0);
+                        go = false;
+                    } else {
+                        const int op = (int)((hb >> f) & 1u) * 2 + (int)((lb >> f) & 1u);
+                        if (cnt >= p.L) {
+                            lost = true;
+                            go = false;
+                        } else {
+                            if (gl == 0) tok[cnt] = (uint32_t)(run << 2 | op);
+                            ++cnt;
+                            run = 0;
+                            rho -= op != OP_INS;
+                            gam -= op != OP_DEL;
+                        }
+                    }
+                }
+                go = go && rho >= 0 && gam >= 0;
+            }
+            fresh = false;
+        }
+    }
+    if (!mine || lost) return -1;
+    // rows or columns before the other's first
+    const int left = rho >= 0 ? rho + 1 : gam + 1;
+    if (cnt + left > p.L) return -1;
+    const uint32_t op = rho >= 0 ? OP_DEL : OP_INS;
+    for (int i = gl; i < left; i += GL) tok[cnt + i] = i == 0 ? (uint32_t)run << 2 | op : op;
+    if (left > 0) run = 0;
+    return cnt + left;
+}
+
+// The CIGAR stream of a pair from its tokens, by the whole wave, and its result
+// (cnt edits, -1: deferred; run: the matches before the first op).
+__device__ __forceinline__ void bp_emit(const BpArgs& a, uint32_t pidx, int cnt, int run, const uint32_t* tok, int lane) {
+    ewfa_result_t* res = a.results + pidx;
+    if (cnt < 0) {
         if (lane == 0) {
             a.defer_list[atomicAdd(a.defer_count, 1u)] = pidx;
             res->status = PAIR_DEFERRED;
         }
         return;
     }
-    if ((pr.cigar_off & 3u) || (pr.cigar_cap & 3u)) {
-        if (lane == 0) *res = ewfa_result_t{cnt + left, 0, EWFA_PAIR_BADARG, 0};
+    const uint64_t coff = a.pairs[pidx].cigar_off;
+    const uint32_t cap = a.pairs[pidx].cigar_cap;
+    if ((coff & 3u) || (cap & 3u)) {
+        if (lane == 0) *res = ewfa_result_t{cnt, 0, EWFA_PAIR_BADARG, 0};
         return;
     }
-    for (int i = 0; i < left; ++i) push(rho >= 0 ? OP_DEL : OP_INS);
-    if (cnt & 63) tok[(cnt & ~63) + lane] = (uint32_t)tokv;
-    __threadfence_block();  // the tokens are read back by other lanes
-    // the stream: step s's run and op from tokens cnt - s and cnt - 1 - s
-    int8_t* out = a.cigars + pr.cigar_off;
-    const uint32_t cap = pr.cigar_cap;
+    // step s's run and op from tokens cnt - s and cnt - 1 - s
+    int8_t* out = a.cigars + coff;
     uint32_t at0 = 0;
     const auto put_run = [&](uint32_t at, int rb) -> uint32_t {
         for (; rb >= 127; rb -= 127, ++at)
@@ -448,23 +700,42 @@ __device__ __forceinline__ void bp_finish(const BpArgs& a, uint32_t pidx, const 
     }
 }
 
-template <int GL, int W>
-__device__ __forceinline__ void bp_item(const BpArgs& a, const uint32_t* list, uint32_t first, uint32_t count,
-                                        uint2* rec, uint32_t* tok, uint2* tiles, int lane) {
-    constexpr int NG = 64 / GL;
-    // lanes of groups past the list's end repeat its last pair
-    const uint32_t mine = list[min(first + (uint32_t)(lane / GL), count - 1u)];
-    const ewfa_pair_t pr = a.pairs[mine];
-    const BpPair p = bp_load(a, pr, GL * W);
+// One wave's pairs: list[first ..] up to 64/GL of them, below `end`, of bands of
+// N words.
+template <int GL>
+__device__ __forceinline__ void bp_item(const BpArgs& a, uint32_t first, uint32_t end, int N, uint2* rec, uint32_t* tok,
+                                        uint2* tiles, int lane) {
+    const uint32_t g = (uint32_t)(lane / GL);
+    // lanes of groups past the list's end repeat its last pair, unwalked
+    const uint32_t pidx = a.list[min(first + g, end - 1u)];
+    const ewfa_pair_t pr = a.pairs[pidx];
+    const int W = (N + GL - 1) / GL;
+    const BpPair p = bp_load(a, pidx, pr, GL * W);
     int nblk = 0;
 #pragma unroll
-    for (int g = 0; g < NG; ++g) nblk = max(nblk, (int)__builtin_amdgcn_readlane(p.nwt, g * GL));
-    bp_forward<GL, W>(p, nblk, rec, lane);
+    for (int q = 0; q < 64 / GL; ++q) nblk = max(nblk, (int)__builtin_amdgcn_readlane(p.nwt, q * GL));
+    BpSegs sg;
+    bp_forward<GL>(p, W, nblk, rec, sg, reinterpret_cast<uint32_t*>(tiles), lane);
     __threadfence_block();  // the records are read back by other lanes
-    for (uint32_t g = 0; g < (uint32_t)NG && first + g < count; ++g) {
-        const uint32_t pidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[first + g]);
-        const ewfa_pair_t pg = a.pairs[pidx];
-        bp_finish<GL, W>(a, pidx, pg, bp_load(a, pg, GL * W), (int)g * GL, rec, tok, tiles, lane);
+    int run = 0, cnt = 0;
+    if constexpr (GL < 32) cnt = bp_walk<GL>(p, first + g < end, sg, rec, tok + g * BP_TOK_STRIDE(GL), tiles, run, lane);
+    for (uint32_t q = 0; q < 64u / GL && first + q < end; ++q) {
+        const int src = (int)q * GL;
+        const uint32_t mine = (uint32_t)__builtin_amdgcn_readlane((int)pidx, src);
+        uint32_t* const t = tok + q * BP_TOK_STRIDE(GL);
+        if constexpr (GL < 32) {
+            __threadfence_block();  // the tokens are read back by other lanes
+            bp_emit(a, mine, __builtin_amdgcn_readlane(cnt, src), __builtin_amdgcn_readlane(run, src), t, lane);
+        } else {
+            const ewfa_pair_t pg = a.pairs[mine];
+            const BpPair pu = bp_load(a, mine, pg, GL * W);
+            BpSegs su = sg;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) su.S[k] = __builtin_amdgcn_readlane(sg.S[k], src);
+            const int c = bp_walk_wave<GL>(pu, su, src, rec, t, tiles, run, lane);
+            __threadfence_block();
+            bp_emit(a, mine, c, run, t, lane);
+        }
     }
 }
 
@@ -472,36 +743,42 @@ __device__ __forceinline__ void bp_item(const BpArgs& a, const uint32_t* list, u
 
 // Persistent, one wave per block.  The list holds the pairs class by class,
 // widest band first (BP_CLASSES classes from seg[c], seg[BP_CLASSES] the end),
-// each by decreasing length; an item is the 64/GL pairs of a wave.
-__global__ __launch_bounds__(64, 4) void bp_kernel(BpArgs a) {
-    __shared__ uint2 tiles[TRACE_TILES * TILE_STRIDE];
+// each by decreasing length; an item is the 64/GL pairs of a wave.  PART: the
+// classes of 32 lanes and more (BP_WIDE), the others (BP_NARROW) or all.  Long
+// reads take the first two one after the other, since the wide bands alone need
+// half the LDS (four waves per SIMD instead of two and a half: 20,000 pairs of
+// 10..50 kbp in 44.5 ms, 51.6 with one kernel for all); shorter pairs, of which
+// few are wide, one kernel, whose narrow pairs hide the wide ones' long chains
+// (15,001 pairs of 3..7 kbp at 8..15% edits: 3.5 ms, 4.9 apart).
+template <int PART>
+__global__ __launch_bounds__(64, PART == BP_WIDE ? 4 : 3) void bp_kernel(BpArgs a) {
+    __shared__ uint2 tiles[TraceShape<PART == BP_WIDE ? 64 : 16>::TILES * TILE_WORDS];
     const int lane = threadIdx.x;
     if (a.seg[BP_CLASSES] == 0) return;
     uint8_t* slot = a.slots + (size_t)blockIdx.x * a.slot_bytes;
     uint32_t* tok = reinterpret_cast<uint32_t*>(slot);
     uint2* rec = reinterpret_cast<uint2*>(slot + a.tok_bytes);
     for (;;) {
-        uint32_t item = wave_take(a.queue, 1u, lane);
-        int c = 0;
+        uint32_t item = wave_take(a.queue + (PART == BP_NARROW ? 1 : 0), 1u, lane);
+        int c = 0, gl = 64;
         uint32_t lo = 0, hi = 0, per = 1;
         for (; c < BP_CLASSES; ++c) {
+            gl = bp_group(c, a.spread);
+            if (PART != BP_ALL && (gl >= 32) != (PART == BP_WIDE)) continue;
             lo = a.seg[c];
             hi = a.seg[c + 1];
-            per = bp_pairs_per_wave(c);
+            per = 64u / (uint32_t)gl;
             const uint32_t items = (hi - lo + per - 1u) / per;
             if (item < items) break;
             item -= items;
         }
         if (c == BP_CLASSES) break;
         const uint32_t first = lo + item * per;
-        switch (c) {
-            case 0: bp_item<64, 4>(a, a.list, first, hi, rec, tok, tiles, lane); break;
-            case 1: bp_item<64, 3>(a, a.list, first, hi, rec, tok, tiles, lane); break;
-            case 2: bp_item<64, 2>(a, a.list, first, hi, rec, tok, tiles, lane); break;
-            case 3: bp_item<64, 1>(a, a.list, first, hi, rec, tok, tiles, lane); break;
-            case 4: bp_item<32, 1>(a, a.list, first, hi, rec, tok, tiles, lane); break;
-            default: bp_item<16, 1>(a, a.list, first, hi, rec, tok, tiles, lane); break;
-        }
+        const int N = bp_words(c);
+        if (PART != BP_NARROW && gl == 64) bp_item<64>(a, first, hi, N, rec, tok, tiles, lane);
+        else if (PART != BP_NARROW && gl == 32) bp_item<32>(a, first, hi, N, rec, tok, tiles, lane);
+        else if (PART != BP_WIDE && gl == 16) bp_item<16>(a, first, hi, N, rec, tok, tiles, lane);
+        else if (PART != BP_WIDE) bp_item<8>(a, first, hi, N, rec, tok, tiles, lane);
         group_sync<1>();
     }
 }
@@ -653,7 +930,7 @@ __device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& p
             // to calls: 500,000 pairs of 100..10,000 bp at 1..10% edits took 25.1,
             // 20.6, 20.1 and 20.7 ms with 0.22, 0.5, 1 and 2 per u * u)
             const float wfa = 0.6f * (float)u * (float)u + 100.0f * (float)u;
-            const float bp = (float)pr.tlen * (bp_column_cost(c) + 4.0f) + 25.0f * (float)u;
+            const float bp = (float)pr.tlen * (bp_column_cost(c) + 2.0f) + 25.0f * (float)u;
             return wfa < bp ? BP_CLASSES : c;
         }
     }
@@ -742,17 +1019,22 @@ hipError_t launch_bp_sort(const BpArgs& a, const uint32_t* list, const uint32_t*
     return hipGetLastError();
 }
 
-hipError_t launch_bp(const BpArgs& a, uint32_t grid, hipStream_t stream) {
+hipError_t launch_bp(const BpArgs& a, int part, uint32_t grid, hipStream_t stream) {
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(bp_kernel, dim3(grid), dim3(64), 0, stream, a);
+    switch (part) {
+        case BP_WIDE: hipLaunchKernelGGL(bp_kernel<BP_WIDE>, dim3(grid), dim3(64), 0, stream, a); break;
+        case BP_NARROW: hipLaunchKernelGGL(bp_kernel<BP_NARROW>, dim3(grid), dim3(64), 0, stream, a); break;
+        default: hipLaunchKernelGGL(bp_kernel<BP_ALL>, dim3(grid), dim3(64), 0, stream, a); break;
+    }
     return hipGetLastError();
 }
 
-int bp_blocks_per_cu() {
+int bp_blocks_per_cu(int part) {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&bp_kernel), 64, 0) !=
-        hipSuccess)
-        return 0;
+    const void* f = part == BP_WIDE     ? reinterpret_cast<const void*>(&bp_kernel<BP_WIDE>)
+                    : part == BP_NARROW ? reinterpret_cast<const void*>(&bp_kernel<BP_NARROW>)
+                                        : reinterpret_cast<const void*>(&bp_kernel<BP_ALL>);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, f, 64, 0) != hipSuccess) return 0;
     return blocks;
 }
 

@@ -170,13 +170,22 @@ inline int reg_chunks_for(int dcap) {
 
 
 // ---- bit-parallel passes (bitpar.hip) ----
-// Classes of pairs by the words of 32 diagonals their band holds, widest first.
-constexpr int BP_CLASSES = 6;
-__host__ __device__ inline int bp_words(int c) { return c == 0 ? 256 : c == 1 ? 192 : c == 2 ? 128 : c == 3 ? 64 : c == 4 ? 32 : 16; }
-// Pairs that share a wave, and a column's wave instructions per pair.
-__host__ __device__ inline uint32_t bp_pairs_per_wave(int c) { return c <= 3 ? 1u : c == 4 ? 2u : 4u; }
+// Classes of pairs by the words of 32 diagonals their band starts with, widest
+// first.
+constexpr int BP_CLASSES = 10;
+__host__ __device__ inline int bp_words(int c) {
+    return c == 0 ? 256 : c == 1 ? 192 : c == 2 ? 128 : c == 3 ? 96 : c == 4 ? 64 : c == 5 ? 48 : c == 6 ? 32 : c == 7 ? 24 : c == 8 ? 16 : 8;
+}
+// Lanes per pair: 64 for 129..256 words, 32 for 65..128, 16 for 33..64, 8 below,
+// four words a lane at most; `spread` doubles them (for short lists, where more
+// lanes per pair make a pair's columns shorter chains).
+__host__ __device__ inline int bp_group(int c, int spread) {
+    const int g = (c <= 1 ? 64 : c <= 3 ? 32 : c <= 5 ? 16 : 8) << spread;
+    return g < 64 ? g : 64;
+}
+// A column's wave instructions per pair, over the band's narrowing.
 __host__ __device__ inline float bp_column_cost(int c) {
-    return c == 0 ? 60.f : c == 1 ? 47.f : c == 2 ? 34.f : c == 3 ? 20.f : c == 4 ? 13.f : 6.5f;
+    return c == 0 ? 45.f : c == 1 ? 36.f : c == 2 ? 22.f : c == 3 ? 18.f : c == 4 ? 11.f : c == 5 ? 9.f : c == 6 ? 5.5f : c == 7 ? 4.5f : c == 8 ? 3.5f : 2.7f;
 }
 constexpr int BP_LEN_BINS = 32;
 constexpr int BP_BINS = (BP_CLASSES + 1) * BP_LEN_BINS;
@@ -210,16 +219,21 @@ struct BpArgs {
     const uint32_t* list;     // ... and as read
     uint32_t* rest;           // pairs left to the wavefront, and their count
     uint32_t* rest_count;
-    uint32_t* queue;          // work counter of the pass
+    uint32_t* queue;          // work counters of the wide and the narrow classes
+    int spread;               // bp_group
     uint32_t* defer_list;
     uint32_t* defer_count;
     uint8_t* slots;           // per block: tok_bytes of tokens, then the records
     size_t slot_bytes, tok_bytes;
 };
 
-// Token bytes and record bytes of a slot for texts up to max_len bases.
-inline size_t bp_tok_bytes() { return 4u * (size_t)(64 * 256 + 128); }
-inline size_t bp_rec_bytes(uint32_t max_len) { return (size_t)(max_len / 32u + 1u) * 64u * 5u * 8u; }
+// Tokens a pair of a group of gl lanes may have: its band's most edits (below
+// 32 * 4 * gl) and room for a flush.
+#define BP_TOK_STRIDE(gl) (128u * (unsigned)(gl) + 64u)
+// Token bytes and record bytes of a slot for texts up to max_len bases: 64 / gl
+// pairs' tokens, and per block of 32 columns up to four words a lane of 16 bytes.
+inline size_t bp_tok_bytes() { return 4u * 8u * (size_t)BP_TOK_STRIDE(64) / 4u; }
+inline size_t bp_rec_bytes(uint32_t max_len) { return (size_t)(max_len / 32u + 1u) * 64u * 4u * 16u; }
 // Upper bounds on the distances of a list's pairs, a lane each.
 hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* list, const uint32_t* count_ptr,
                            uint32_t count, uint32_t max_grid, hipStream_t stream);
@@ -227,8 +241,9 @@ hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* lis
 // when not null).
 hipError_t launch_bp_sort(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
                           hipStream_t stream);
-hipError_t launch_bp(const BpArgs& a, uint32_t grid, hipStream_t stream);
-int bp_blocks_per_cu();
+enum : int { BP_ALL = 0, BP_WIDE = 1, BP_NARROW = 2 };
+hipError_t launch_bp(const BpArgs& a, int part, uint32_t grid, hipStream_t stream);
+int bp_blocks_per_cu(int part);
 
 // Bytes of a pair's CIGAR region the emit kernel wrote: whole dwords from
 // cigar_off up to and including the terminator (or up to cigar_cap when the
