@@ -82,7 +82,8 @@ enum : int {
     BP_SEG = 2 * ewfa::BP_BINS,
     BP_REST = BP_SEG + ewfa::BP_CLASSES + 1,
     BP_QUEUE = BP_REST + 1,
-    BP_CTRL = (BP_QUEUE + 2 + 31) & ~31,
+    BP_FLAG = BP_QUEUE + 2,
+    BP_CTRL = (BP_FLAG + 1 + 31) & ~31,
     CTRL_WORDS = CTRL_BP + ewfa::MAX_BUCKETS * BP_CTRL
 };
 
@@ -310,7 +311,7 @@ constexpr size_t BP_BUDGET = (size_t)20 << 30;
 // as its pair's columns (0.4 ms at 5 kbp) whatever the count, which a small
 // call waits for.
 constexpr uint32_t LANE_BOUND_MIN = 8192;
-constexpr uint32_t BP_MIN_LEN = 2500;
+constexpr uint32_t BP_PROBE_MIN = 4096;
 // Lists below this get twice the lanes per pair: eight pairs a wave would leave
 // SIMDs with less than two waves (15,001 pairs of 3..7 kbp: 4.0 -> 3.5 ms; 500,000
 // pairs of up to 10 kbp 17.5 -> 20.8 ms, so large lists keep the narrow groups).
@@ -324,10 +325,9 @@ void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     p.bp_slot_bytes = 0;
     if (p.reg || p.gslot || p.bt_lds || c->opts.max_distance > 0) return;
     if (p.seq_words > ewfa::BOUND_MAX_SEQ_WORDS) return;
-    // passes without bounds of their own: only where the bounds are cheap, and
-    // from BP_MIN_LEN on (pairs of 1,200..2,500 bp at 1..10% edits lose more to
-    // the two passes ahead than they gain)
-    if (p.dcap < BOUND_MIN_DCAP && (items < LANE_BOUND_MIN || blen <= BP_MIN_LEN)) return;
+    // passes without bounds of their own: lists long enough for the sample that
+    // decides on them (bp_probe_kernel)
+    if (p.dcap < BOUND_MIN_DCAP && items < BP_PROBE_MIN) return;
     p.bp_spread = items < BP_SPREAD_BELOW ? 1 : 0;
     p.bp_slot_bytes = ewfa::bp_tok_bytes() + ewfa::bp_rec_bytes(blen);
     const uint64_t room = std::max<size_t>(BP_BUDGET / p.bp_slot_bytes, 1);
@@ -934,9 +934,14 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;
                 x.slot_bytes = p.bp_slot_bytes;
                 x.tok_bytes = ewfa::bp_tok_bytes();
-                if (n >= LANE_BOUND_MIN) {
+                const bool probe = p.dcap < BOUND_MIN_DCAP;
+                if (probe) {
+                    HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, ctl + BP_FLAG, q));
+                    x.flag = ctl + BP_FLAG;
+                }
+                if (probe || n >= LANE_BOUND_MIN) {
                     HIPCHK(ewfa::launch_bp_bound(x, sx.bound, a.list, a.count_ptr, n, (uint32_t)c->num_cus * 16u, q));
-                    a.bound = p.dcap < BOUND_MIN_DCAP ? nullptr : sx.bound;
+                    a.bound = probe ? nullptr : sx.bound;
                 } else {
                     CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
                 }

@@ -783,6 +783,11 @@ __global__ __launch_bounds__(64, PART == BP_WIDE ? 4 : 3) void bp_kernel(BpArgs 
     }
 }
 
+// Wave instructions of a wavefront search of d levels (weights fitted to calls:
+// 500,000 pairs of 100..10,000 bp at 1..10% edits took 25.1, 20.6, 20.1 and 20.7 ms
+// with 0.22, 0.5, 1 and 2 per d * d).
+__device__ __forceinline__ float wavefront_cost(float d) { return 0.6f * d * d + 100.0f * d; }
+
 // ---- distance bounds ------------------------------------------------------------
 // An upper bound on each pair's distance from a window of 64 diagonals that
 // follows the path: the same table, one pair per lane, the window's vertical
@@ -889,9 +894,48 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
 
 }  // namespace
 
+// Whether a list takes the bit-parallel way at all, from a sample: 64 of its
+// pairs, a lane each, and the edits in the first PROBE_BASES of each.  The
+// wavefront's time is its work, or its longest pair's levels of about 0.45 us
+// each; the bit-parallel one its work, or its longest pair's columns of about
+// 0.4 us (bounds, table and path).  (Short lists of moderate lengths go faster
+// through the wavefront: jobs of 100..5,000 bp at 1..10% edits in batches of
+// 25,000 pairs 5.6 against 7.4 ms, while 15,001 pairs of 3..7 kbp at 8..15%
+// take 3.3 against 5.9.)  The sample takes about 50 us.
+constexpr int PROBE_BASES = 512;
+
+__global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
+                                                      uint32_t count, uint32_t* flag) {
+    const uint32_t n = count_ptr ? *count_ptr : count;
+    if (n == 0) return;
+    const uint32_t item = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) / 128u);
+    const uint32_t pidx = list ? list[item] : item;
+    const ewfa_pair_t pr = a.pairs[pidx];
+    float wfa = 0.f, bp = 0.f, levels = 0.f, columns = 0.f;
+    if (pr.plen <= a.max_len && pr.tlen <= a.max_len && pr.tlen > 0u) {
+        const int tl = min((int)pr.tlen, PROBE_BASES), pl = min((int)pr.plen, PROBE_BASES);
+        const uint32_t u = lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl);
+        columns = (float)pr.tlen;
+        levels = (float)u / (float)tl * columns;
+        wfa = wavefront_cost(levels);
+        bp = columns * 7.5f + 25.0f * levels;
+    }
+    for (int d = 32; d; d >>= 1) {
+        wfa += __shfl_xor(wfa, d);
+        bp += __shfl_xor(bp, d);
+        levels = fmaxf(levels, __shfl_xor(levels, d));
+        columns = fmaxf(columns, __shfl_xor(columns, d));
+    }
+    // wave instructions a microsecond: 256 CUs at about 2.3 GHz
+    const float us = (float)n / 64.0f / 590000.0f;
+    if (threadIdx.x == 0) *flag = fmaxf(bp * us, columns * 0.4f) < fmaxf(wfa * us, levels * 0.45f) ? 1u : 0u;
+}
+
 __global__ __launch_bounds__(64, 4) void bp_bound_kernel(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
                                                          uint32_t* bound, const uint32_t* list,
-                                                         const uint32_t* count_ptr, uint32_t count) {
+                                                         const uint32_t* count_ptr, uint32_t count,
+                                                         const uint32_t* flag) {
+    if (flag && *flag == 0u) return;
     const uint32_t n = count_ptr ? *count_ptr : count;
     for (uint32_t item = blockIdx.x * 64u + threadIdx.x; item < n; item += gridDim.x * 64u) {
         const uint32_t pidx = list ? list[item] : item;
@@ -908,7 +952,13 @@ hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* lis
     if (count == 0) return hipSuccess;
     const uint32_t blocks = (count + 63u) / 64u;
     hipLaunchKernelGGL(bp_bound_kernel, dim3(blocks < max_grid ? blocks : max_grid), dim3(64), 0, stream, a.words,
-                       a.pairs, a.max_len, bound, list, count_ptr, count);
+                       a.pairs, a.max_len, bound, list, count_ptr, count, a.flag);
+    return hipGetLastError();
+}
+
+hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
+                           uint32_t* flag, hipStream_t stream) {
+    hipLaunchKernelGGL(bp_probe_kernel, dim3(1), dim3(64), 0, stream, a, list, count_ptr, count, flag);
     return hipGetLastError();
 }
 
@@ -926,10 +976,8 @@ __device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& p
     for (int c = BP_CLASSES - 1; c >= 0; --c) {
         int S;
         if (bp_band(bp_words(c), tk, S) >= (int)u) {
-            // wave instructions of either way (the wavefront's weights fitted
-            // to calls: 500,000 pairs of 100..10,000 bp at 1..10% edits took 25.1,
-            // 20.6, 20.1 and 20.7 ms with 0.22, 0.5, 1 and 2 per u * u)
-            const float wfa = 0.6f * (float)u * (float)u + 100.0f * (float)u;
+            // wave instructions of either way
+            const float wfa = wavefront_cost((float)u);
             const float bp = (float)pr.tlen * (bp_column_cost(c) + 2.0f) + 25.0f * (float)u;
             return wfa < bp ? BP_CLASSES : c;
         }
@@ -946,7 +994,7 @@ __device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& p
 // Bin of a pair in the sort: its class, then its length, longest first.
 __device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, uint32_t u) {
     const ewfa_pair_t pr = a.pairs[pidx];
-    const int c = bp_class_of(a, pr, u);
+    const int c = a.flag && *a.flag == 0u ? BP_CLASSES : bp_class_of(a, pr, u);
     const uint32_t b = min((uint32_t)((uint64_t)pr.tlen * BP_LEN_BINS / (a.max_len + 1u)), (uint32_t)BP_LEN_BINS - 1u);
     return c * BP_LEN_BINS + (int)(BP_LEN_BINS - 1u - b);
 }
