@@ -519,9 +519,14 @@ void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t n, Chain& 
     g_err.clear();
 }
 
+// Longest pairs of a banded pass over a whole list: up to here (5.7 KB of LDS a
+// wave) a CU holds 28 of its waves.
+constexpr uint32_t BANDED_ONE_LEN = 3000;
+
 int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
     pl = Plan{};
-    if (n <= (uint32_t)c->num_cus && max_len > c->policy.buckets.front().len_hi) {
+    const bool capped = c->opts.max_distance > 0 && c->opts.max_distance <= 64;
+    if (!capped && n <= (uint32_t)c->num_cus && max_len > c->policy.buckets.front().len_hi) {
         // at most a pair per CU: the call lasts as long as its longest pair,
         // so all go through that pair's pass, without bucketing and the fork
         // over streams (60 pairs of 100..2,000 bp: 175 -> 130 us)
@@ -532,7 +537,16 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         assign_slots(pl);
         return EWFA_OK;
     }
-    for (const ewfa::BucketPolicy& b : c->policy.buckets) {
+    // Under a cap of at most 64 every search ends within 63 levels, which the
+    // banded register pass holds whatever the length: one such pass without
+    // bucketing while its slots (which hold the longest pair) leave a CU full
+    // of waves, else buckets of it (200,000 pairs of 300..1,200 bp: 1,031 -> 560 us).
+    std::vector<ewfa::BucketPolicy> banded;
+    if (capped) {
+        banded.push_back({std::min(max_len, BANDED_ONE_LEN), 1, 63, 1, 4});
+        for (uint32_t hi : {10500u, 25000u, 0xFFFFFFFFu}) banded.push_back({hi, 1, 63, 1, 1});
+    }
+    for (const ewfa::BucketPolicy& b : banded.empty() ? c->policy.buckets : banded) {
         if (pl.nb == ewfa::MAX_BUCKETS) break;
         pl.table.hi[pl.nb] = b.len_hi;
         pl.blen[pl.nb] = std::min(b.len_hi, max_len);

@@ -27,7 +27,7 @@ Policy default_policy() {
     // holds no LDS) runs beside the other's block pass (189 -> 184 ms)
     //              len_hi   waves dcap  bt_lds grab
     p.buckets.push_back({300u, 1, 63, 1, 16});
-    p.buckets.push_back({700u, 1, 127, 1, 4});
+    p.buckets.push_back({700u, 1, 63, 1, 4});
     p.buckets.push_back({1200u, 1, 127, 1, 4});
     p.buckets.push_back({2500u, 2, 768, 0, 1});
     p.buckets.push_back({5000u, 2, 512, 0, 1});
