@@ -207,6 +207,18 @@ int set_device(ewfa_ctx* c) {
     return EWFA_OK;
 }
 
+// Orders the context's work after what the caller queued on its stream.  A
+// stream with nothing left to do needs no event: the wait on another queue's
+// event cost half of a small call (one pair 46 -> 23 us).  (A query of the null
+// stream covers the blocking streams, as an event on it does.)
+int order_after(ewfa_ctx* c, hipStream_t stream) {
+    if (hipStreamQuery(stream) == hipSuccess) return EWFA_OK;
+    (void)hipGetLastError();  // "not ready" is no failure
+    HIPCHK(hipEventRecord(c->ev_in, stream));
+    HIPCHK(hipStreamWaitEvent(c->stream, c->ev_in, 0));
+    return EWFA_OK;
+}
+
 // Pass configuration: one launch of the align kernel.
 struct Pass {
     int waves;
@@ -1384,8 +1396,7 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
     for (int k = 0; k < pl.nb; ++k) CHK(fit(pl.pass[k]));
     for (int k = 0; k < pl.chain.np; ++k) CHK(fit(pl.chain.pass[k]));
     hipStream_t s = c->stream;
-    HIPCHK(hipEventRecord(c->ev_in, (hipStream_t)stream));
-    HIPCHK(hipStreamWaitEvent(s, c->ev_in, 0));
+    CHK(order_after(c, (hipStream_t)stream));
     c->align_ms = c->emit_ms = 0.f;
     c->ext = &x;
     const int rc = enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s, c->timing);
@@ -1718,9 +1729,7 @@ int ewfa_align_device(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t*
     if (n > 0xFFFFFFF0u) return fail(EWFA_ERR_RANGE, "too many pairs in one call");
     CHK(set_device(c));
     hipStream_t s = c->stream;
-    // order the work after what the caller queued on its stream
-    HIPCHK(hipEventRecord(c->ev_in, (hipStream_t)stream));
-    HIPCHK(hipStreamWaitEvent(s, c->ev_in, 0));
+    CHK(order_after(c, (hipStream_t)stream));
     CHK(reserve_scratch(c, n, max_len));
     c->align_ms = c->emit_ms = 0.f;
 
