@@ -106,7 +106,7 @@ struct ewfa_ctx {
     int num_cus = 0;
     size_t lds_max = 0;
     DevBuf ops, bt, ctrl, list_a, list_b, buckets, runs, list_fb, bound, gslot, order;
-    DevBuf bp_list, bp_rest, bp_slots;  // bit-parallel passes
+    DevBuf bp_list, bp_rest, bp_guess, bp_slots;  // bit-parallel passes
     uint32_t* host_ctrl = nullptr;  // pinned mirror of the control words
     float align_ms = 0.f, emit_ms = 0.f;
     bool timing = false;
@@ -675,6 +675,7 @@ int reserve_plan(ewfa_ctx* c, const Plan& pl, size_t n) {
     if (pl.bp_bytes) {
         CHK(c->bp_slots.reserve(c, pl.bp_bytes));
         CHK(c->bp_list.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
+        CHK(c->bp_guess.reserve(c, std::max<size_t>(n, 1) * 4));
         CHK(c->bp_rest.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
     }
     bool narrow = false;
@@ -962,10 +963,11 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.tok_bytes = ewfa::bp_tok_bytes();
                 const bool probe = p.dcap < BOUND_MIN_DCAP;
                 if (probe) {
-                    HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, ctl + BP_FLAG, q));
+                    HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, p.dcap, ctl + BP_FLAG, q));
                     x.flag = ctl + BP_FLAG;
                 }
                 if (probe || n >= LANE_BOUND_MIN) {
+                    x.guess = c->bp_guess.as<uint32_t>();
                     HIPCHK(ewfa::launch_bp_bound(x, sx.bound, a.list, a.count_ptr, n, (uint32_t)c->num_cus * 16u, q));
                     a.bound = probe ? nullptr : sx.bound;
                 } else {
@@ -1600,7 +1602,7 @@ int ewfa_destroy(ewfa_ctx_t* c) {
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     for (DevBuf* b : {&c->ops, &c->bt, &c->ctrl, &c->list_a, &c->list_b, &c->buckets, &c->runs, &c->list_fb, &c->bound,
-                      &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results, &c->h_cigars, &c->dense, &c->scan})
+                      &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_guess, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results, &c->h_cigars, &c->dense, &c->scan})
         b->release();
     if (c->host_ctrl) (void)hipHostFree(c->host_ctrl);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
@@ -1687,7 +1689,7 @@ int ewfa_context_memory(ewfa_ctx_t* c, size_t* bytes) {
     if (!c || !bytes) return fail(EWFA_ERR_ARG, "null argument");
     size_t b = 0;
     for (const DevBuf* d : {&c->ops, &c->bt, &c->ctrl, &c->list_a, &c->list_b, &c->buckets, &c->runs,
-                            &c->list_fb, &c->bound, &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results,
+                            &c->list_fb, &c->bound, &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_guess, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results,
                             &c->h_cigars, &c->dense, &c->scan})
         b += d->bytes;
     *bytes = b + c->retired_bytes;

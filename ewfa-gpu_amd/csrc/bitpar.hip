@@ -828,8 +828,14 @@ __device__ __forceinline__ uint64_t sign_mask(uint32_t planes, int i) {
     return (uint64_t)(int64_t)m;
 }
 
-__device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen, int tlen) {
+// The bound, and in `slope` the least growth of the window's middle value over
+// SLOPE_BLOCKS column blocks (the edit rate while the window was on the path;
+// unchanged when the text has fewer).
+constexpr int SLOPE_BLOCKS = 32;
+
+__device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen, int tlen, int& slope) {
     const int nwp = (plen + 31) >> 5;
+    int mid0 = 0;
     LaneBand b{~0ull << 32, ~0ull >> 32, 32, -32};
     uint32_t a[4], c[4];  // pattern planes from row r0 & ~31
     const auto load = [&]() {
@@ -875,6 +881,11 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
             b.vn >>= -up;
         }
         b.r0 -= up;
+        if ((j & (SLOPE_BLOCKS - 1)) == SLOPE_BLOCKS - 1) {
+            const int mid = b.sc + __popc((uint32_t)b.vp) - __popc((uint32_t)b.vn);
+            slope = min(slope, mid - mid0);
+            mid0 = mid;
+        }
     }
     const int rest = tlen & 31;
     if (rest) {
@@ -896,16 +907,17 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
 
 // Whether a list takes the bit-parallel way at all, from a sample: 64 of its
 // pairs, a lane each, and the edits in the first PROBE_BASES of each.  The
-// wavefront's time is its work, or its longest pair's levels of about 0.45 us
-// each; the bit-parallel one its work, or its longest pair's columns of about
-// 0.4 us (bounds, table and path).  (Short lists of moderate lengths go faster
+// wavefront's time is its work, or its longest pair's levels (about 0.4 us and
+// 0.5 ns a diagonal each, and 0.7 us an op for the stream), twice where the pass's
+// budget of levels defers the pair; the bit-parallel one its work, or its longest
+// pair's columns of about 0.35 us (bounds, table and path).  (Short lists of moderate lengths go faster
 // through the wavefront: jobs of 100..5,000 bp at 1..10% edits in batches of
 // 25,000 pairs 5.6 against 7.4 ms, while 15,001 pairs of 3..7 kbp at 8..15%
 // take 3.3 against 5.9.)  The sample takes about 50 us.
 constexpr int PROBE_BASES = 512;
 
 __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
-                                                      uint32_t count, uint32_t* flag) {
+                                                      uint32_t count, int budget, uint32_t* flag) {
     const uint32_t n = count_ptr ? *count_ptr : count;
     if (n == 0) return;
     const uint32_t item = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) / 128u);
@@ -914,7 +926,8 @@ __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* 
     float wfa = 0.f, bp = 0.f, levels = 0.f, columns = 0.f;
     if (pr.plen <= a.max_len && pr.tlen <= a.max_len && pr.tlen > 0u) {
         const int tl = min((int)pr.tlen, PROBE_BASES), pl = min((int)pr.plen, PROBE_BASES);
-        const uint32_t u = lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl);
+        int slope = 0;
+        const uint32_t u = lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl, slope);
         columns = (float)pr.tlen;
         levels = (float)u / (float)tl * columns;
         wfa = wavefront_cost(levels);
@@ -928,11 +941,12 @@ __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* 
     }
     // wave instructions a microsecond: 256 CUs at about 2.3 GHz
     const float us = (float)n / 64.0f / 590000.0f;
-    if (threadIdx.x == 0) *flag = fmaxf(bp * us, columns * 0.4f) < fmaxf(wfa * us, levels * 0.45f) ? 1u : 0u;
+    const float chain = levels * (1.1f + 0.0005f * levels) * (levels > (float)budget ? 2.0f : 1.0f);
+    if (threadIdx.x == 0) *flag = fmaxf(bp * us, columns * 0.35f) < fmaxf(wfa * us, chain) ? 1u : 0u;
 }
 
 __global__ __launch_bounds__(64, 4) void bp_bound_kernel(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
-                                                         uint32_t* bound, const uint32_t* list,
+                                                         uint32_t* bound, uint32_t* guess, const uint32_t* list,
                                                          const uint32_t* count_ptr, uint32_t count,
                                                          const uint32_t* flag) {
     if (flag && *flag == 0u) return;
@@ -940,10 +954,16 @@ __global__ __launch_bounds__(64, 4) void bp_bound_kernel(const uint64_t* words, 
     for (uint32_t item = blockIdx.x * 64u + threadIdx.x; item < n; item += gridDim.x * 64u) {
         const uint32_t pidx = list ? list[item] : item;
         const ewfa_pair_t pr = pairs[pidx];
-        uint32_t u = BOUND_NONE;
-        if (pr.plen <= max_len && pr.tlen <= max_len)
-            u = lane_bound(words + pr.pattern_off, words + pr.text_off, (int)pr.plen, (int)pr.tlen);
+        uint32_t u = BOUND_NONE, d = BOUND_NONE;
+        if (pr.plen <= max_len && pr.tlen <= max_len) {
+            int slope = 1 << 20;
+            u = lane_bound(words + pr.pattern_off, words + pr.text_off, (int)pr.plen, (int)pr.tlen, slope);
+            // a guess at the distance for when the window lost the path
+            if (slope < (1 << 20))
+                d = (uint32_t)((float)max(slope, 0) * 1.25f * (float)pr.tlen / (32.0f * SLOPE_BLOCKS)) + 64u;
+        }
         bound[pidx] = u;
+        guess[pidx] = min(u, d);
     }
 }
 
@@ -952,13 +972,13 @@ hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* lis
     if (count == 0) return hipSuccess;
     const uint32_t blocks = (count + 63u) / 64u;
     hipLaunchKernelGGL(bp_bound_kernel, dim3(blocks < max_grid ? blocks : max_grid), dim3(64), 0, stream, a.words,
-                       a.pairs, a.max_len, bound, list, count_ptr, count, a.flag);
+                       a.pairs, a.max_len, bound, a.guess, list, count_ptr, count, a.flag);
     return hipGetLastError();
 }
 
 hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
-                           uint32_t* flag, hipStream_t stream) {
-    hipLaunchKernelGGL(bp_probe_kernel, dim3(1), dim3(64), 0, stream, a, list, count_ptr, count, flag);
+                           int budget, uint32_t* flag, hipStream_t stream) {
+    hipLaunchKernelGGL(bp_probe_kernel, dim3(1), dim3(64), 0, stream, a, list, count_ptr, count, budget, flag);
     return hipGetLastError();
 }
 
@@ -966,35 +986,43 @@ hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t
 
 namespace {
 
-// The class of a pair with distance bound u: the narrowest band that holds
-// every path of u edits, or BP_CLASSES for the wavefront (no bound, no band wide
-// enough, or so few edits that the wavefront is cheaper).
-__device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& pr, uint32_t u) {
+// Lists below this leave the chip idle, and a call lasts as long as its longest
+// chain: a pair's levels (about 1.1 us and half a ns a diagonal each, its stream
+// included) or columns (0.25 us each).
+constexpr uint32_t BP_CHAIN_BELOW = 2048;
+
+// The class of a pair of a list of n: the narrowest band that holds every path
+// within its distance bound, or BP_CLASSES for the wavefront (no bound, or so few
+// edits that the wavefront is faster).
+// A bound beyond the widest band, or above a fifth of the text, mostly comes of a
+// search whose window lost the path at a long gap: it then says nothing of the
+// distance.  The guess from the part before the gap then says which way is the
+// faster, and a bound beyond the widest band takes that band, where the distance
+// most likely lies (if not the pair is deferred); without a guess such pairs stay
+// with the wavefront.
+__device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& pr, uint32_t pidx, uint32_t n) {
+    uint32_t u = a.bound[pidx];
     if (u == BOUND_NONE || pr.plen > a.max_len || pr.tlen > a.max_len || pr.tlen == 0u || pr.plen == 0u)
         return BP_CLASSES;
     const int tk = (int)pr.tlen - (int)pr.plen;
-    for (int c = BP_CLASSES - 1; c >= 0; --c) {
-        int S;
-        if (bp_band(bp_words(c), tk, S) >= (int)u) {
-            // wave instructions of either way
-            const float wfa = wavefront_cost((float)u);
-            const float bp = (float)pr.tlen * (bp_column_cost(c) + 2.0f) + 25.0f * (float)u;
-            return wfa < bp ? BP_CLASSES : c;
-        }
+    int S, c = BP_CLASSES - 1;
+    while (c > 0 && bp_band(bp_words(c), tk, S) < (int)u) --c;
+    const int L = bp_band(bp_words(c), tk, S);
+    if (L < (int)u || u > pr.tlen / 5u + 64u) {
+        if (!a.guess || L < 0) return BP_CLASSES;
+        u = a.guess[pidx];
     }
-    // A bound beyond the widest band mostly comes of a window that lost the
-    // path at a long gap (values then grow at the rate of unrelated sequences,
-    // several times that of 10..15% edits): the distance is likely within the
-    // band, and a pair whose is not has wasted little next to the wavefront
-    // passes it goes on to.
-    int S;
-    return bp_band(bp_words(0), tk, S) >= 0 ? 0 : BP_CLASSES;
+    const float d = (float)u, cols = (float)pr.tlen;
+    const bool wave = n < BP_CHAIN_BELOW
+                          ? d * (1.1f + 0.0005f * d) < cols * 0.25f
+                          : wavefront_cost(d) < cols * (bp_column_cost(c) + 2.0f) + 25.0f * d;
+    return wave ? BP_CLASSES : c;
 }
 
 // Bin of a pair in the sort: its class, then its length, longest first.
-__device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, uint32_t u) {
+__device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, uint32_t n) {
     const ewfa_pair_t pr = a.pairs[pidx];
-    const int c = a.flag && *a.flag == 0u ? BP_CLASSES : bp_class_of(a, pr, u);
+    const int c = a.flag && *a.flag == 0u ? BP_CLASSES : bp_class_of(a, pr, pidx, n);
     const uint32_t b = min((uint32_t)((uint64_t)pr.tlen * BP_LEN_BINS / (a.max_len + 1u)), (uint32_t)BP_LEN_BINS - 1u);
     return c * BP_LEN_BINS + (int)(BP_LEN_BINS - 1u - b);
 }
@@ -1013,7 +1041,7 @@ __global__ __launch_bounds__(256) void bp_count_kernel(BpArgs a, const uint32_t*
     const uint32_t at = base + threadIdx.x;
     if (at < n) {
         const uint32_t pidx = list ? list[at] : at;
-        atomicAdd(&h[bp_bin_of(a, pidx, a.bound[pidx])], 1u);
+        atomicAdd(&h[bp_bin_of(a, pidx, n)], 1u);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < BP_BINS; i += 256)
@@ -1048,7 +1076,7 @@ __global__ __launch_bounds__(256) void bp_place_kernel(BpArgs a, const uint32_t*
     uint32_t pidx = 0, local = 0;
     if (item < n) {
         pidx = list ? list[item] : item;
-        b = bp_bin_of(a, pidx, a.bound[pidx]);
+        b = bp_bin_of(a, pidx, n);
         local = atomicAdd(&h[b], 1u);
     }
     __syncthreads();

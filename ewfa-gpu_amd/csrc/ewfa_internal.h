@@ -212,6 +212,7 @@ struct BpArgs {
     int8_t* cigars;
     uint32_t max_len;
     const uint32_t* bound;    // per pair
+    uint32_t* guess;          // per pair, a guess at the distance (null: none)
     const uint32_t* flag;     // 0: the whole list is the wavefront's (null: no)
     uint32_t* bins;           // BP_BINS counts and BP_BINS cursors, zero at first
     uint32_t* cursors;
@@ -235,9 +236,10 @@ struct BpArgs {
 // pairs' tokens, and per block of 32 columns up to four words a lane of 16 bytes.
 inline size_t bp_tok_bytes() { return 4u * 8u * (size_t)BP_TOK_STRIDE(64) / 4u; }
 inline size_t bp_rec_bytes(uint32_t max_len) { return (size_t)(max_len / 32u + 1u) * 64u * 4u * 16u; }
-// *flag = 1 when a sample of the list says the bit-parallel way is the faster.
+// *flag = 1 when a sample of the list says the bit-parallel way is the faster
+// (budget: the levels of the wavefront pass).
 hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
-                           uint32_t* flag, hipStream_t stream);
+                           int budget, uint32_t* flag, hipStream_t stream);
 // Upper bounds on the distances of a list's pairs, a lane each.
 hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* list, const uint32_t* count_ptr,
                            uint32_t count, uint32_t max_grid, hipStream_t stream);
