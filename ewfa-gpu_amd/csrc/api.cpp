@@ -956,6 +956,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.rest_count = ctl + BP_REST;
                 x.queue = ctl + BP_QUEUE;
                 x.spread = p.bp_spread;
+                x.budget = p.dcap;
                 x.defer_list = sx.list_a;
                 x.defer_count = ctrl + CTRL_DEFER_A;
                 x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;

@@ -988,7 +988,7 @@ namespace {
 
 // Lists below this leave the chip idle, and a call lasts as long as its longest
 // chain: a pair's levels (about 1.1 us and half a ns a diagonal each, its stream
-// included) or columns (0.25 us each).
+// included; twice where the pass's budget of levels defers it) or columns (0.25 us each).
 constexpr uint32_t BP_CHAIN_BELOW = 2048;
 
 // The class of a pair of a list of n: the narrowest band that holds every path
@@ -1014,7 +1014,7 @@ __device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& p
     }
     const float d = (float)u, cols = (float)pr.tlen;
     const bool wave = n < BP_CHAIN_BELOW
-                          ? d * (1.1f + 0.0005f * d) < cols * 0.25f
+                          ? d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f) < cols * 0.25f
                           : wavefront_cost(d) < cols * (bp_column_cost(c) + 2.0f) + 25.0f * d;
     return wave ? BP_CLASSES : c;
 }

@@ -223,6 +223,7 @@ struct BpArgs {
     uint32_t* rest_count;
     uint32_t* queue;          // work counters of the wide and the narrow classes
     int spread;               // bp_group
+    int budget;               // levels of the wavefront pass over the rest
     uint32_t* defer_list;
     uint32_t* defer_count;
     uint8_t* slots;           // per block: tok_bytes of tokens, then the records
