@@ -314,9 +314,9 @@ void choose_band_cap(ewfa_ctx* c, Pass& p) {
     p.band_cap = std::min(cap, p.dcap);
 }
 
-// Bytes of slots a bit-parallel pass may hold: at 50 kbp (4.1 MB a slot) three
+// Bytes of slots a bit-parallel pass may hold: at 50 kbp (6.5 MB a slot) four
 // waves per SIMD.
-constexpr size_t BP_BUDGET = (size_t)20 << 30;
+constexpr size_t BP_BUDGET = (size_t)26 << 30;
 
 // Pairs from which a list's distance bounds are searched a lane per pair
 // (bp_bound_kernel), below that a wave per pair: a lane's search lasts as long

@@ -416,14 +416,16 @@ struct TraceShape {
     static constexpr int TW = GL >= 32 ? 4 : 2, TB = GL >= 32 ? 8 : GL / TW, RL = 16;
     static constexpr int TILES = GL >= 32 ? TW * TB : 64;  // of the wave
 };
-constexpr int TILE_WORDS = 32;  // uint2 per tile, column c of tile t at c ^ (t & 31)
+// uint2 per tile; column c of tile t at c ^ tile_swizzle(t), which keeps pairs of
+// columns together and spreads the tiles over the banks
+constexpr int TILE_WORDS = 32;
+__device__ __forceinline__ int tile_swizzle(int t) { return (t & 15) << 1; }
 
 // Codes of one tile: pv, mv the word's deltas before the block, h the
 // horizontal deltas above it, p0, p1 and T0, T1 the pattern's and text's planes.
 __device__ __forceinline__ void trace_tile(uint32_t pv, uint32_t mv, uint2 h, uint32_t p0, uint32_t p1, uint32_t T0,
                                            uint32_t T1, uint2* out, int swz) {
-#pragma unroll 4
-    for (int i = 0; i < 32; ++i) {
+    const auto column = [&](int i) -> uint2 {
         const uint32_t c0 = (uint32_t)((int)(T0 << (31 - i)) >> 31);
         const uint32_t c1 = (uint32_t)((int)(T1 << (31 - i)) >> 31);
         const uint32_t E = ~(p0 ^ c0) & ~(p1 ^ c1);
@@ -432,14 +434,19 @@ __device__ __forceinline__ void trace_tile(uint32_t pv, uint32_t mv, uint2 h, ui
         const uint32_t Xh = (((Eq & pv) + pv) ^ pv) | Eq;
         const uint32_t Ph = mv | ~(Xh | pv), Mh = pv & Xh;
         const uint32_t D0 = Xh | mv;  // diagonal delta 0
-        const uint32_t ps = (Ph << 1) | (h.x >> 31), ms = (Mh << 1) | (h.y >> 31);
+        const uint32_t ps = __builtin_amdgcn_alignbit(Ph, h.x, 31), ms = __builtin_amdgcn_alignbit(Mh, h.y, 31);
         h.x <<= 1;
         h.y <<= 1;
         pv = ms | ~(Xv | ps);
         mv = ps & Xv;
         // DEL 3: vertical +1; else SUB 2: diagonal +1; else INS 1: horizontal +1
         const uint32_t hi = pv | ~D0;
-        out[i ^ swz] = make_uint2(hi, pv | (Ph & ~hi));
+        return make_uint2(hi, pv | (Ph & ~hi));
+    };
+#pragma unroll 4
+    for (int i = 0; i < 32; i += 2) {
+        const uint2 a = column(i), b = column(i + 1);
+        *reinterpret_cast<uint4*>(out + (i ^ swz)) = make_uint4(a.x, a.y, b.x, b.y);
     }
 }
 
@@ -515,14 +522,14 @@ __device__ __forceinline__ int bp_walk_wave(const BpPair& p, const BpSegs& sg, i
             const bool in = J >= 0 && idx >= 0 && idx < GL * w;
             tm = __builtin_amdgcn_ballot_w64(in);
             group_sync<1>();
-            if (in && lane < T::TILES) bp_tile(p, rec, J, idx, S, w, at, lane0, tiles + t * TILE_WORDS, t & 31);
+            if (in && lane < T::TILES) bp_tile(p, rec, J, idx, S, w, at, lane0, tiles + t * TILE_WORDS, tile_swizzle(t));
             group_sync<1>();
             have = true;
         }
         const int r = rho - lane, g = gam - lane;
         const int Jc = g >> 5, q = j0 - Jc, u = (r >> 5) - Jc - base, t = q * T::TW + u;
         const bool in = r >= 0 && g >= 0 && q < T::TB && (unsigned)u < (unsigned)T::TW && ((tm >> (t & 63)) & 1u);
-        const uint2 cc = tiles[in ? t * TILE_WORDS + ((g & 31) ^ (t & 31)) : 0];
+        const uint2 cc = tiles[in ? t * TILE_WORDS + ((g & 31) ^ tile_swizzle(t)) : 0];
         const uint64_t hib = __builtin_amdgcn_ballot_w64(in && ((cc.x >> (r & 31)) & 1u));
         const uint64_t lob = __builtin_amdgcn_ballot_w64(in && ((cc.y >> (r & 31)) & 1u));
         const uint64_t out = __builtin_amdgcn_ballot_w64(!in);
@@ -564,13 +571,28 @@ __device__ __forceinline__ int bp_walk_wave(const BpPair& p, const BpSegs& sg, i
     return cnt;
 }
 
+// The least key of a group of GL lanes (8 or 16), in every lane of it: lanes
+// paired by DPP (the other of two, of two twos, the mirrored half row and row).
+template <int GL>
+__device__ __forceinline__ uint32_t group_min(uint32_t k) {
+    k = min(k, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k, 0xB1, 0xF, 0xF, true));   // quad_perm 1,0,3,2
+    k = min(k, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k, 0x4E, 0xF, 0xF, true));   // quad_perm 2,3,0,1
+    k = min(k, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k, 0x141, 0xF, 0xF, true));  // row_half_mirror
+    if constexpr (GL == 16) k = min(k, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k, 0x140, 0xF, 0xF, true));  // row_mirror
+    return k;
+}
+
 // The path of the lane's pair as tokens (run << 2 | op), last op first, at tok.
 // Returns the edits (-1: more than p.L) and in `run` the matches before the
 // first op.
+// A step: each lane looks at RL/GL cells of the path's diagonal and makes a key of
+// the first that is an op or outside the tiles (steps back << 2 | op, op 0:
+// outside); the group's least key is the next event.
 template <int GL>
 __device__ __forceinline__ int bp_walk(const BpPair& p, bool mine, const BpSegs& sg, const uint2* rec, uint32_t* tok,
                                        uint2* tiles, int& run, int lane) {
     typedef TraceShape<GL> T;
+    static_assert(GL <= 16, "a group's tiles are one 16-bit mask");
     const int gl = lane & (GL - 1), g0 = lane & ~(GL - 1);
     int rho = p.plen - 1, gam = p.tlen - 1;  // the cell's row and column, from 0
     int cnt = 0;
@@ -588,54 +610,55 @@ __device__ __forceinline__ int bp_walk(const BpPair& p, bool mine, const BpSegs&
         int S, w, at;
         bp_segment_of(sg, J, S, w, at);
         const int idx = base + gl % T::TW - S;  // word of the band
-        const bool have = go && J >= 0 && idx >= 0 && idx < GL * w;
-        const uint64_t tm = group_bits<GL>(__builtin_amdgcn_ballot_w64(have), lane);
+        // (a word above row 0 is outside: the path ends there)
+        const bool have = go && J >= 0 && idx >= 0 && idx < GL * w && J + S + idx >= 0;
+        const uint32_t tm = (uint32_t)group_bits<GL>(__builtin_amdgcn_ballot_w64(have), lane);
         group_sync<1>();
-        if (have) bp_tile(p, rec, J, idx, S, w, at, g0, my, lane & 31);
+        if (have) bp_tile(p, rec, J, idx, S, w, at, g0, my, tile_swizzle(lane));
         group_sync<1>();
+        // the lane's first cell, in columns left of the tiles' last column (G)
+        // and rows below their first row (R)
+        int G = 32 * j0 + 31 - gam + gl, R = rho - 32 * (j0 + base) - gl;
+        const int G0 = G, R0 = R;
         bool fresh = true;
         while (__builtin_amdgcn_ballot_w64(go)) {
-            uint64_t hb = 0, lb = 0, ob = 0;  // by cells back: op bits, outside the tiles
+            uint32_t key = ~0u;
 #pragma unroll
-            for (int c = 0; c < T::RL; c += GL) {
-                const int r = rho - gl - c, g = gam - gl - c;
-                const int Jc = g >> 5, q = j0 - Jc, u = (r >> 5) - Jc - base, t = q * T::TW + u;
-                const bool in = r >= 0 && g >= 0 && q < T::TB && (unsigned)u < (unsigned)T::TW && ((tm >> (t & 63)) & 1u);
-                const uint2 cc = tiles[in ? (g0 + t) * TILE_WORDS + ((g & 31) ^ ((g0 + t) & 31)) : 0];
-                hb |= group_bits<GL>(__builtin_amdgcn_ballot_w64(in && ((cc.x >> (r & 31)) & 1u)), lane) << c;
-                lb |= group_bits<GL>(__builtin_amdgcn_ballot_w64(in && ((cc.y >> (r & 31)) & 1u)), lane) << c;
-                ob |= group_bits<GL>(__builtin_amdgcn_ballot_w64(!in), lane) << c;
+            for (int c = T::RL - GL; c >= 0; c -= GL) {
+                const int q = (G + c) >> 5, u = ((R - c) >> 5) + q, t = q * T::TW + u;
+                const bool in = (unsigned)u < (unsigned)T::TW && ((tm >> (t & 31)) & 1u);
+                const uint2 cc = tiles[in ? (g0 + t) * TILE_WORDS + ((~(G + c) & 31) ^ tile_swizzle(g0 + t)) : 0];
+                const uint32_t b = (uint32_t)(R - c) & 31u;
+                const uint32_t op = in ? ((cc.x >> b) & 1u) << 1 | ((cc.y >> b) & 1u) : 0u;
+                if (!in || op) key = (uint32_t)(gl + c) << 2 | op;
             }
+            key = group_min<GL>(key);
+            const bool event = key != ~0u;
+            const int f = event ? (int)(key >> 2) : T::RL;
+            const uint32_t op = key & 3u;
+            const bool edit = event && op != 0u;
             if (go) {
-                const uint64_t stop = hb | lb | ob;
-                const int f = stop ? (int)__builtin_ctzll(stop) : T::RL;
+                // on to new tiles at a cell outside these, unless it is the
+                // first: then the path left the band, with more than L edits
+                lost = event && !edit && fresh && f == 0;
+                go = !event || edit;
                 run += f;
-                rho -= f;
-                gam -= f;
-                if (stop) {
-                    if ((ob >> f) & 1u) {
-                        // on to new tiles, unless the path left the band: then
-                        // it has more than L edits
-                        lost = lost || (fresh && f == 0);
-                        go = false;
-                    } else {
-                        const int op = (int)((hb >> f) & 1u) * 2 + (int)((lb >> f) & 1u);
-                        if (cnt >= p.L) {
-                            lost = true;
-                            go = false;
-                        } else {
-                            if (gl == 0) tok[cnt] = (uint32_t)(run << 2 | op);
-                            ++cnt;
-                            run = 0;
-                            rho -= op != OP_INS;
-                            gam -= op != OP_DEL;
-                        }
-                    }
+                if (edit) {
+                    if (gl == 0) tok[cnt] = (uint32_t)run << 2 | op;
+                    ++cnt;
+                    run = 0;
                 }
-                go = go && rho >= 0 && gam >= 0;
+                G += f + (edit && op != OP_DEL);
+                R -= f + (edit && op != OP_INS);
+                if (cnt > p.L) {
+                    lost = true;
+                    go = false;
+                }
             }
             fresh = false;
         }
+        gam -= G - G0;
+        rho += R - R0;
     }
     if (!mine || lost) return -1;
     // rows or columns before the other's first
