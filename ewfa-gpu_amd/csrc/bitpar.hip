@@ -832,24 +832,31 @@ struct LaneBand {
     int r0;  // the window's first row (from 0) at the next column
 };
 
-// One column: p0, p1 the window's pattern planes, c0, c1 the text base's masks;
-// returns bit 0 of the diagonal-delta-0 vector (of the first row).
-__device__ __forceinline__ uint32_t band_column(LaneBand& b, uint64_t p0, uint64_t p1, uint64_t c0, uint64_t c1) {
-    const uint64_t eq = ~(p0 ^ c0) & ~(p1 ^ c1);
-    const uint64_t xh = (((eq & b.vp) + b.vp) ^ b.vp) | eq;
-    const uint64_t ph = b.vn | ~(xh | b.vp);
-    const uint64_t mh = b.vp & xh;
-    const uint64_t d0 = (uint64_t)((uint32_t)xh | (uint32_t)b.vn);
-    const uint64_t xv = (eq | b.vn) >> 1;
-    b.vp = mh | ~(xv | ph);
-    b.vn = ph & xv;
-    return (uint32_t)d0;
+// One column over 32-bit halves (64-bit shifts and adds take several cycles a
+// lane): p, q the window's pattern planes' halves, c0, c1 the text base's masks;
+// returns the low half of the diagonal-delta-0 vector (bit 0: the first row).
+__device__ __forceinline__ uint32_t band_column(uint32_t (&vp)[2], uint32_t (&vn)[2], const uint32_t (&p)[2],
+                                                const uint32_t (&q)[2], uint32_t c0, uint32_t c1) {
+    uint32_t xh[2], ph[2], mh[2], xv[2];
+    unsigned c = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t eq = ~(p[h] ^ c0) & ~(q[h] ^ c1);
+        xh[h] = (__builtin_addc(eq & vp[h], vp[h], c, &c) ^ vp[h]) | eq;
+        ph[h] = vn[h] | ~(xh[h] | vp[h]);
+        mh[h] = vp[h] & xh[h];
+        xv[h] = eq | vn[h];
+    }
+    const uint32_t d0 = xh[0] | vn[0];
+    const uint32_t x0 = __builtin_amdgcn_alignbit(xv[1], xv[0], 1), x1 = xv[1] >> 1;
+    vp[0] = mh[0] | ~(x0 | ph[0]);
+    vp[1] = mh[1] | ~(x1 | ph[1]);
+    vn[0] = ph[0] & x0;
+    vn[1] = ph[1] & x1;
+    return d0;
 }
 
-__device__ __forceinline__ uint64_t sign_mask(uint32_t planes, int i) {
-    const int m = (int)(planes << (31 - i)) >> 31;
-    return (uint64_t)(int64_t)m;
-}
+__device__ __forceinline__ uint32_t sign_mask(uint32_t planes, int i) { return (uint32_t)((int)(planes << (31 - i)) >> 31); }
 
 // The bound, and in `slope` the least growth of the window's middle value over
 // SLOPE_BLOCKS column blocks (the edit rate while the window was on the path;
@@ -873,9 +880,10 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
             c[x] = __builtin_amdgcn_alignbit(c[x + 1], c[x], sh);
         }
     };
-    const auto window = [&](const uint32_t (&v)[4], int i) -> uint64_t {
-        return (uint64_t)__builtin_amdgcn_alignbit(v[1], v[0], (uint32_t)i) |
-               ((uint64_t)__builtin_amdgcn_alignbit(v[2], v[1], (uint32_t)i) << 32);
+    const auto column = [&](uint32_t (&vp)[2], uint32_t (&vn)[2], uint32_t t0, uint32_t t1, int i) -> uint32_t {
+        const uint32_t p[2] = {__builtin_amdgcn_alignbit(a[1], a[0], (uint32_t)i), __builtin_amdgcn_alignbit(a[2], a[1], (uint32_t)i)};
+        const uint32_t q[2] = {__builtin_amdgcn_alignbit(c[1], c[0], (uint32_t)i), __builtin_amdgcn_alignbit(c[2], c[1], (uint32_t)i)};
+        return band_column(vp, vn, p, q, sign_mask(t0, i), sign_mask(t1, i));
     };
     const int full = tlen >> 5;
     for (int j = 0; j < full; ++j) {
@@ -883,11 +891,11 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
         load();
         planes_of(gt[j], t0, t1);
         uint32_t z = 0;
-#pragma unroll 16
-        for (int i = 0; i < 32; ++i) {
-            const uint32_t d0 = band_column(b, window(a, i), window(c, i), sign_mask(t0, i), sign_mask(t1, i));
-            z = __builtin_amdgcn_alignbit(d0, z, 1);
-        }
+        uint32_t vp[2] = {(uint32_t)b.vp, (uint32_t)(b.vp >> 32)}, vn[2] = {(uint32_t)b.vn, (uint32_t)(b.vn >> 32)};
+#pragma unroll
+        for (int i = 0; i < 32; ++i) z = __builtin_amdgcn_alignbit(column(vp, vn, t0, t1, i), z, 1);
+        b.vp = (uint64_t)vp[1] << 32 | vp[0];
+        b.vn = (uint64_t)vn[1] << 32 | vn[0];
         b.sc += 32 - __popc(z);
         b.r0 += 32;
         // bottom edge's value less the top edge's, halved: rows to move up
@@ -915,8 +923,10 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
         uint32_t t0, t1;
         load();
         planes_of(gt[full], t0, t1);
-        for (int i = 0; i < rest; ++i)
-            b.sc += 1 - (int)(band_column(b, window(a, i), window(c, i), sign_mask(t0, i), sign_mask(t1, i)) & 1u);
+        uint32_t vp[2] = {(uint32_t)b.vp, (uint32_t)(b.vp >> 32)}, vn[2] = {(uint32_t)b.vn, (uint32_t)(b.vn >> 32)};
+        for (int i = 0; i < rest; ++i) b.sc += 1 - (int)(column(vp, vn, t0, t1, i) & 1u);
+        b.vp = (uint64_t)vp[1] << 32 | vp[0];
+        b.vn = (uint64_t)vn[1] << 32 | vn[0];
         b.r0 += rest;
     }
     // row plen - 1 of the last column
