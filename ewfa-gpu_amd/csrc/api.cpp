@@ -107,6 +107,7 @@ struct ewfa_ctx {
     size_t lds_max = 0;
     DevBuf ops, bt, ctrl, list_a, list_b, buckets, runs, list_fb, bound, gslot, order;
     DevBuf bp_list, bp_rest, bp_guess, bp_slots;  // bit-parallel passes
+    size_t bp_budget = SIZE_MAX;  // bytes of slots a bit-parallel pass may hold (less after a failed allocation)
     uint32_t* host_ctrl = nullptr;  // pinned mirror of the control words
     float align_ms = 0.f, emit_ms = 0.f;
     bool timing = false;
@@ -317,6 +318,9 @@ void choose_band_cap(ewfa_ctx* c, Pass& p) {
 // Bytes of slots a bit-parallel pass may hold: at 50 kbp (6.5 MB a slot) four
 // waves per SIMD.
 constexpr size_t BP_BUDGET = (size_t)26 << 30;
+// ... and the least for which the pass is worth its launches: where not even
+// that can be allocated, the pairs stay with the wavefront.
+constexpr size_t BP_LEAST = (size_t)256 << 20;
 
 // Pairs from which a list's distance bounds are searched a lane per pair
 // (bp_bound_kernel), below that a wave per pair: a lane's search lasts as long
@@ -341,8 +345,10 @@ void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     // decides on them (bp_probe_kernel)
     if (p.dcap < BOUND_MIN_DCAP && items < BP_PROBE_MIN) return;
     p.bp_spread = items < BP_SPREAD_BELOW ? 1 : 0;
+    const size_t budget = std::min(c->bp_budget, BP_BUDGET);
+    if (budget < BP_LEAST) return;
     p.bp_slot_bytes = ewfa::bp_tok_bytes() + ewfa::bp_rec_bytes(blen);
-    const uint64_t room = std::max<size_t>(BP_BUDGET / p.bp_slot_bytes, 1);
+    const uint64_t room = std::max<size_t>(budget / p.bp_slot_bytes, 1);
     const bool apart = p.dcap >= BOUND_MIN_DCAP;
     for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW}) {
         p.bp_part[part] = 0;
@@ -666,14 +672,23 @@ int reserve_bt(ewfa_ctx* c, const Pass& p) {
     return c->bt.reserve(c, p.slot_off + slot_bytes(p) * p.grid);
 }
 
-int reserve_plan(ewfa_ctx* c, const Plan& pl, size_t n) {
+int reserve_plan(ewfa_ctx* c, Plan& pl, size_t n) {
+    // slots for the bit-parallel passes, fewer when the device has no room for
+    // all (every later plan of the context then asks for fewer)
+    while (pl.bp_bytes && c->bp_slots.reserve(c, pl.bp_bytes) != EWFA_OK) {
+        (void)hipGetLastError();
+        g_err.clear();
+        c->bp_budget = std::min(c->bp_budget, BP_BUDGET) / 4;
+        ++c->policy_gen;
+        for (int b = 0; b < pl.nb; ++b) choose_bp(c, pl.pass[b], pl.blen[b], (uint32_t)n);
+        assign_slots(pl);
+    }
     CHK(c->runs.reserve(c, pl.runs_bytes));
     CHK(c->bt.reserve(c, pl.bt_bytes));
     CHK(c->gslot.reserve(c, pl.gslot_bytes));
     if (pl.nb > 1) CHK(c->buckets.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
     CHK(c->bound.reserve(c, std::max<size_t>(n, 1) * 4));
     if (pl.bp_bytes) {
-        CHK(c->bp_slots.reserve(c, pl.bp_bytes));
         CHK(c->bp_list.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
         CHK(c->bp_guess.reserve(c, std::max<size_t>(n, 1) * 4));
         CHK(c->bp_rest.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
