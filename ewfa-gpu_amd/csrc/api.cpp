@@ -1178,10 +1178,36 @@ int pipeline_upload(ewfa_ctx* c, const Chunk& ch, size_t k, const uint64_t* h_wo
     return EWFA_OK;
 }
 
+// Device address of `bytes` of host memory at p when they are pinned (one
+// allocation, by both ends), else null.
+template <typename T>
+T* mapped_host(T* p, size_t bytes) {
+    hipPointerAttribute_t a{}, b{};
+    char* const last = reinterpret_cast<char*>(p) + (bytes ? bytes - 1 : 0);
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&b, last) != hipSuccess) {
+        (void)hipGetLastError();  // ordinary memory
+        return nullptr;
+    }
+    if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || !a.devicePointer || !b.devicePointer ||
+        static_cast<char*>(b.devicePointer) - static_cast<char*>(a.devicePointer) != last - reinterpret_cast<char*>(p))
+        return nullptr;
+    return static_cast<T*>(a.devicePointer);
+}
+
+// The caller's output buffers of a host-pipeline call, and their device
+// addresses where they are pinned: such streams and results go straight to
+// their places, without the stage and the host threads that place it.
+struct HostOut {
+    ewfa_result_t* results;
+    int8_t* cigars;
+    ewfa_result_t* results_dev;
+    int8_t* cigars_dev;
+};
+
 // Enqueues chunk k on the compute stream, after its uploads: the persistent
 // plan, the compaction into the stage's pinned buffer and the results copy.
 // The stage must be free (its previous chunk placed by the host).
-int pipeline_enqueue(ewfa_ctx* c, const Chunk& ch, size_t k) {
+int pipeline_enqueue(ewfa_ctx* c, const Chunk& ch, size_t k, const HostOut& out) {
     uint64_t* d_words = c->h_words.as<uint64_t>();
     ewfa_pair_t* d_pairs = c->h_pairs.as<ewfa_pair_t>();
     ewfa_result_t* d_results = c->h_results.as<ewfa_result_t>();
@@ -1189,36 +1215,42 @@ int pipeline_enqueue(ewfa_ctx* c, const Chunk& ch, size_t k) {
     const size_t n = ch.hi - ch.lo;
     HIPCHK(hipStreamWaitEvent(c->stream, c->ev_up[k], 0));
     ewfa_ctx::Stage& st = c->stage[k & 1];
-    if (ch.caps > st.dense_cap || !st.dense) {
+    if (!out.cigars_dev && (ch.caps > st.dense_cap || !st.dense)) {
         CHK(grow_pinned(c, (void**)&st.dense, &st.dense_cap, ch.caps, true));
         void* dp = nullptr;
         HIPCHK(hipHostGetDevicePointer(&dp, st.dense, 0));
         st.dense_dev = static_cast<int8_t*>(dp);
     }
-    size_t res_bytes = st.res_cap;
-    CHK(grow_pinned(c, (void**)&st.res, &res_bytes, n * sizeof(ewfa_result_t), false));
-    st.res_cap = res_bytes;
+    if (!out.results_dev) {
+        size_t res_bytes = st.res_cap;
+        CHK(grow_pinned(c, (void**)&st.res, &res_bytes, n * sizeof(ewfa_result_t), false));
+        st.res_cap = res_bytes;
+    }
     Plan pl;
     CHK(reserve_scratch(c, n, ch.max_len));
     CHK(plan_persistent(c, ch.max_len, (uint32_t)n, pl));
     CHK(reserve_plan(c, pl, n));
     CHK(enqueue_plan(c, pl, d_words, d_pairs + ch.lo, (uint32_t)n, ch.max_len, d_results + ch.lo, d_cigars,
                      c->stream, false));
-    CHK(c->scan.reserve(c, 16 * ((n + ewfa::COMPACT_BLOCK - 1) / ewfa::COMPACT_BLOCK)));
-    HIPCHK(ewfa::launch_compact(d_pairs + ch.lo, d_results + ch.lo, d_cigars, n, c->scan.as<uint64_t>(), st.dense_dev,
-                                c->stream));
-    HIPCHK(hipMemcpyAsync(st.res, d_results + ch.lo, n * sizeof(ewfa_result_t), hipMemcpyDeviceToHost, c->stream));
+    if (out.cigars_dev) {
+        HIPCHK(ewfa::launch_place_streams(d_pairs + ch.lo, d_results + ch.lo, d_cigars, n, out.cigars_dev, c->stream));
+    } else {
+        CHK(c->scan.reserve(c, 16 * ((n + ewfa::COMPACT_BLOCK - 1) / ewfa::COMPACT_BLOCK)));
+        HIPCHK(ewfa::launch_compact(d_pairs + ch.lo, d_results + ch.lo, d_cigars, n, c->scan.as<uint64_t>(),
+                                    st.dense_dev, c->stream));
+    }
+    HIPCHK(hipMemcpyAsync(out.results_dev ? out.results + ch.lo : st.res, d_results + ch.lo, n * sizeof(ewfa_result_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipEventRecord(st.done, c->stream));
     return EWFA_OK;
 }
 
-int pipeline_complete(ewfa_ctx* c, const Chunk& ch, size_t k, const ewfa_pair_t* h_pairs, ewfa_result_t* h_results,
-                      int8_t* h_cigars) {
+int pipeline_complete(ewfa_ctx* c, const Chunk& ch, size_t k, const ewfa_pair_t* h_pairs, const HostOut& out) {
     ewfa_ctx::Stage& st = c->stage[k & 1];
     HIPCHK(hipEventSynchronize(st.done));
     const size_t n = ch.hi - ch.lo;
-    memcpy(h_results + ch.lo, st.res, n * sizeof(ewfa_result_t));
-    if (ewfa::scatter_streams(st.dense, ch.caps, h_pairs + ch.lo, h_results + ch.lo, n, h_cigars, 16) == SIZE_MAX)
+    if (!out.results_dev) memcpy(out.results + ch.lo, st.res, n * sizeof(ewfa_result_t));
+    if (!out.cigars_dev && ewfa::scatter_streams(st.dense, ch.caps, h_pairs + ch.lo, out.results + ch.lo, n,
+                                                 out.cigars, 16) == SIZE_MAX)
         return fail(EWFA_ERR_STATE, "compacted streams exceed their regions");
     return EWFA_OK;
 }
@@ -1270,8 +1302,9 @@ int run_pipeline(ewfa_ctx* c, const uint64_t* h_words, size_t n_words, const ewf
         while (ch.hi < n && ch.hi - ch.lo < per &&
                (ch.hi == ch.lo || ch.caps + h_pairs[ch.hi].cigar_cap <= PIPE_CAPS)) {
             const ewfa_pair_t& p = h_pairs[ch.hi];
-            if (p.pattern_off + ewfa_packed_words(p.plen) - 1 > n_words ||
-                p.text_off + ewfa_packed_words(p.tlen) - 1 > n_words) {
+            // words read: up to the pad word (a sequence's last may be the upload's)
+            const uint64_t pe = p.pattern_off + ewfa::packed_words(p.plen), te = p.text_off + ewfa::packed_words(p.tlen);
+            if (pe - 1 > n_words || te - 1 > n_words) {
                 rc = fail(EWFA_ERR_ARG, "pair %zu reads past the packed words", ch.hi);
                 break;
             }
@@ -1280,8 +1313,7 @@ int run_pipeline(ewfa_ctx* c, const uint64_t* h_words, size_t n_words, const ewf
                 break;
             }
             ch.w_lo = std::min<size_t>(ch.w_lo, std::min(p.pattern_off, p.text_off));
-            ch.w_hi = std::max<size_t>(ch.w_hi, std::max(p.pattern_off + ewfa_packed_words(p.plen),
-                                                         p.text_off + ewfa_packed_words(p.tlen)));
+            ch.w_hi = std::max<size_t>(ch.w_hi, std::max(pe, te));
             ch.caps += p.cigar_cap;
             ch.max_len = std::max(ch.max_len, std::max(p.plen, p.tlen));
             ++ch.hi;
@@ -1299,17 +1331,19 @@ int run_pipeline(ewfa_ctx* c, const uint64_t* h_words, size_t n_words, const ewf
     // size the per-chunk scratch for the largest chunk before any chunk
     // computes, so that no buffer is replaced while chunks are in flight
     if (rc == EWFA_OK) rc = reserve_scratch(c, most, max_len);
+    const HostOut out{h_results, h_cigars, mapped_host(h_results, n * sizeof(ewfa_result_t)),
+                      mapped_host(h_cigars, cigar_bytes)};
     size_t enq = 0, done = 0;
     for (size_t k = 0; k < chunks.size() && rc == EWFA_OK; ++k) {
         if (!h_words) rc = words_wait(c, chunks[k].w_hi);
-        if (rc == EWFA_OK) rc = pipeline_enqueue(c, chunks[k], k);
+        if (rc == EWFA_OK) rc = pipeline_enqueue(c, chunks[k], k, out);
         if (rc == EWFA_OK) ++enq;
         if (rc == EWFA_OK && k >= 1) {
-            rc = pipeline_complete(c, chunks[k - 1], k - 1, h_pairs, h_results, h_cigars);
+            rc = pipeline_complete(c, chunks[k - 1], k - 1, h_pairs, out);
             if (rc == EWFA_OK) ++done;
         }
     }
-    if (rc == EWFA_OK && done < enq) rc = pipeline_complete(c, chunks[enq - 1], enq - 1, h_pairs, h_results, h_cigars);
+    if (rc == EWFA_OK && done < enq) rc = pipeline_complete(c, chunks[enq - 1], enq - 1, h_pairs, out);
     if (rc != EWFA_OK) {
         // leave nothing in flight that uses the context's buffers
         (void)hipStreamSynchronize(c->up);

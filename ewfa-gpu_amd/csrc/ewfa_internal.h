@@ -322,6 +322,12 @@ hipError_t launch_bucketize(const ewfa_pair_t* pairs, uint32_t n, const BucketTa
 // `scan` holds 2 * ceil(n / COMPACT_BLOCK) words.
 hipError_t launch_compact(const ewfa_pair_t* pairs, const ewfa_result_t* results, const int8_t* cigars, size_t n,
                           uint64_t* scan, int8_t* dense, hipStream_t stream);
+// Copies every pair's written CIGAR bytes to its place in host memory mapped
+// for the device.
+hipError_t launch_place_streams(const ewfa_pair_t* pairs, const ewfa_result_t* results, const int8_t* cigars, size_t n,
+                                int8_t* host, hipStream_t stream);
+// Words of a packed sequence and its pad word (ewfa_packed_words, inlined).
+inline size_t packed_words(uint32_t len) { return ((size_t)len + 31) / 32 + 1; }
 // Waves per pair of the passes with their slots in HBM.
 constexpr int GSLOT_WAVES = 16;
 // Resident blocks per CU of a block-kernel variant (0: backtrace in HBM, 1: in

@@ -2096,6 +2096,22 @@ __global__ __launch_bounds__(256) void compact_copy_kernel(const ewfa_pair_t* pa
     }
 }
 
+// The written bytes of every pair's region straight into its place in the
+// caller's buffer, host memory the device can write: 16 lanes per pair, so that
+// a store of theirs is a 64-byte transfer.
+__global__ __launch_bounds__(256) void place_streams_kernel(const ewfa_pair_t* pairs, const ewfa_result_t* results,
+                                                            const int8_t* cigars, size_t n, int8_t* host) {
+    const uint32_t part = threadIdx.x & 15u;
+    const size_t stride = (size_t)gridDim.x * 16u;
+    for (size_t i = (size_t)blockIdx.x * 16u + (threadIdx.x >> 4); i < n; i += stride) {
+        const ewfa_pair_t p = pairs[i];
+        const uint32_t nd = written_cigar_bytes(results[i], p) >> 2;
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(cigars + p.cigar_off);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(host + p.cigar_off);
+        for (uint32_t q = part; q < nd; q += 16u) dst[q] = src[q];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // pack and fill
 
@@ -2381,6 +2397,15 @@ hipError_t launch_compact(const ewfa_pair_t* pairs, const ewfa_result_t* results
     hipLaunchKernelGGL(compact_scan_kernel, dim3(1), dim3(256), 0, stream, bsum, boff, (uint32_t)nb);
     hipLaunchKernelGGL(compact_copy_kernel, dim3((unsigned)nb), dim3(256), 0, stream, pairs, results, cigars, n,
                        boff, dense);
+    return hipGetLastError();
+}
+
+hipError_t launch_place_streams(const ewfa_pair_t* pairs, const ewfa_result_t* results, const int8_t* cigars, size_t n,
+                                int8_t* host, hipStream_t stream) {
+    if (n == 0) return hipSuccess;
+    const size_t blocks = (n + 15) / 16;
+    hipLaunchKernelGGL(place_streams_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
+                       pairs, results, cigars, n, host);
     return hipGetLastError();
 }
 
