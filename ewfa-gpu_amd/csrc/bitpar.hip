@@ -450,9 +450,6 @@ __device__ __forceinline__ void trace_tile(uint32_t pv, uint32_t mv, uint2 h, ui
     }
 }
 
-// Bytes of a run of r matches in the stream.
-__device__ __forceinline__ int run_bytes(int r) { return (r + 126) / 127; }
-
 // A group's bits of a wave mask.
 template <int GL>
 __device__ __forceinline__ uint64_t group_bits(uint64_t m, int lane) {
@@ -688,39 +685,16 @@ __device__ __forceinline__ void bp_emit(const BpArgs& a, uint32_t pidx, int cnt,
         return;
     }
     // step s's run and op from tokens cnt - s and cnt - 1 - s
-    int8_t* out = a.cigars + coff;
-    uint32_t at0 = 0;
-    const auto put_run = [&](uint32_t at, int rb) -> uint32_t {
-        for (; rb >= 127; rb -= 127, ++at)
-            if (at < cap) out[at] = (int8_t)-127;
-        if (rb) {
-            if (at < cap) out[at] = (int8_t)-rb;
-            ++at;
-        }
-        return at;
-    };
+    WaveStream w{a.cigars + coff, cap, 0u};
     for (int s0 = 0; s0 < cnt; s0 += 64) {
         const int s = s0 + lane;
         const bool act = s < cnt;
         const int op = act ? (int)(tok[cnt - 1 - s] & 3u) : 0;
-        const int rb = !act ? 0 : s == 0 ? run : (int)(tok[cnt - s] >> 2);
-        const int nb = act ? run_bytes(rb) + 1 : 0;
-        const int incl = wave_incl_scan_i32(nb);
-        if (act) {
-            const uint32_t at = put_run(at0 + (uint32_t)(incl - nb), rb);
-            if (at < cap) out[at] = (int8_t)(op == OP_DEL ? 'D' : op == OP_SUB ? 'X' : 'I');
-        }
-        at0 += (uint32_t)__builtin_amdgcn_readlane(incl, 63);
+        w.put(act, !act ? 0 : s == 0 ? run : (int)(tok[cnt - s] >> 2), op);
     }
-    const int fin = cnt ? (int)(tok[0] >> 2) : run;
-    const uint32_t len = at0 + (uint32_t)run_bytes(fin);
-    if (lane == 0) {
-        put_run(at0, fin);
-        // the terminator: zeros to the end of its dword, inside the region
-        const uint32_t end = min((len & ~3u) + 4u, cap);
-        for (uint32_t i = len; i < end; ++i) out[i] = 0;
-        *res = ewfa_result_t{cnt, (int32_t)len, len > cap ? EWFA_PAIR_OVERFLOW : EWFA_PAIR_OK, 0};
-    }
+    w.finish(cnt ? (int)(tok[0] >> 2) : run, lane);
+    if (lane == 0)
+        *res = ewfa_result_t{cnt, (int32_t)w.len, w.len > cap ? EWFA_PAIR_OVERFLOW : EWFA_PAIR_OK, 0};
 }
 
 // One wave's pairs: list[first ..] up to 64/GL of them, below `end`, of bands of

@@ -62,4 +62,49 @@ __device__ __forceinline__ int wave_incl_scan_i32(int x) {
     return x;
 }
 
+// ---- CIGAR streams written by a wave -----------------------------------------
+
+// Stream bytes of a match run of r bases: floor(r/127) bytes of -127, then
+// -(r%127) when nonzero (src/kernels.cu:436-446).
+__device__ __forceinline__ int run_bytes(int r) { return (r + 126) / 127; }
+
+// A pair's stream region and the bytes of the stream so far (uniform).
+struct WaveStream {
+    int8_t* out;
+    uint32_t cap, len;
+
+    // a run at `at`, bytes at or past the region's end dropped
+    __device__ __forceinline__ uint32_t put_run(uint32_t at, int r) const {
+        for (; r >= 127; r -= 127, ++at)
+            if (at < cap) out[at] = (int8_t)-127;
+        if (r) {
+            if (at < cap) out[at] = (int8_t)-r;
+            ++at;
+        }
+        return at;
+    }
+    // lane by lane, a run and the op (OP_*) after it; lanes with act false add
+    // nothing
+    __device__ __forceinline__ void put(bool act, int run, int op) {
+        const int nb = act ? run_bytes(run) + 1 : 0;
+        const int incl = wave_incl_scan_i32(nb);
+        if (act) {
+            const uint32_t at = put_run(len + (uint32_t)(incl - nb), run);
+            if (at < cap) out[at] = (int8_t)(op == 3 ? 'D' : op == 2 ? 'X' : 'I');
+        }
+        len += (uint32_t)__builtin_amdgcn_readlane(incl, 63);
+    }
+    // the last run and the terminator (zeros to the end of its dword, inside
+    // the region), by one lane
+    __device__ __forceinline__ void finish(int run, int lane) {
+        const uint32_t end = len + (uint32_t)run_bytes(run);
+        if (lane == 0) {
+            put_run(len, run);
+            const uint32_t stop = min((end & ~3u) + 4u, cap);
+            for (uint32_t i = end; i < stop; ++i) out[i] = 0;
+        }
+        len = end;
+    }
+};
+
 }  // namespace ewfa
