@@ -83,7 +83,8 @@ enum : int {
     BP_REST = BP_SEG + ewfa::BP_CLASSES + 1,
     BP_QUEUE = BP_REST + 1,
     BP_FLAG = BP_QUEUE + 2,
-    BP_CTRL = (BP_FLAG + 1 + 31) & ~31,
+    BP_WEIGH = (BP_FLAG + 2) & ~1,
+    BP_CTRL = (BP_WEIGH + (int)(sizeof(ewfa::BpWeigh) / 4) + 31) & ~31,
     CTRL_WORDS = CTRL_BP + ewfa::MAX_BUCKETS * BP_CTRL
 };
 
@@ -94,6 +95,7 @@ struct ewfa_ctx {
     ewfa_opts_t opts{};
     std::string policy_path;
     ewfa::Policy policy;
+    bool builtin_policy = true;
     hipStream_t stream = nullptr;
     hipEvent_t ev_in = nullptr, ev_a0 = nullptr, ev_a1 = nullptr, ev_e1 = nullptr;
     // the persistent plan's bucket passes spread over `fanout` streams: the
@@ -295,6 +297,14 @@ void choose_off16(Pass& p, uint32_t max_len) {
     p.off16 = (!p.reg && !p.bt_lds && p.dcap < BOUND_MIN_DCAP && (size_t)max_len + (size_t)p.dcap <= 16383) ? 1 : 0;
 }
 
+// A pair per CU or less goes without distance bounds up to 40 kbp: their search
+// lengthens the longest pair's chain by more than the cells it saves (60 pairs of
+// 10..30 kbp 4,376 -> 3,736 us, 8 of 20..40 kbp 2,318 -> 1,657, 250 of 40..60 kbp
+// 9,513 and 9,715).
+bool unbounded(const ewfa_ctx* c, uint32_t max_len, uint32_t n) {
+    return n > 0 && n <= (uint32_t)c->num_cus && max_len <= 40000u;
+}
+
 // A bounded block pass (a budget of BOUND_MIN_DCAP levels or more, sequences
 // of at most BOUND_MAX_SEQ_WORDS words) whose slot lets fewer blocks share a
 // CU than its narrow slot would: narrow slots sized for one block more per
@@ -302,9 +312,9 @@ void choose_off16(Pass& p, uint32_t max_len) {
 // U + 1 (against 2 * dcap + 5 cells a generation), and holds bounds up to
 // band_cap; pairs with larger bounds go to the deferral chain.  Only bucket
 // passes take it: the chain's passes must hold every pair they get.
-void choose_band_cap(ewfa_ctx* c, Pass& p) {
+void choose_band_cap(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     p.band_cap = 0;
-    if (p.reg || p.gslot || p.bt_lds || p.off16 || p.dcap < BOUND_MIN_DCAP) return;
+    if (unbounded(c, blen, items) || p.reg || p.gslot || p.bt_lds || p.off16 || p.dcap < BOUND_MIN_DCAP) return;
     if (p.seq_words > ewfa::BOUND_MAX_SEQ_WORDS) return;  // no bounds for this pass
     const size_t budget = lds_budget(c);
     const size_t per_cu = budget / ewfa::lds_bytes(p.seq_words, p.dcap, 0, 0);
@@ -327,11 +337,18 @@ constexpr size_t BP_LEAST = (size_t)256 << 20;
 // as its pair's columns (0.4 ms at 5 kbp) whatever the count, which a small
 // call waits for.
 constexpr uint32_t LANE_BOUND_MIN = 8192;
-constexpr uint32_t BP_PROBE_MIN = 4096;
+// A list without bounds of its own is sampled for its way (50 us) when the square
+// of its longest length, as which the wavefront's work grows, comes to this over
+// its pairs (2,500 pairs of 3..7 kbp at 5..15% edits 3,118 -> 2,064 us, 3,000 of
+// 1..4 kbp at 1..10% 661 unsampled and 772 sampled).
+constexpr uint64_t BP_PROBE_MIN = 60000000000ull;
 // Lists below this get twice the lanes per pair: eight pairs a wave would leave
 // SIMDs with less than two waves (15,001 pairs of 3..7 kbp: 4.0 -> 3.5 ms; 500,000
 // pairs of up to 10 kbp 17.5 -> 20.8 ms, so large lists keep the narrow groups).
 constexpr uint32_t BP_SPREAD_BELOW = 32768;
+
+// Pairs per CU up to which a list counts as few.
+constexpr uint32_t FEW_PER_CU = 4;
 
 // The bit-parallel pass ahead of a block bucket pass: it takes the pairs for
 // which it is the cheaper way (bp_class_of).  Not under a distance cap, whose
@@ -341,9 +358,13 @@ void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     p.bp_slot_bytes = 0;
     if (p.reg || p.gslot || p.bt_lds || c->opts.max_distance > 0) return;
     if (p.seq_words > ewfa::BOUND_MAX_SEQ_WORDS) return;
+    // few pairs are faster by levels shared by many waves than by a wave each (60
+    // pairs of 10..30 kbp at 8..12% edits 7,395 -> 4,376 us, 600 of 20..40 kbp at
+    // 1..12% 11,778 -> 8,110)
+    if (items <= FEW_PER_CU * (uint32_t)c->num_cus) return;
     // passes without bounds of their own: lists long enough for the sample that
     // decides on them (bp_probe_kernel)
-    if (p.dcap < BOUND_MIN_DCAP && items < BP_PROBE_MIN) return;
+    if (p.dcap < BOUND_MIN_DCAP && (uint64_t)items * blen * blen < BP_PROBE_MIN) return;
     p.bp_spread = items < BP_SPREAD_BELOW ? 1 : 0;
     const size_t budget = std::min(c->bp_budget, BP_BUDGET);
     if (budget < BP_LEAST) return;
@@ -399,6 +420,11 @@ int pass_from_bucket(ewfa_ctx* c, const ewfa::BucketPolicy& b, uint32_t blen, ui
     p.seq_words = seq_words_for(blen);
     p.persistent = true;
     p.waves = b.waves;
+    // few pairs leave CUs idle, and a call lasts as long as its longest chain of
+    // levels: more waves share a level (100 pairs of 5..10 kbp: 1,480, 1,069, 873
+    // and 787 us with 2, 4, 8 and 16 waves; 60 of 100..2,000 bp 128, 120, 122, 121)
+    if (c->builtin_policy && b.waves > 1 && items <= FEW_PER_CU * (uint32_t)c->num_cus)
+        p.waves = std::max(b.waves, items <= (uint32_t)c->num_cus && blen > 4000 ? 16 : 8);
     p.bt_lds = b.bt_lds;
     p.grab = std::max(1, b.grab);
     p.dcap = b.dcap;
@@ -426,7 +452,7 @@ int pass_from_bucket(ewfa_ctx* c, const ewfa::BucketPolicy& b, uint32_t blen, ui
         }
     }
     choose_off16(p, blen);
-    choose_band_cap(c, p);
+    choose_band_cap(c, p, blen, items);
     choose_bp(c, p, blen, items);
     return finish_pass(c, p, items);
 }
@@ -719,6 +745,7 @@ int enqueue_bound(ewfa_ctx* c, ewfa::AlignArgs& a, const Pass& p, uint32_t* queu
     // (a pass with narrow slots always gets its bounds, as it must read them)
     if (p.reg || p.dcap < BOUND_MIN_DCAP || p.seq_words > ewfa::BOUND_MAX_SEQ_WORDS || (n == 0 && !p.band_cap))
         return EWFA_OK;
+    if (!p.band_cap && unbounded(c, a.max_len, n)) return EWFA_OK;
     ewfa::AlignArgs b = a;
     b.queue = queue;
     b.bound = scratch_of(c).bound;
@@ -783,7 +810,7 @@ int emit_list(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max
 int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, bool staged, hipStream_t s) {
     // few pairs: a wave each, whose walk takes a tenth of a lane's (a lane's
     // steps wait for memory; large lists hide that over many pairs)
-    if (staged && items <= (uint32_t)c->num_cus * 4u) return emit_list(c, e, items, max_len, s);
+    if (staged && items <= (uint32_t)c->num_cus * FEW_PER_CU) return emit_list(c, e, items, max_len, s);
     const int sw = seq_words_for(max_len);
     if (staged && sw <= ewfa::EMIT_LDS_MAX_SW)
         HIPCHK(ewfa::launch_emit_lds(e, items, sw, s));
@@ -965,6 +992,8 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.bins = ctl;
                 x.cursors = ctl + ewfa::BP_BINS;
                 x.seg = ctl + BP_SEG;
+                static_assert(CTRL_BP % 2 == 0 && BP_WEIGH % 2 == 0, "64-bit sums");
+                x.weigh = reinterpret_cast<ewfa::BpWeigh*>(ctl + BP_WEIGH);
                 x.list_out = c->bp_list.as<uint32_t>() + (size_t)b * n;
                 x.list = x.list_out;
                 x.rest = c->bp_rest.as<uint32_t>() + (size_t)b * n;
@@ -972,6 +1001,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.queue = ctl + BP_QUEUE;
                 x.spread = p.bp_spread;
                 x.budget = p.dcap;
+                x.deep = p.dcap >= BOUND_MIN_DCAP;
                 x.defer_list = sx.list_a;
                 x.defer_count = ctrl + CTRL_DEFER_A;
                 x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;
@@ -1519,6 +1549,7 @@ int fetch_compact(ewfa_ctx_t* c, size_t total, hipStream_t s, const int8_t** out
 int set_context_policy(ewfa_ctx_t* c, const Policy& p) {
     if (!c || p.buckets.empty()) return fail(EWFA_ERR_ARG, "empty policy");
     c->policy = p;
+    c->builtin_policy = false;
     c->policy.buckets.back().len_hi = 0xFFFFFFFFu;
     ++c->policy_gen;
     return EWFA_OK;
@@ -1593,6 +1624,7 @@ int ewfa_create(ewfa_ctx_t** out, const ewfa_opts_t* opts) {
         rc = fail(EWFA_ERR_HIP, "could not raise the block kernels' LDS limit to %zu bytes", lds_budget(c));
     if (rc == EWFA_OK) {
         rc = ewfa::load_policy(c->opts.policy_path, c->policy);
+        c->builtin_policy = !c->opts.policy_path || !*c->opts.policy_path;
         if (rc == EWFA_ERR_IO) fail(rc, "could not open the policy file %s", c->opts.policy_path);
         if (rc == EWFA_ERR_FORMAT) fail(rc, "bad policy file %s", c->opts.policy_path);
     }

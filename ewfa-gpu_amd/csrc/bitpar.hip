@@ -780,10 +780,18 @@ __global__ __launch_bounds__(64, PART == BP_WIDE ? 4 : 3) void bp_kernel(BpArgs 
     }
 }
 
-// Wave instructions of a wavefront search of d levels (weights fitted to calls:
-// 500,000 pairs of 100..10,000 bp at 1..10% edits took 25.1, 20.6, 20.1 and 20.7 ms
-// with 0.22, 0.5, 1 and 2 per d * d).
-__device__ __forceinline__ float wavefront_cost(float d) { return 0.6f * d * d + 100.0f * d; }
+// Wave instructions of a wavefront search of d levels: weights fitted to calls, of
+// the two-wave passes (500,000 pairs of 100..10,000 bp at 1..10% edits took 25.1,
+// 20.6, 20.1 and 20.7 ms with 0.22, 0.5, 1 and 2 per d * d) and of the eight-wave
+// passes within distance bounds, whose levels cost much the same until they are
+// wider than the block (10..20 kbp pairs 0.55 us each at 1..3% edits and 1.6 at
+// 5..12%, 10..50 kbp pairs 9.2 at 10..15%).
+__device__ __forceinline__ float wavefront_cost(float d, bool deep) {
+    return d * (deep ? 750.0f + 0.2f * d : 100.0f + 0.6f * d);
+}
+// Microseconds a wave instruction takes of the whole chip (256 CUs at about
+// 2.3 GHz), and a column of a pair from table to path.
+constexpr float BP_INSTR_US = 1.7e-6f, BP_COLUMN_US = 0.105f;
 
 // ---- distance bounds ------------------------------------------------------------
 // An upper bound on each pair's distance from a window of 64 diagonals that
@@ -937,7 +945,7 @@ __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* 
         const uint32_t u = lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl, slope);
         columns = (float)pr.tlen;
         levels = (float)u / (float)tl * columns;
-        wfa = wavefront_cost(levels);
+        wfa = wavefront_cost(levels, false);
         bp = columns * 7.5f + 25.0f * levels;
     }
     for (int d = 32; d; d >>= 1) {
@@ -993,48 +1001,115 @@ hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t
 
 namespace {
 
-// Lists below this leave the chip idle, and a call lasts as long as its longest
-// chain: a pair's levels (about 1.1 us and half a ns a diagonal each, its stream
-// included; twice where the pass's budget of levels defers it) or columns (0.25 us each).
-constexpr uint32_t BP_CHAIN_BELOW = 2048;
+// What a pair costs each way: wave instructions of the chip's work, and the us its
+// own chain takes: its levels (about 1.1 us and half a ns a diagonal each, its
+// stream included; twice where the pass's budget of levels defers it), or its
+// columns.
+struct BpCost {
+    int c;  // class: the narrowest band that holds every path within the bound
+            // (BP_CLASSES: no bound, the pair is the wavefront's)
+    float wave, bits, wave_us, bits_us;
+};
 
-// The class of a pair of a list of n: the narrowest band that holds every path
-// within its distance bound, or BP_CLASSES for the wavefront (no bound, or so few
-// edits that the wavefront is faster).
 // A bound beyond the widest band, or above a fifth of the text, mostly comes of a
 // search whose window lost the path at a long gap: it then says nothing of the
-// distance.  The guess from the part before the gap then says which way is the
-// faster, and a bound beyond the widest band takes that band, where the distance
-// most likely lies (if not the pair is deferred); without a guess such pairs stay
-// with the wavefront.
-__device__ __forceinline__ int bp_class_of(const BpArgs& a, const ewfa_pair_t& pr, uint32_t pidx, uint32_t n) {
+// distance.  The guess from the part before the gap then gives the costs, and a
+// bound beyond the widest band takes that band, where the distance most likely
+// lies (if not the pair is deferred); without a guess such pairs stay with the
+// wavefront.
+__device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx) {
+    BpCost k{BP_CLASSES, 0.f, 0.f, 0.f, 0.f};
+    const ewfa_pair_t pr = a.pairs[pidx];
     uint32_t u = a.bound[pidx];
-    if (u == BOUND_NONE || pr.plen > a.max_len || pr.tlen > a.max_len || pr.tlen == 0u || pr.plen == 0u)
-        return BP_CLASSES;
+    if (u == BOUND_NONE || pr.plen > a.max_len || pr.tlen > a.max_len || pr.tlen == 0u || pr.plen == 0u) return k;
     const int tk = (int)pr.tlen - (int)pr.plen;
     int S, c = BP_CLASSES - 1;
     while (c > 0 && bp_band(bp_words(c), tk, S) < (int)u) --c;
     const int L = bp_band(bp_words(c), tk, S);
     if (L < (int)u || u > pr.tlen / 5u + 64u) {
-        if (!a.guess || L < 0) return BP_CLASSES;
+        if (!a.guess || L < 0) return k;
         u = a.guess[pidx];
     }
     const float d = (float)u, cols = (float)pr.tlen;
-    const bool wave = n < BP_CHAIN_BELOW
-                          ? d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f) < cols * 0.25f
-                          : wavefront_cost(d) < cols * (bp_column_cost(c) + 2.0f) + 25.0f * d;
-    return wave ? BP_CLASSES : c;
+    k.c = c;
+    k.wave = wavefront_cost(d, a.deep);
+    k.bits = cols * (bp_column_cost(c) + 2.0f) + 25.0f * d;
+    k.wave_us = d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f);
+    k.bits_us = cols * BP_COLUMN_US;
+    return k;
+}
+
+// The list's way, from its pairs' costs together: every pair by the wavefront
+// (0), each the way with less work (1), or every pair that has a class by the
+// bit-parallel kernel (2).  A way's time is its work and its longest chain, of
+// which few pairs hide nothing (1,500, 5,000 and 15,000 pairs of 10..20 kbp at
+// 1..3% edits: 1.8, 3.4 and 9.0 ms by the wavefront, 3.0, 3.4 and 6.4
+// bit-parallel); the two ways of one list run one after the other.
+__device__ __forceinline__ int bp_way(const BpWeigh& w) {
+    auto time = [](uint64_t work, uint32_t chain) { return (float)work * BP_INSTR_US + (float)chain; };
+    const float t0 = time(w.wave, w.wave_us);
+    const float t1 = time(w.split_bits, w.split_bits_us) + time(w.split_wave, w.split_wave_us);
+    const float t2 = time(w.bits, w.bits_us);
+    return t0 <= t1 && t0 <= t2 ? 0 : t1 <= t2 ? 1 : 2;
 }
 
 // Bin of a pair in the sort: its class, then its length, longest first.
-__device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, uint32_t n) {
-    const ewfa_pair_t pr = a.pairs[pidx];
-    const int c = a.flag && *a.flag == 0u ? BP_CLASSES : bp_class_of(a, pr, pidx, n);
-    const uint32_t b = min((uint32_t)((uint64_t)pr.tlen * BP_LEN_BINS / (a.max_len + 1u)), (uint32_t)BP_LEN_BINS - 1u);
+__device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, int way) {
+    int c = BP_CLASSES;
+    if (way) {
+        const BpCost k = bp_cost(a, pidx);
+        if (way == 2 || k.bits <= k.wave) c = k.c;
+    }
+    const uint32_t b = min((uint32_t)((uint64_t)a.pairs[pidx].tlen * BP_LEN_BINS / (a.max_len + 1u)), (uint32_t)BP_LEN_BINS - 1u);
     return c * BP_LEN_BINS + (int)(BP_LEN_BINS - 1u - b);
 }
 
+// The way of a list: what the sample said, else its pairs' sums.
+__device__ __forceinline__ int bp_list_way(const BpArgs& a) {
+    return a.flag && *a.flag == 0u ? 0 : bp_way(*a.weigh);
+}
+
+__device__ __forceinline__ float wave_add(float v) {
+    for (int d = 32; d; d >>= 1) v += __shfl_xor(v, d);
+    return v;
+}
+
+__device__ __forceinline__ float wave_most(float v) {
+    for (int d = 32; d; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
+    return v;
+}
+
 }  // namespace
+
+// Adds up the costs of the list's pairs (a.weigh, zero at first).
+__global__ __launch_bounds__(256) void bp_weigh_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
+                                                       uint32_t count) {
+    const uint32_t n = count_ptr ? *count_ptr : count;
+    if (a.flag && *a.flag == 0u) return;
+    float sum[4] = {}, most[4] = {};
+    for (uint32_t at = blockIdx.x * 256u + threadIdx.x; at < n; at += gridDim.x * 256u) {
+        const BpCost k = bp_cost(a, list ? list[at] : at);
+        const bool bits = k.bits <= k.wave;
+        if (k.c == BP_CLASSES) continue;
+        sum[0] += k.wave;
+        sum[1] += k.bits;
+        sum[2] += bits ? 0.f : k.wave;
+        sum[3] += bits ? k.bits : 0.f;
+        most[0] = fmaxf(most[0], k.wave_us);
+        most[1] = fmaxf(most[1], k.bits_us);
+        most[2] = fmaxf(most[2], bits ? 0.f : k.wave_us);
+        most[3] = fmaxf(most[3], bits ? k.bits_us : 0.f);
+    }
+    uint64_t* const sums = &a.weigh->wave;
+    uint32_t* const mosts = &a.weigh->wave_us;
+    for (int i = 0; i < 4; ++i) {
+        const float v = wave_add(sum[i]), m = wave_most(most[i]);
+        if ((threadIdx.x & 63u) == 0u && v > 0.f) {
+            atomicAdd((unsigned long long*)(sums + i), (unsigned long long)v);
+            atomicMax(mosts + i, (uint32_t)m);
+        }
+    }
+}
 
 // Counts the list's pairs per bin.
 __global__ __launch_bounds__(256) void bp_count_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
@@ -1043,12 +1118,13 @@ __global__ __launch_bounds__(256) void bp_count_kernel(BpArgs a, const uint32_t*
     const uint32_t n = count_ptr ? *count_ptr : count;
     const uint32_t base = blockIdx.x * 256u;
     if (base >= n) return;
+    const int way = bp_list_way(a);
     for (int i = threadIdx.x; i < BP_BINS; i += 256) h[i] = 0u;
     __syncthreads();
     const uint32_t at = base + threadIdx.x;
     if (at < n) {
         const uint32_t pidx = list ? list[at] : at;
-        atomicAdd(&h[bp_bin_of(a, pidx, n)], 1u);
+        atomicAdd(&h[bp_bin_of(a, pidx, way)], 1u);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < BP_BINS; i += 256)
@@ -1064,6 +1140,7 @@ __global__ __launch_bounds__(256) void bp_place_kernel(BpArgs a, const uint32_t*
     const uint32_t n = count_ptr ? *count_ptr : count;
     const uint32_t base = blockIdx.x * 256u;
     if (base >= n && blockIdx.x) return;
+    const int way = bp_list_way(a);
     constexpr int FIRST_REST = BP_CLASSES * BP_LEN_BINS;
     for (int i = threadIdx.x; i < BP_BINS; i += 256) h[i] = 0u;
     if (threadIdx.x == 0) {
@@ -1083,7 +1160,7 @@ __global__ __launch_bounds__(256) void bp_place_kernel(BpArgs a, const uint32_t*
     uint32_t pidx = 0, local = 0;
     if (item < n) {
         pidx = list ? list[item] : item;
-        b = bp_bin_of(a, pidx, n);
+        b = bp_bin_of(a, pidx, way);
         local = atomicAdd(&h[b], 1u);
     }
     __syncthreads();
@@ -1097,6 +1174,7 @@ hipError_t launch_bp_sort(const BpArgs& a, const uint32_t* list, const uint32_t*
                           hipStream_t stream) {
     if (count == 0) return hipSuccess;
     const uint32_t blocks = (count + 255u) / 256u;
+    hipLaunchKernelGGL(bp_weigh_kernel, dim3(blocks < 512u ? blocks : 512u), dim3(256), 0, stream, a, list, count_ptr, count);
     hipLaunchKernelGGL(bp_count_kernel, dim3(blocks), dim3(256), 0, stream, a, list, count_ptr, count);
     hipLaunchKernelGGL(bp_place_kernel, dim3(blocks), dim3(256), 0, stream, a, list, count_ptr, count);
     return hipGetLastError();

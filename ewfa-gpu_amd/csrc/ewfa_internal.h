@@ -205,6 +205,13 @@ __host__ __device__ inline int bp_band(int N, int tk, int& S) {
     return L >= (tk < 0 ? -tk : tk) ? L : -1;
 }
 
+// A list's costs each way (bp_cost): all by the wavefront, all bit-parallel,
+// each the way with less work.
+struct BpWeigh {
+    uint64_t wave, bits, split_wave, split_bits;          // wave instructions
+    uint32_t wave_us, bits_us, split_wave_us, split_bits_us;  // longest chains
+};
+
 struct BpArgs {
     const uint64_t* words;
     const ewfa_pair_t* pairs;
@@ -214,6 +221,7 @@ struct BpArgs {
     const uint32_t* bound;    // per pair
     uint32_t* guess;          // per pair, a guess at the distance (null: none)
     const uint32_t* flag;     // 0: the whole list is the wavefront's (null: no)
+    BpWeigh* weigh;           // zero at first
     uint32_t* bins;           // BP_BINS counts and BP_BINS cursors, zero at first
     uint32_t* cursors;
     uint32_t* seg;            // BP_CLASSES + 1 places in list
@@ -224,6 +232,7 @@ struct BpArgs {
     uint32_t* queue;          // work counters of the wide and the narrow classes
     int spread;               // bp_group
     int budget;               // levels of the wavefront pass over the rest
+    bool deep;                // ... an eight-wave one within distance bounds
     uint32_t* defer_list;
     uint32_t* defer_count;
     uint8_t* slots;           // per block: tok_bytes of tokens, then the records

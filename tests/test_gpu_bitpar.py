@@ -1,10 +1,10 @@
 """The bit-parallel pass (bitpar.hip) against the oracle, bit for bit.
 
-A policy whose only bucket has a budget above 2,048 levels sends every pair
-that is cheaper that way through it once a call has 2,048 pairs: here mostly
-short ones, so that the oracle stays quick, around the pairs of the case.  From
-8,192 pairs on the distance bounds come from the lane-per-pair search, and from
-32,768 on the groups of lanes are at their narrowest.
+A policy whose only bucket has a budget above 2,048 levels weighs the pass for
+every call of more than 1,024 pairs: here mostly short ones, so that the oracle
+stays quick, around the pairs of the case.  From 8,192 pairs on the distance
+bounds come from the lane-per-pair search, and from 32,768 on the groups of lanes
+are at their narrowest.
 """
 import numpy as np
 import pytest
@@ -173,3 +173,38 @@ def test_short_lists_over_the_grid(count):
     with ewfa.Context() as ctx:
         ctx.align_device(dw.ptr, dp.ptr, w.n, w.max_len, dr.ptr, dc.ptr)
     check(dr.download(ewfa.RESULT_DTYPE, w.n), w.pairs[:w.n], dc.download(np.int8), d, st, count)
+
+
+@pytest.mark.parametrize("name,count,near,far", [("wavefront", 1500, 3000, 0), ("bit-parallel", 1500, 0, 600),
+                                                 ("both", 16000, 400, 400)])
+def test_a_list_goes_one_way_or_both(tmp_path, name, count, near, far):
+    """Lists of pairs of a few edits (the wavefront's), of many (bit-parallel),
+    and of half and half, enough of them that both ways pay."""
+    print(f"case ways {name}: {count} pairs", flush=True)
+    rng = np.random.default_rng(count + near)
+    pool = []
+    for i in range(200):
+        n = near if near and (not far or i % 2) else far
+        p = rng.choice(BASES, n - int(rng.integers(40))).tobytes()
+        pool.append((p, mutate(rng, p, 0.15 if n == far and not (near and i % 2) else 0.0005)))
+    P, T = [pool[i % 200][0] for i in range(count)], [pool[i % 200][1] for i in range(count)]
+    d, st = oracle_streams([p for p, _ in pool], [t for _, t in pool])
+    d, st = [d[i % 200] for i in range(count)], [st[i % 200] for i in range(count)]
+    words, pairs, cb, ml = ewfa.from_sequences(P, T)
+    with ewfa.Context(policy_path=policy_file(tmp_path, "ways", POLICY)) as ctx:
+        dw, dp = ewfa.DeviceBuffer.from_array(words), ewfa.DeviceBuffer.from_array(pairs)
+        dr, dc = ewfa.DeviceBuffer(count * 16), ewfa.DeviceBuffer(cb)
+        dc.fill_zero()
+        ctx.align_device(dw.ptr, dp.ptr, count, ml, dr.ptr, dc.ptr)
+        check(dr.download(ewfa.RESULT_DTYPE, count), pairs, dc.download(np.int8), d, st, name)
+
+
+@pytest.mark.parametrize("count,lo,hi", [(2, 4100, 9000), (256, 2600, 4100), (257, 1300, 6000), (1025, 1300, 2600)])
+def test_few_pairs_share_levels_over_more_waves(count, lo, hi):
+    """Calls around a pair, and four pairs, per CU: 16, 8 and 2 waves a pair."""
+    print(f"case few {count} pairs {lo}..{hi} bp", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=count, len_lo=lo, len_hi=hi, err_lo=0.02, err_hi=0.1), count)
+    ok, d, sl, st = orc.batch_workload(w)
+    with ewfa.Context() as ctx:
+        res, cig = ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes)
+    check(res, w.pairs, cig, d, st, "few")
