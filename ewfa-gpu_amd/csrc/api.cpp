@@ -108,7 +108,7 @@ struct ewfa_ctx {
     int num_cus = 0;
     size_t lds_max = 0;
     DevBuf ops, bt, ctrl, list_a, list_b, buckets, runs, list_fb, bound, gslot, order;
-    DevBuf bp_list, bp_rest, bp_guess, bp_slots;  // bit-parallel passes
+    DevBuf bp_list, bp_rest, bp_guess;  // bit-parallel passes
     size_t bp_budget = SIZE_MAX;  // bytes of slots a bit-parallel pass may hold (less after a failed allocation)
     uint32_t* host_ctrl = nullptr;  // pinned mirror of the control words
     float align_ms = 0.f, emit_ms = 0.f;
@@ -243,7 +243,7 @@ struct Pass {
     // the bit-parallel pass ahead of a bounded bucket pass (0 blocks: none)
     uint32_t bp_grid, bp_part[3];  // the most, and by part (BP_ALL, ..)
     int bp_spread;
-    size_t bp_slot_bytes, bp_off;
+    size_t bp_slot_bytes;
 };
 
 // Passes whose wavefront LDS cannot hold keep their slots in HBM.  Their
@@ -368,7 +368,7 @@ void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     p.bp_spread = items < BP_SPREAD_BELOW ? 1 : 0;
     const size_t budget = std::min(c->bp_budget, BP_BUDGET);
     if (budget < BP_LEAST) return;
-    p.bp_slot_bytes = ewfa::bp_tok_bytes() + ewfa::bp_rec_bytes(blen);
+    p.bp_slot_bytes = ewfa::bp_slot_bytes(blen);
     const uint64_t room = std::max<size_t>(budget / p.bp_slot_bytes, 1);
     const bool apart = p.dcap >= BOUND_MIN_DCAP;
     for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW}) {
@@ -499,7 +499,7 @@ struct Plan {
     int fanout = 1;
     size_t bt_bytes = 0, runs_bytes = 0;  // regions the plan's slots need
     size_t gslot_bytes = 0;               // HBM slots of the passes beyond LDS
-    size_t bp_bytes = 0;                  // slots of the bit-parallel passes
+    bool bp = false;                      // some pass has a bit-parallel one ahead
 };
 
 // Bytes of one block's slot in the backtrace region (block passes with the
@@ -514,7 +514,9 @@ void assign_slots(Plan& pl) {
         Pass& p = pl.pass[b];
         size_t& at = p.reg ? runs : bt;
         p.slot_off = pl.fanout > 1 ? at : 0;
-        const size_t need = p.slot_off + slot_bytes(p) * p.grid;
+        // (the bit-parallel kernels' slots are there before the pass needs its own)
+        const size_t most = std::max(slot_bytes(p) * p.grid, p.bp_slot_bytes * p.bp_grid);
+        const size_t need = p.slot_off + ((most + 255) & ~(size_t)255);
         if (pl.fanout > 1) at = need;
         else at = std::max(at, need);
     }
@@ -532,13 +534,8 @@ void assign_slots(Plan& pl) {
         bt = std::max(bt, slot_bytes(p) * p.grid);
         if (p.gslot) gs = std::max(gs, p.gslot_bytes * p.grid);
     }
-    size_t bp = 0;
-    for (int b = 0; b < pl.nb; ++b) {
-        Pass& p = pl.pass[b];
-        p.bp_off = pl.fanout > 1 ? bp : 0;
-        bp = std::max(bp, p.bp_off + p.bp_slot_bytes * p.bp_grid);
-    }
-    pl.bp_bytes = bp;
+    pl.bp = false;
+    for (int b = 0; b < pl.nb; ++b) pl.bp = pl.bp || pl.pass[b].bp_grid;
     pl.bt_bytes = bt;
     pl.runs_bytes = runs;
     pl.gslot_bytes = gs;
@@ -699,9 +696,12 @@ int reserve_bt(ewfa_ctx* c, const Pass& p) {
 }
 
 int reserve_plan(ewfa_ctx* c, Plan& pl, size_t n) {
-    // slots for the bit-parallel passes, fewer when the device has no room for
-    // all (every later plan of the context then asks for fewer)
-    while (pl.bp_bytes && c->bp_slots.reserve(c, pl.bp_bytes) != EWFA_OK) {
+    // where the device has no room for all slots, fewer for the bit-parallel
+    // passes (every later plan of the context then asks for fewer)
+    for (;;) {
+        const int rc = c->bt.reserve(c, pl.bt_bytes);
+        if (rc == EWFA_OK) break;
+        if (!pl.bp) return rc;
         (void)hipGetLastError();
         g_err.clear();
         c->bp_budget = std::min(c->bp_budget, BP_BUDGET) / 4;
@@ -710,11 +710,10 @@ int reserve_plan(ewfa_ctx* c, Plan& pl, size_t n) {
         assign_slots(pl);
     }
     CHK(c->runs.reserve(c, pl.runs_bytes));
-    CHK(c->bt.reserve(c, pl.bt_bytes));
     CHK(c->gslot.reserve(c, pl.gslot_bytes));
     if (pl.nb > 1) CHK(c->buckets.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
     CHK(c->bound.reserve(c, std::max<size_t>(n, 1) * 4));
-    if (pl.bp_bytes) {
+    if (pl.bp) {
         CHK(c->bp_list.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
         CHK(c->bp_guess.reserve(c, std::max<size_t>(n, 1) * 4));
         CHK(c->bp_rest.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
@@ -949,7 +948,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
     for (int b = 0; b < pl.nb; ++b) fused = fused || pl.pass[b].reg;
     if (phase & PLAN_ALIGN) {
         HIPCHK(ewfa::launch_fill_u32(ctrl, 0u, CTRL_XQ + (size_t)pl.nb * ewfa::XCDS * ewfa::XQ_STRIDE, s));
-        if (pl.bp_bytes) HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_BP, 0u, (size_t)pl.nb * BP_CTRL, s));
+        if (pl.bp) HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_BP, 0u, (size_t)pl.nb * BP_CTRL, s));
         if (bucketed) HIPCHK(ewfa::launch_bucketize(pairs, n, pl.table, lists, ctrl + CTRL_BCOUNT, s));
         if (timing) HIPCHK(hipEventRecord(c->ev_a0, s));
         if (F > 1) {
@@ -1004,7 +1003,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.deep = p.dcap >= BOUND_MIN_DCAP;
                 x.defer_list = sx.list_a;
                 x.defer_count = ctrl + CTRL_DEFER_A;
-                x.slots = c->bp_slots.as<uint8_t>() + p.bp_off;
+                x.slots = c->bt.as<uint8_t>() + p.slot_off;  // the pass's own, which runs after
                 x.slot_bytes = p.bp_slot_bytes;
                 x.tok_bytes = ewfa::bp_tok_bytes();
                 const bool probe = p.dcap < BOUND_MIN_DCAP;
@@ -1684,7 +1683,7 @@ int ewfa_destroy(ewfa_ctx_t* c) {
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     for (DevBuf* b : {&c->ops, &c->bt, &c->ctrl, &c->list_a, &c->list_b, &c->buckets, &c->runs, &c->list_fb, &c->bound,
-                      &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_guess, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results, &c->h_cigars, &c->dense, &c->scan})
+                      &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_guess, &c->h_words, &c->h_pairs, &c->h_results, &c->h_cigars, &c->dense, &c->scan})
         b->release();
     if (c->host_ctrl) (void)hipHostFree(c->host_ctrl);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
@@ -1771,7 +1770,7 @@ int ewfa_context_memory(ewfa_ctx_t* c, size_t* bytes) {
     if (!c || !bytes) return fail(EWFA_ERR_ARG, "null argument");
     size_t b = 0;
     for (const DevBuf* d : {&c->ops, &c->bt, &c->ctrl, &c->list_a, &c->list_b, &c->buckets, &c->runs,
-                            &c->list_fb, &c->bound, &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_guess, &c->bp_slots, &c->h_words, &c->h_pairs, &c->h_results,
+                            &c->list_fb, &c->bound, &c->gslot, &c->order, &c->bp_list, &c->bp_rest, &c->bp_guess, &c->h_words, &c->h_pairs, &c->h_results,
                             &c->h_cigars, &c->dense, &c->scan})
         b += d->bytes;
     *bytes = b + c->retired_bytes;

@@ -242,10 +242,10 @@ struct BpArgs {
 // Tokens a pair of a group of gl lanes may have: its band's most edits (below
 // 32 * 4 * gl) and room for a flush.
 #define BP_TOK_STRIDE(gl) (128u * (unsigned)(gl) + 64u)
-// Token bytes and record bytes of a slot for texts up to max_len bases: 64 / gl
-// pairs' tokens, and per block of 32 columns up to four words a lane of 16 bytes.
+// A slot for texts up to max_len bases: the tokens of 64 / gl pairs, then the
+// records, per block of 32 columns up to four words a lane of 16 bytes.
 inline size_t bp_tok_bytes() { return 4u * 8u * (size_t)BP_TOK_STRIDE(64) / 4u; }
-inline size_t bp_rec_bytes(uint32_t max_len) { return (size_t)(max_len / 32u + 1u) * 64u * 4u * 16u; }
+inline size_t bp_slot_bytes(uint32_t max_len) { return bp_tok_bytes() + (size_t)(max_len / 32u + 1u) * 64u * 4u * 16u; }
 // *flag = 1 when a sample of the list says the bit-parallel way is the faster
 // (budget: the levels of the wavefront pass).
 hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
