@@ -1442,7 +1442,7 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
     const auto r256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t ops_bytes = op_scratch_bytes(n, max_len);
     const size_t list = r256(n * 4);
-    const size_t fixed = r256(ops_bytes) + r256(CTRL_WORDS * 4) + 4 * list + (pl.nb > 1 ? r256((size_t)pl.nb * n * 4) : 0);
+    const size_t fixed = r256(ops_bytes) + r256(CTRL_BP * 4) + 4 * list + (pl.nb > 1 ? r256((size_t)pl.nb * n * 4) : 0);
     if (fixed > bytes)
         return fail(EWFA_ERR_RANGE, "%zu pairs of up to %u bases need %zu bytes of scratch before any pass; the "
                     "allocation-free call holds %zu", n, max_len, fixed, bytes);
@@ -1451,7 +1451,7 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
     size_t off = 0;
     const auto take = [&](size_t sz) { char* p = b + off; off += r256(sz); return p; };
     x.ops = reinterpret_cast<uint64_t*>(take(ops_bytes));
-    x.ctrl = reinterpret_cast<uint32_t*>(take(CTRL_WORDS * 4));
+    x.ctrl = reinterpret_cast<uint32_t*>(take(CTRL_BP * 4));
     x.list_a = reinterpret_cast<uint32_t*>(take(n * 4));
     x.list_b = reinterpret_cast<uint32_t*>(take(n * 4));
     x.list_fb = reinterpret_cast<uint32_t*>(take(n * 4));
