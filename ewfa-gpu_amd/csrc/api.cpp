@@ -531,7 +531,8 @@ void assign_slots(Plan& pl) {
         Pass& p = pl.chain.pass[k];
         p.slot_off = 0;
         p.gslot_off = 0;
-        bt = std::max(bt, slot_bytes(p) * p.grid);
+        if (p.reg) runs = std::max(runs, slot_bytes(p) * p.grid);
+        else bt = std::max(bt, slot_bytes(p) * p.grid);
         if (p.gslot) gs = std::max(gs, p.gslot_bytes * p.grid);
     }
     pl.bp = false;
@@ -543,9 +544,36 @@ void assign_slots(Plan& pl) {
 
 int next_pass(ewfa_ctx* c, uint32_t max_len, int prev_dcap, uint32_t items, Pass& p);
 
+// Levels of the four-chunk register pass, and the LDS a wave of it may take ahead
+// of the deferral chain (four waves a SIMD).
+constexpr int REG4_LEVELS = 127;
+constexpr size_t REG4_CHAIN_LDS = 10240;
+// The longest pairs of the built-in policy's register passes.
+constexpr uint32_t REG_LEN = 1200;
+
 void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t n, Chain& ch) {
     ch = Chain{};
     int dcap = dcap_min;
+    // what a banded pass defers (63 levels) mostly ends within 127, which a wave
+    // holds in registers: 100,000 pairs of 521 bp at 14.5% edits, all deferred,
+    // took 10,154 us through the block passes below alone, 1,570 so
+    if (dcap < REG4_LEVELS) {
+        const int ow = overlapped_words_for(max_len);
+        if (ewfa::lds_bytes_reg(ow, REG4_LEVELS, 4) <= REG4_CHAIN_LDS) {
+            Pass p{};
+            p.seq_words = ow;
+            p.persistent = true;
+            p.waves = 1;
+            p.bt_lds = 1;
+            p.grab = 4;
+            p.reg = 4;
+            p.dcap = REG4_LEVELS;
+            if (finish_pass(c, p, n) == EWFA_OK) {
+                ch.pass[ch.np++] = p;
+                dcap = p.dcap;
+            }
+        }
+    }
     while (ch.np < MAX_CHAIN) {
         Pass p;
         if (next_pass(c, max_len, dcap, n, p) != EWFA_OK) break;  // no larger budget fits
@@ -573,7 +601,11 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         // over streams (60 pairs of 100..2,000 bp: 175 -> 130 us)
         pl.nb = 1;
         pl.blen[0] = max_len;
-        CHK(pass_from_bucket(c, c->policy.bucket_for(max_len), max_len, n, pl.pass[0]));
+        ewfa::BucketPolicy bp = c->policy.bucket_for(max_len);
+        // nothing to gain from 63 levels alone here, and a second pass to lose
+        // where a pair has more (7 pairs of 135..675 bp at 4..15%: 153 -> 105 us)
+        if (c->builtin_policy && bp.dcap == 63 && max_len > 420) bp.dcap = REG4_LEVELS;
+        CHK(pass_from_bucket(c, bp, max_len, n, pl.pass[0]));
         plan_chain(c, max_len, pl.pass[0].dcap, n, pl.chain);
         assign_slots(pl);
         return EWFA_OK;
@@ -591,7 +623,12 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         if (pl.nb == ewfa::MAX_BUCKETS) break;
         pl.table.hi[pl.nb] = b.len_hi;
         pl.blen[pl.nb] = std::min(b.len_hi, max_len);
-        CHK(pass_from_bucket(c, b, pl.blen[pl.nb], n, pl.pass[pl.nb]));
+        ewfa::BucketPolicy bp = b;
+        // beside block passes, whose longer pairs the call waits for, a second pass
+        // over this bucket's deferred pairs costs more than 63 levels save (16,423
+        // pairs of 566..2,831 bp at 4..11%: 1,065 -> 859 us)
+        if (!capped && c->builtin_policy && b.dcap == 63 && b.len_hi > 420 && max_len > REG_LEN) bp.dcap = REG4_LEVELS;
+        CHK(pass_from_bucket(c, bp, pl.blen[pl.nb], n, pl.pass[pl.nb]));
         ++pl.nb;
         if (max_len <= b.len_hi) break;
     }
@@ -782,6 +819,17 @@ void fill_pass_args(ewfa::AlignArgs& a, const Pass& p, ewfa_ctx* c) {
     a.gslot_words = p.gslot ? p.gslot_bytes / 8 : 0;
 }
 
+// The register kernels write their pairs' streams themselves, all but those left
+// to the fallback emit.
+void reg_args(ewfa::AlignArgs& a, const Pass& p, int8_t* cigars, ewfa_ctx* c) {
+    const ewfa::Scratch sx = scratch_of(c);
+    a.runs = sx.runs + p.slot_off;
+    a.runs_slot = runs_slot_of(p);
+    a.cigars = cigars;
+    a.fallback_list = sx.list_fb;
+    a.fallback_count = sx.ctrl + CTRL_FALLBACK;
+}
+
 // The emit kernel for a pass: sequences staged in LDS when they fit (the
 // persistent path), read from global memory otherwise (and on the plain
 // path, which keeps the reference's one-lane-per-pair global walk).
@@ -888,6 +936,14 @@ int enqueue_chain(ewfa_ctx* c, const Chain& ch, const uint64_t* words, const ewf
         a.queue = ctrl + CTRL_QUEUE;
         a.defer_list = lists[1 - cur];
         a.defer_count = ctrl + ctr[1 - cur];
+        if (p.reg) {
+            HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_XQ, 0u, (size_t)ewfa::XCDS * ewfa::XQ_STRIDE, s));
+            a.xqueue = ctrl + CTRL_XQ;  // (the first bucket's, whose pass has ended)
+            reg_args(a, p, cigars, c);
+            CHK(launch_pass(a, p, s));
+            cur = 1 - cur;
+            continue;
+        }
         CHK(enqueue_bound(c, a, p, ctrl + CTRL_CHAIN_BQ, n, s));
         CHK(launch_pass(a, p, s));
         ewfa::EmitArgs e{};
@@ -971,13 +1027,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
             a.defer_list = sx.list_a;
             a.defer_count = ctrl + CTRL_DEFER_A;
             a.max_len = pl.blen[b];
-            if (p.reg) {  // the register kernel writes its pairs' streams itself
-                a.runs = sx.runs + p.slot_off;
-                a.runs_slot = runs_slot_of(p);
-                a.cigars = cigars;
-                a.fallback_list = sx.list_fb;
-                a.fallback_count = ctrl + CTRL_FALLBACK;
-            }
+            if (p.reg) reg_args(a, p, cigars, c);
             if (p.bp_grid) {
                 // the bit-parallel pass takes its pairs, the rest stay
                 uint32_t* ctl = ctrl + CTRL_BP + (size_t)b * BP_CTRL;
@@ -1060,7 +1110,10 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
         HIPCHK(ewfa::launch_publish_counts(ctrl + CTRL_DEFER_A, ctrl + CTRL_FALLBACK, c->host_ctrl + CTRL_DEFER_A,
                                            c->host_ctrl + CTRL_FALLBACK, s));
     if (!(phase & PLAN_EMIT)) return EWFA_OK;
-    if (fused && fallbacks > 0) {
+    if (deferred > 0)
+        CHK(enqueue_chain(c, pl.chain, words, pairs, std::min(n, deferred), max_len, results, cigars, s));
+    const bool chain_reg = deferred > 0 && pl.chain.np > 0 && pl.chain.pass[0].reg;
+    if ((fused && fallbacks > 0) || chain_reg) {
         // paths with a match run of 255 bases or more go through the emit kernel
         ewfa::EmitArgs e{};
         e.words = words;
@@ -1070,12 +1123,10 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
         e.ops_stride = ewfa::ops_words(max_len + 1);
         e.cigars = cigars;
         e.list = sx.list_fb;
-        e.count = std::min(n, fallbacks);
+        e.count = chain_reg ? n : std::min(n, fallbacks);
         e.count_ptr = ctrl + CTRL_FALLBACK;
         CHK(emit_list(c, e, e.count, max_len, s));
     }
-    if (deferred > 0)
-        CHK(enqueue_chain(c, pl.chain, words, pairs, std::min(n, deferred), max_len, results, cigars, s));
     if (timing) HIPCHK(hipEventRecord(c->ev_e1, s));
     return EWFA_OK;
 }

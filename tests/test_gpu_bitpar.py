@@ -208,3 +208,16 @@ def test_few_pairs_share_levels_over_more_waves(count, lo, hi):
     with ewfa.Context() as ctx:
         res, cig = ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes)
     check(res, w.pairs, cig, d, st, "few")
+
+
+@pytest.mark.parametrize("count,lo,hi,err", [(257, 640, 700, 0.15), (9000, 420, 440, 0.17), (700, 600, 700, 0.30)])
+def test_deferred_banded_pairs_end_in_four_chunks(count, lo, hi, err):
+    """Around 63 and 127 edits: what the banded pass defers, a wave's worth and
+    more at a time, and what the register pass after it defers again."""
+    print(f"case deferred {count} pairs {lo}..{hi} bp {err}", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=count, len_lo=lo, len_hi=hi, err_lo=err / 3, err_hi=err), count)
+    ok, d, sl, st = orc.batch_workload(w)
+    assert max(d) > 63
+    with ewfa.Context() as ctx:
+        res, cig = ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes)
+    check(res, w.pairs, cig, d, st, "deferred")
