@@ -337,7 +337,7 @@ constexpr size_t BP_LEAST = (size_t)256 << 20;
 // as its pair's columns (0.4 ms at 5 kbp) whatever the count, which a small
 // call waits for.
 constexpr uint32_t LANE_BOUND_MIN = 8192;
-// A list without bounds of its own is sampled for its way (50 us) when the square
+// A list without bounds of its own is sampled for its way (25 us) when the square
 // of its longest length, as which the wavefront's work grows, comes to this over
 // its pairs (2,500 pairs of 3..7 kbp at 5..15% edits 3,118 -> 2,064 us, 3,000 of
 // 1..4 kbp at 1..10% 661 unsampled and 772 sampled).
@@ -848,16 +848,18 @@ uint32_t emit_per_wave(const ewfa_ctx* c, uint32_t items) {
 int emit_list(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, hipStream_t s) {
     const int ow = overlapped_words_for(max_len);
     if ((size_t)2 * ow * 8 <= ewfa::EMIT_WAVE_MAX_LDS)
-        HIPCHK(ewfa::launch_emit_wave(e, items, ow, (uint32_t)c->num_cus * 8u, s));
+        HIPCHK(ewfa::launch_emit_wave(e, items, ow, (uint32_t)c->num_cus * 32u, s));
     else
         HIPCHK(ewfa::launch_emit(e, items, emit_per_wave(c, items), s));
     return EWFA_OK;
 }
 
 int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, bool staged, hipStream_t s) {
-    // few pairs: a wave each, whose walk takes a tenth of a lane's (a lane's
-    // steps wait for memory; large lists hide that over many pairs)
-    if (staged && items <= (uint32_t)c->num_cus * FEW_PER_CU) return emit_list(c, e, items, max_len, s);
+    // a wave a pair while its lists are short: a lane's steps wait for memory,
+    // which takes many more pairs to hide (3,000 pairs of 1..10 kbp at 1..5% edits
+    // 1,098 -> 815 us, 30,000 of 8 kbp at 1.1% 1,630 -> 1,480; but 86,000 of 2.3 kbp
+    // at 2.1% 1,498 by lanes and 1,776 by waves)
+    if (staged && items <= (uint32_t)c->num_cus * 128u) return emit_list(c, e, items, max_len, s);
     const int sw = seq_words_for(max_len);
     if (staged && sw <= ewfa::EMIT_LDS_MAX_SW)
         HIPCHK(ewfa::launch_emit_lds(e, items, sw, s));

@@ -928,8 +928,8 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
 // pair's columns of about 0.35 us (bounds, table and path).  (Short lists of moderate lengths go faster
 // through the wavefront: jobs of 100..5,000 bp at 1..10% edits in batches of
 // 25,000 pairs 5.6 against 7.4 ms, while 15,001 pairs of 3..7 kbp at 8..15%
-// take 3.3 against 5.9.)  The sample takes about 50 us.
-constexpr int PROBE_BASES = 512;
+// take 3.3 against 5.9.)  The sample takes about 25 us.
+constexpr int PROBE_BASES = 256;
 
 __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
                                                       uint32_t count, int budget, uint32_t* flag) {
@@ -1141,18 +1141,35 @@ __global__ __launch_bounds__(256) void bp_place_kernel(BpArgs a, const uint32_t*
     const uint32_t base = blockIdx.x * 256u;
     if (base >= n && blockIdx.x) return;
     const int way = bp_list_way(a);
-    constexpr int FIRST_REST = BP_CLASSES * BP_LEN_BINS;
+    constexpr int FIRST_REST = BP_CLASSES * BP_LEN_BINS, BINS = 8;
     for (int i = threadIdx.x; i < BP_BINS; i += 256) h[i] = 0u;
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int i = 0; i < BP_BINS; ++i) {
-            if (i == FIRST_REST) run = 0;
-            at[i] = run;
-            if (blockIdx.x == 0 && i < FIRST_REST && i % BP_LEN_BINS == 0) a.seg[i / BP_LEN_BINS] = run;
-            run += a.bins[i];
-            if (blockIdx.x == 0 && i == FIRST_REST - 1) a.seg[BP_CLASSES] = run;
+    if (threadIdx.x < 64) {
+        // running sums of the classes' bins, and of the rest's, BINS bins a lane
+        constexpr int LANES = FIRST_REST / BINS, REST = BP_BINS - FIRST_REST;
+        static_assert(FIRST_REST % BINS == 0 && LANES + (REST + BINS - 1) / BINS <= 64, "a wave holds the bins");
+        const int lane = threadIdx.x;
+        const int from = lane * BINS;
+        uint32_t c[BINS], sum = 0;
+#pragma unroll
+        for (int i = 0; i < BINS; ++i) {
+            c[i] = from + i < BP_BINS ? a.bins[from + i] : 0u;
+            sum += c[i];
         }
-        if (blockIdx.x == 0) *a.rest_count = run;
+        const uint32_t upto = (uint32_t)wave_incl_scan_i32((int)sum);
+        const uint32_t classes = (uint32_t)__builtin_amdgcn_readlane((int)upto, LANES - 1);
+        const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+        uint32_t run = upto - sum - (lane >= LANES ? classes : 0u);
+#pragma unroll
+        for (int i = 0; i < BINS; ++i) {
+            const int bin = from + i;
+            if (bin < BP_BINS) at[bin] = run;
+            if (blockIdx.x == 0 && bin < FIRST_REST && bin % BP_LEN_BINS == 0) a.seg[bin / BP_LEN_BINS] = run;
+            run += c[i];
+        }
+        if (blockIdx.x == 0 && lane == 0) {
+            a.seg[BP_CLASSES] = classes;
+            *a.rest_count = all - classes;
+        }
     }
     __syncthreads();
     const uint32_t item = base + threadIdx.x;
