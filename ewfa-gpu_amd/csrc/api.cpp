@@ -854,12 +854,17 @@ int emit_list(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max
     return EWFA_OK;
 }
 
-int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, bool staged, hipStream_t s) {
+int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, bool staged, hipStream_t s,
+         bool deeper = false) {
     // a wave a pair while its lists are short: a lane's steps wait for memory,
     // which takes many more pairs to hide (3,000 pairs of 1..10 kbp at 1..5% edits
     // 1,098 -> 815 us, 30,000 of 8 kbp at 1.1% 1,630 -> 1,480; but 86,000 of 2.3 kbp
-    // at 2.1% 1,498 by lanes and 1,776 by waves)
-    if (staged && items <= (uint32_t)c->num_cus * 128u) return emit_list(c, e, items, max_len, s);
+    // at 2.1% 1,498 by lanes and 1,776 by waves; where both sequences take more than
+    // 12 KB of LDS, few waves: 1,500 pairs of 10..20 kbp 1,926 -> 1,628, none of it
+    // left at 3,000).  Beside a bucket whose narrow slots just fill the LDS (deeper),
+    // its blocks would keep one of those off every CU.
+    const uint32_t per_cu = deeper ? FEW_PER_CU : (size_t)2 * overlapped_words_for(max_len) * 8 <= 12288 ? 128u : 8u;
+    if (staged && items <= (uint32_t)c->num_cus * per_cu) return emit_list(c, e, items, max_len, s);
     const int sw = seq_words_for(max_len);
     if (staged && sw <= ewfa::EMIT_LDS_MAX_SW)
         HIPCHK(ewfa::launch_emit_lds(e, items, sw, s));
@@ -1063,12 +1068,17 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                     HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, p.dcap, ctl + BP_FLAG, q));
                     x.flag = ctl + BP_FLAG;
                 }
+                // a part of a long call may be a short list: both searches are
+                // launched, and the list's count picks one (20,000 pairs of
+                // 200..20,000 bp at 1..4% edits 5,151 -> 3,964 us; at half the
+                // calls' limit, since lanes give guesses for lost paths too:
+                // 20,000 of 10..50 kbp, 7,500 of them up to 25 kbp, 51.8 -> 44.2 ms)
+                x.lane_min = probe ? 0u : LANE_BOUND_MIN / 2u;
+                a.below = n < LANE_BOUND_MIN ? 0u : LANE_BOUND_MIN / 2u;
+                if (!probe) CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
                 if (probe || n >= LANE_BOUND_MIN) {
                     x.guess = c->bp_guess.as<uint32_t>();
                     HIPCHK(ewfa::launch_bp_bound(x, sx.bound, a.list, a.count_ptr, n, (uint32_t)c->num_cus * 16u, q));
-                    a.bound = probe ? nullptr : sx.bound;
-                } else {
-                    CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
                 }
                 HIPCHK(ewfa::launch_bp_sort(x, a.list, a.count_ptr, n, q));
                 for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW})
@@ -1099,7 +1109,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 e.list = emit_items;
                 e.count = n;
                 e.count_ptr = a.count_ptr;
-                CHK(emit(c, e, n, pl.blen[b], true, q));
+                CHK(emit(c, e, n, pl.blen[b], true, q, b < pl.nb - 1 && pl.pass[pl.nb - 1].band_cap > 0));
             }
         }
         for (int i = 1; i < F; ++i) {

@@ -961,11 +961,12 @@ __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* 
 }
 
 __global__ __launch_bounds__(64, 4) void bp_bound_kernel(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
-                                                         uint32_t* bound, uint32_t* guess, const uint32_t* list,
+                                                         uint32_t* bound, uint32_t* guess, uint32_t least, const uint32_t* list,
                                                          const uint32_t* count_ptr, uint32_t count,
                                                          const uint32_t* flag) {
     if (flag && *flag == 0u) return;
     const uint32_t n = count_ptr ? *count_ptr : count;
+    if (n < least) return;
     for (uint32_t item = blockIdx.x * 64u + threadIdx.x; item < n; item += gridDim.x * 64u) {
         const uint32_t pidx = list ? list[item] : item;
         const ewfa_pair_t pr = pairs[pidx];
@@ -987,7 +988,7 @@ hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* lis
     if (count == 0) return hipSuccess;
     const uint32_t blocks = (count + 63u) / 64u;
     hipLaunchKernelGGL(bp_bound_kernel, dim3(blocks < max_grid ? blocks : max_grid), dim3(64), 0, stream, a.words,
-                       a.pairs, a.max_len, bound, a.guess, list, count_ptr, count, a.flag);
+                       a.pairs, a.max_len, bound, a.guess, a.lane_min, list, count_ptr, count, a.flag);
     return hipGetLastError();
 }
 
@@ -1017,7 +1018,7 @@ struct BpCost {
 // bound beyond the widest band takes that band, where the distance most likely
 // lies (if not the pair is deferred); without a guess such pairs stay with the
 // wavefront.
-__device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx) {
+__device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32_t n) {
     BpCost k{BP_CLASSES, 0.f, 0.f, 0.f, 0.f};
     const ewfa_pair_t pr = a.pairs[pidx];
     uint32_t u = a.bound[pidx];
@@ -1027,7 +1028,7 @@ __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx) {
     while (c > 0 && bp_band(bp_words(c), tk, S) < (int)u) --c;
     const int L = bp_band(bp_words(c), tk, S);
     if (L < (int)u || u > pr.tlen / 5u + 64u) {
-        if (!a.guess || L < 0) return k;
+        if (!a.guess || n < a.lane_min || L < 0) return k;
         u = a.guess[pidx];
     }
     const float d = (float)u, cols = (float)pr.tlen;
@@ -1054,10 +1055,10 @@ __device__ __forceinline__ int bp_way(const BpWeigh& w) {
 }
 
 // Bin of a pair in the sort: its class, then its length, longest first.
-__device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, int way) {
+__device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, int way, uint32_t n) {
     int c = BP_CLASSES;
     if (way) {
-        const BpCost k = bp_cost(a, pidx);
+        const BpCost k = bp_cost(a, pidx, n);
         if (way == 2 || k.bits <= k.wave) c = k.c;
     }
     const uint32_t b = min((uint32_t)((uint64_t)a.pairs[pidx].tlen * BP_LEN_BINS / (a.max_len + 1u)), (uint32_t)BP_LEN_BINS - 1u);
@@ -1088,7 +1089,7 @@ __global__ __launch_bounds__(256) void bp_weigh_kernel(BpArgs a, const uint32_t*
     if (a.flag && *a.flag == 0u) return;
     float sum[4] = {}, most[4] = {};
     for (uint32_t at = blockIdx.x * 256u + threadIdx.x; at < n; at += gridDim.x * 256u) {
-        const BpCost k = bp_cost(a, list ? list[at] : at);
+        const BpCost k = bp_cost(a, list ? list[at] : at, n);
         const bool bits = k.bits <= k.wave;
         if (k.c == BP_CLASSES) continue;
         sum[0] += k.wave;
@@ -1124,7 +1125,7 @@ __global__ __launch_bounds__(256) void bp_count_kernel(BpArgs a, const uint32_t*
     const uint32_t at = base + threadIdx.x;
     if (at < n) {
         const uint32_t pidx = list ? list[at] : at;
-        atomicAdd(&h[bp_bin_of(a, pidx, way)], 1u);
+        atomicAdd(&h[bp_bin_of(a, pidx, way, n)], 1u);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < BP_BINS; i += 256)
@@ -1177,7 +1178,7 @@ __global__ __launch_bounds__(256) void bp_place_kernel(BpArgs a, const uint32_t*
     uint32_t pidx = 0, local = 0;
     if (item < n) {
         pidx = list ? list[item] : item;
-        b = bp_bin_of(a, pidx, way);
+        b = bp_bin_of(a, pidx, way, n);
         local = atomicAdd(&h[b], 1u);
     }
     __syncthreads();

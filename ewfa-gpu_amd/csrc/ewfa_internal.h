@@ -103,6 +103,7 @@ struct AlignArgs {
     // 64-bit addresses.
     uint64_t* gslot;
     uint64_t gslot_words;
+    uint32_t below;  // bound search: lists of this many pairs or more have another (0: none have)
 };
 
 constexpr uint32_t BOUND_NONE = 0xFFFFFFFFu;
@@ -220,6 +221,7 @@ struct BpArgs {
     uint32_t max_len;
     const uint32_t* bound;    // per pair
     uint32_t* guess;          // per pair, a guess at the distance (null: none)
+    uint32_t lane_min;        // lists below it have their bounds a wave each, without guesses
     const uint32_t* flag;     // 0: the whole list is the wavefront's (null: no)
     BpWeigh* weigh;           // zero at first
     uint32_t* bins;           // BP_BINS counts and BP_BINS cursors, zero at first

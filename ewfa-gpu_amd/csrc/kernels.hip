@@ -1547,7 +1547,7 @@ __device__ __forceinline__ uint32_t band_bound(const AlignArgs& a, uint32_t pidx
 __global__ __launch_bounds__(64) void bound_kernel(AlignArgs a) {
     const int lane = threadIdx.x;
     const uint32_t count = a.count_ptr ? *a.count_ptr : a.count;
-    if (count == 0) return;  // as in align_reg_kernel
+    if (count == 0 || (a.below && count >= a.below)) return;  // as in align_reg_kernel
     for (;;) {
         const uint32_t item = wave_take(a.queue, 1u, lane);
         if (item >= count) break;
