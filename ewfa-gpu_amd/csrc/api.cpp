@@ -415,7 +415,8 @@ int finish_pass(ewfa_ctx* c, Pass& p, uint32_t items) {
 }
 
 // Pass for pairs up to blen bases under one bucket's policy.
-int pass_from_bucket(ewfa_ctx* c, const ewfa::BucketPolicy& b, uint32_t blen, uint32_t items, Pass& p) {
+int pass_from_bucket(ewfa_ctx* c, const ewfa::BucketPolicy& b, uint32_t blen, uint32_t items, Pass& p,
+                     bool bounds = true) {
     p = Pass{};
     p.seq_words = seq_words_for(blen);
     p.persistent = true;
@@ -452,7 +453,7 @@ int pass_from_bucket(ewfa_ctx* c, const ewfa::BucketPolicy& b, uint32_t blen, ui
         }
     }
     choose_off16(p, blen);
-    choose_band_cap(c, p, blen, items);
+    if (bounds) choose_band_cap(c, p, blen, items);
     choose_bp(c, p, blen, items);
     return finish_pass(c, p, items);
 }
@@ -492,6 +493,7 @@ struct Plan {
     int nb = 0;
     ewfa::BucketTable table{};
     Pass pass[ewfa::MAX_BUCKETS];
+    Pass free_pass[ewfa::MAX_BUCKETS];  // the same without bounds, for few pairs (grid 0: none)
     uint32_t blen[ewfa::MAX_BUCKETS];
     Chain chain;
     // streams the bucket passes are spread over (1: one after another); with
@@ -515,7 +517,9 @@ void assign_slots(Plan& pl) {
         size_t& at = p.reg ? runs : bt;
         p.slot_off = pl.fanout > 1 ? at : 0;
         // (the bit-parallel kernels' slots are there before the pass needs its own)
-        const size_t most = std::max(slot_bytes(p) * p.grid, p.bp_slot_bytes * p.bp_grid);
+        Pass& f = pl.free_pass[b];
+        f.slot_off = p.slot_off;
+        const size_t most = std::max({slot_bytes(p) * p.grid, p.bp_slot_bytes * p.bp_grid, f.grid ? slot_bytes(f) * f.grid : 0});
         const size_t need = p.slot_off + ((most + 255) & ~(size_t)255);
         if (pl.fanout > 1) at = need;
         else at = std::max(at, need);
@@ -629,6 +633,11 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         // pairs of 566..2,831 bp at 4..11%: 1,065 -> 859 us)
         if (!capped && c->builtin_policy && b.dcap == 63 && b.len_hi > 420 && max_len > REG_LEN) bp.dcap = REG4_LEVELS;
         CHK(pass_from_bucket(c, bp, pl.blen[pl.nb], n, pl.pass[pl.nb]));
+        // up to two pairs per CU (400 pairs of 10..20 kbp at 0.2..2% edits 682 -> 546
+        // us; at 1,000 of 1..2% nothing is left of it, 890 and 946)
+        if (n <= 2u * (uint32_t)c->num_cus && pl.pass[pl.nb].band_cap > 0 && pl.blen[pl.nb] <= 40000u &&
+            c->opts.max_distance == 0)
+            CHK(pass_from_bucket(c, bp, pl.blen[pl.nb], n, pl.free_pass[pl.nb], false));
         ++pl.nb;
         if (max_len <= b.len_hi) break;
     }
@@ -1035,6 +1044,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
             a.defer_count = ctrl + CTRL_DEFER_A;
             a.max_len = pl.blen[b];
             if (p.reg) reg_args(a, p, cigars, c);
+            const uint32_t* emit_count = nullptr;
             if (p.bp_grid) {
                 // the bit-parallel pass takes its pairs, the rest stay
                 uint32_t* ctl = ctrl + CTRL_BP + (size_t)b * BP_CTRL;
@@ -1085,10 +1095,22 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                     HIPCHK(ewfa::launch_bp(x, part, p.bp_part[part], q));
                 a.list = x.rest;
                 a.count_ptr = x.rest_count;
+            } else if (pl.free_pass[b].grid) {
+                // a sample sends the list to one of the two passes
+                uint32_t* counts = ctrl + CTRL_BP + (size_t)b * BP_CTRL + BP_QUEUE;
+                HIPCHK(ewfa::launch_few_probe(words, pairs, pl.blen[b], a.list, a.count_ptr, n, counts, q));
+                ewfa::AlignArgs f = a;
+                fill_pass_args(f, pl.free_pass[b], c);
+                f.count_ptr = counts;
+                CHK(launch_pass(f, pl.free_pass[b], q));
+                emit_count = a.count_ptr;
+                a.count_ptr = counts + 1;
+                CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
             } else {
                 CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
             }
             const uint32_t* const emit_items = a.list;
+            if (!pl.free_pass[b].grid) emit_count = a.count_ptr;
             if (p.band_cap > 0 && a.bound && sx.order) {
                 // the pass takes its pairs by decreasing bound, share by share
                 uint32_t* ord = sx.order + (size_t)b * n;
@@ -1108,7 +1130,7 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 e.cigars = cigars;
                 e.list = emit_items;
                 e.count = n;
-                e.count_ptr = a.count_ptr;
+                e.count_ptr = emit_count;
                 CHK(emit(c, e, n, pl.blen[b], true, q, b < pl.nb - 1 && pl.pass[pl.nb - 1].band_cap > 0));
             }
         }
@@ -1499,7 +1521,7 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
             break;
         }
     pl.fanout = 1;
-    for (int b = 0; b < pl.nb; ++b) pl.pass[b].bp_grid = 0;  // nor for bit-parallel slots
+    for (int b = 0; b < pl.nb; ++b) pl.pass[b].bp_grid = pl.free_pass[b].grid = 0;  // nor for bit-parallel slots
     assign_slots(pl);
     // per-pair buffers first, then one region for the passes' slots
     const auto r256 = [](size_t x) { return (x + 255) & ~(size_t)255; };

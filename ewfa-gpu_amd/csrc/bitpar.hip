@@ -793,6 +793,17 @@ __device__ __forceinline__ float wavefront_cost(float d, bool deep) {
 // 2.3 GHz), and a column of a pair from table to path.
 constexpr float BP_INSTR_US = 1.7e-6f, BP_COLUMN_US = 0.105f;
 
+// Sum and maximum over the wave, in every lane.
+__device__ __forceinline__ float wave_add(float v) {
+    for (int d = 32; d; d >>= 1) v += __shfl_xor(v, d);
+    return v;
+}
+
+__device__ __forceinline__ float wave_most(float v) {
+    for (int d = 32; d; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
+    return v;
+}
+
 // ---- distance bounds ------------------------------------------------------------
 // An upper bound on each pair's distance from a window of 64 diagonals that
 // follows the path: the same table, one pair per lane, the window's vertical
@@ -930,6 +941,7 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
 // 25,000 pairs 5.6 against 7.4 ms, while 15,001 pairs of 3..7 kbp at 8..15%
 // take 3.3 against 5.9.)  The sample takes about 25 us.
 constexpr int PROBE_BASES = 256;
+constexpr float FEW_LEVELS = 512.0f;
 
 __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
                                                       uint32_t count, int budget, uint32_t* flag) {
@@ -958,6 +970,36 @@ __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* 
     const float us = (float)n / 64.0f / 590000.0f;
     const float chain = levels * (1.1f + 0.0005f * levels) * (levels > (float)budget ? 2.0f : 1.0f);
     if (threadIdx.x == 0) *flag = fmaxf(bp * us, columns * 0.35f) < fmaxf(wfa * us, chain) ? 1u : 0u;
+}
+
+// Splits a list of few long pairs between two passes, by the same sample: all of
+// it goes to the one without distance bounds (counts[0]) while the longest pair has
+// about as many levels as its block has lanes, which the bound search doubles (a
+// level costs no less for fewer diagonals), else to the one within them
+// (counts[1]).  512 pairs of 10..25 kbp at 0.5..2% edits take 736 us without and 875
+// with bounds, at 5..8% 3,498 and 2,955.
+__global__ __launch_bounds__(64) void few_probe_kernel(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
+                                                       const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
+                                                       uint32_t* counts) {
+    const uint32_t n = count_ptr ? *count_ptr : count;
+    bool near = true;
+    if (n) {
+        const uint32_t item = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) / 128u);
+        const ewfa_pair_t pr = pairs[list ? list[item] : item];
+        float edits = 0.f, bases = 0.f, columns = 0.f;
+        if (pr.plen <= max_len && pr.tlen <= max_len && pr.tlen > 0u) {
+            const int tl = min((int)pr.tlen, PROBE_BASES), pl = min((int)pr.plen, PROBE_BASES);
+            int slope = 0;
+            edits = (float)lane_bound(words + pr.pattern_off, words + pr.text_off, pl, tl, slope);
+            bases = (float)tl;
+            columns = (float)pr.tlen;
+        }
+        near = wave_add(edits) * wave_most(columns) < FEW_LEVELS * wave_add(bases);
+    }
+    if (threadIdx.x == 0) {
+        counts[0] = near ? n : 0u;
+        counts[1] = near ? 0u : n;
+    }
 }
 
 __global__ __launch_bounds__(64, 4) void bp_bound_kernel(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
@@ -989,6 +1031,13 @@ hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* lis
     const uint32_t blocks = (count + 63u) / 64u;
     hipLaunchKernelGGL(bp_bound_kernel, dim3(blocks < max_grid ? blocks : max_grid), dim3(64), 0, stream, a.words,
                        a.pairs, a.max_len, bound, a.guess, a.lane_min, list, count_ptr, count, a.flag);
+    return hipGetLastError();
+}
+
+hipError_t launch_few_probe(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len, const uint32_t* list,
+                            const uint32_t* count_ptr, uint32_t count, uint32_t* counts, hipStream_t stream) {
+    hipLaunchKernelGGL(few_probe_kernel, dim3(1), dim3(64), 0, stream, words, pairs, max_len, list, count_ptr, count,
+                       counts);
     return hipGetLastError();
 }
 
@@ -1068,16 +1117,6 @@ __device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, int way
 // The way of a list: what the sample said, else its pairs' sums.
 __device__ __forceinline__ int bp_list_way(const BpArgs& a) {
     return a.flag && *a.flag == 0u ? 0 : bp_way(*a.weigh);
-}
-
-__device__ __forceinline__ float wave_add(float v) {
-    for (int d = 32; d; d >>= 1) v += __shfl_xor(v, d);
-    return v;
-}
-
-__device__ __forceinline__ float wave_most(float v) {
-    for (int d = 32; d; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
-    return v;
 }
 
 }  // namespace

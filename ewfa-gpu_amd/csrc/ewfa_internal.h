@@ -252,6 +252,10 @@ inline size_t bp_slot_bytes(uint32_t max_len) { return bp_tok_bytes() + (size_t)
 // (budget: the levels of the wavefront pass).
 hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
                            int budget, uint32_t* flag, hipStream_t stream);
+// counts[0], counts[1]: the list's count for the pass without and the one within
+// distance bounds, one of them 0.
+hipError_t launch_few_probe(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len, const uint32_t* list,
+                            const uint32_t* count_ptr, uint32_t count, uint32_t* counts, hipStream_t stream);
 // Upper bounds on the distances of a list's pairs, a lane each.
 hipError_t launch_bp_bound(const BpArgs& a, uint32_t* bound, const uint32_t* list, const uint32_t* count_ptr,
                            uint32_t count, uint32_t max_grid, hipStream_t stream);

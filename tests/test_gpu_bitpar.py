@@ -221,3 +221,15 @@ def test_deferred_banded_pairs_end_in_four_chunks(count, lo, hi, err):
     with ewfa.Context() as ctx:
         res, cig = ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes)
     check(res, w.pairs, cig, d, st, "deferred")
+
+
+@pytest.mark.parametrize("lo,hi,err", [(200, 16000, 0.01), (200, 16000, 0.08)])
+def test_few_long_pairs_with_and_without_bounds(lo, hi, err):
+    """Between one and four pairs per CU, of few edits and of many."""
+    print(f"case few long {lo}..{hi} bp {err}", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=7, len_lo=lo, len_hi=hi, err_lo=err / 2, err_hi=err), 300)
+    ok, d, sl, st = orc.batch_workload(w)
+    with ewfa.Context() as ctx:
+        for _ in range(3):  # eager, recorded, replayed
+            res, cig = ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes)
+            check(res, w.pairs, cig, d, st, "few long")
