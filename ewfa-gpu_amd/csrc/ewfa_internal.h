@@ -326,7 +326,7 @@ hipError_t launch_pack(const char* ascii, size_t ascii_stride, const uint32_t* l
                        uint64_t* words, size_t words_stride, hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t stream);
 // Copies the two counts to (mapped) host memory.
-hipError_t launch_publish_counts(const uint32_t* defer, const uint32_t* fallback, uint32_t* host_defer,
+hipError_t launch_publish_counts(uint32_t* ctrl, int defer, int fallback, uint32_t words, uint32_t* host_defer,
                                  uint32_t* host_fallback, hipStream_t stream);
 // zeroes p[i] for every bit i (< 64) set in mask
 hipError_t launch_clear_words(uint32_t* p, uint64_t mask, hipStream_t stream);

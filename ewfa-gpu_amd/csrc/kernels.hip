@@ -173,14 +173,6 @@ __device__ __forceinline__ int slot_bt_word(int seq_words, int dcap) {
     return 2 * seq_words + ((2 * dcap + 5 + 1) & ~1);
 }
 
-// End of a pair's search: status, deferral, and the traceback into the ops
-// scratch.  Called by every thread of the group with the same arguments; the
-// traceback runs on the group's first wave.  For each run of 64 levels, lane
-// j loads the backtrace chunks level top-j can need: the path diagonal moves
-// by at most one per level, so there it lies within j of the diagonal at level
-// top, i.e. in at most three consecutive 64-diagonal chunks.  The walk then
-// takes each op bit out of lane j with readlane (scalar work), from LDS or
-// HBM alike.
 // Maximum of x over the 64 lanes (every lane takes part; x >= -1), by the
 // same DPP steps, read from lane 63.
 __device__ __forceinline__ int wave_max_i32(int x) {
@@ -362,6 +354,14 @@ __device__ __forceinline__ void fused_emit(const AlignArgs& a, uint32_t pidx, co
     }
 }
 
+// End of a pair's search: status, deferral, and the traceback into the ops
+// scratch.  Called by every thread of the group with the same arguments; the
+// traceback runs on the group's first wave.  For each run of 64 levels, lane
+// j loads the backtrace chunks level top-j can need: the path diagonal moves
+// by at most one per level, so there it lies within j of the diagonal at level
+// top, i.e. in at most three consecutive 64-diagonal chunks.  The walk then
+// takes each op bit out of lane j with readlane (scalar work), from LDS or
+// HBM alike.
 template <bool FUSED>
 __device__ __forceinline__ void finish_pair(const AlignArgs& a, uint32_t pidx, const uint64_t* BT, int gtid,
                                             bool done, int d, int limit, int tk, const ewfa_pair_t* prp = nullptr,
@@ -2160,12 +2160,17 @@ __global__ __launch_bounds__(64) void clear_words_kernel(uint32_t* p, uint64_t m
 
 // The deferred and fallback counts of a plan's bucket passes into host
 // memory, for the call to see whether anything is left to enqueue.
-__global__ __launch_bounds__(64) void publish_counts_kernel(const uint32_t* defer, const uint32_t* fallback,
+// With neither, nothing more runs over the control words: the `words` first of
+// them are then set back to 0 for the next call, which saves it a launch.
+__global__ __launch_bounds__(64) void publish_counts_kernel(uint32_t* ctrl, int defer, int fallback, uint32_t words,
                                                             uint32_t* host_defer, uint32_t* host_fallback) {
+    const uint32_t d = ctrl[defer], f = ctrl[fallback];
     if (threadIdx.x == 0) {
-        *host_defer = *defer;
-        *host_fallback = *fallback;
+        *host_defer = d;
+        *host_fallback = f;
     }
+    if (d | f) return;
+    for (uint32_t i = threadIdx.x; i < words; i += 64u) ctrl[i] = 0u;
 }
 
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, uint32_t value, size_t n) {
@@ -2406,9 +2411,9 @@ hipError_t launch_clear_words(uint32_t* p, uint64_t mask, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_publish_counts(const uint32_t* defer, const uint32_t* fallback, uint32_t* host_defer,
+hipError_t launch_publish_counts(uint32_t* ctrl, int defer, int fallback, uint32_t words, uint32_t* host_defer,
                                  uint32_t* host_fallback, hipStream_t stream) {
-    hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(64), 0, stream, defer, fallback, host_defer,
+    hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(64), 0, stream, ctrl, defer, fallback, words, host_defer,
                        host_fallback);
     return hipGetLastError();
 }

@@ -200,10 +200,9 @@ int ewfa_align_resident(ewfa_ctx_t *ctx, const ewfa_pair_t *h_pairs, size_t n,
 int ewfa_last_timing(ewfa_ctx_t *ctx, float *align_ms, float *emit_ms);
 
 /* Context flags (ewfa_set_flags).  Default: 0 (hipGraph replay of the
- * persistent path, no per-kernel timing). */
+ * persistent path's plans of several passes, no per-kernel timing). */
 #define EWFA_FLAG_TIMING    1  /* record HIP events around the align and
-                                  emit kernels (inside the captured graph on
-                                  the persistent path) */
+                                  emit kernels */
 #define EWFA_FLAG_NO_GRAPH  2  /* launch the persistent path eagerly */
 #define EWFA_FLAG_SERIAL    4  /* run the persistent plan's length-bucket
                                   passes one after another on the context's
@@ -211,8 +210,9 @@ int ewfa_last_timing(ewfa_ctx_t *ctx, float *align_ms, float *emit_ms);
                                   so one pass's tail runs beside the next) */
 int ewfa_set_flags(ewfa_ctx_t *ctx, int flags);
 
-/* Device bytes the context holds now: op scratch, backtrace spill buffer,
- * bucket and deferral lists, control words and the host-pipeline buffers.
+/* Device bytes the context holds now: op scratch, backtrace spill buffer (also
+ * the bit-parallel passes' records), bucket and deferral lists, control words
+ * and the host-pipeline buffers.
  * Buffers grow by at least half again and never wait for the device: one
  * that is replaced is kept (and counted here) until ewfa_destroy, or until an
  * allocation fails, since freeing device memory waits for the whole device. */

@@ -233,3 +233,23 @@ def test_few_long_pairs_with_and_without_bounds(lo, hi, err):
         for _ in range(3):  # eager, recorded, replayed
             res, cig = ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes)
             check(res, w.pairs, cig, d, st, "few long")
+
+
+@pytest.mark.parametrize("order", ["abab", "aacaaba", "bdadbca"])
+def test_control_words_between_calls(order):
+    """Calls of one context that leave its counters at zero, or not: one pass
+    (a), one that defers (b), several buckets (c), longer pairs than before (d)."""
+    print(f"case calls {order}", flush=True)
+    shapes = {"a": (300, 100, 150, 0.03), "b": (300, 640, 700, 0.16), "c": (900, 100, 3000, 0.05), "d": (40, 2000, 5000, 0.1)}
+    made = {}
+    for k, (n, lo, hi, err) in shapes.items():
+        w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=n + lo, len_lo=lo, len_hi=hi, err_lo=err / 2, err_hi=err), n)
+        made[k] = (w, orc.batch_workload(w))
+    with ewfa.Context() as ctx:
+        for k in order:
+            w, (ok, d, sl, st) = made[k]
+            dw, dp = ewfa.DeviceBuffer.from_array(w.words), ewfa.DeviceBuffer.from_array(w.pairs[:w.n])
+            dr, dc = ewfa.DeviceBuffer(w.n * 16), ewfa.DeviceBuffer(w.cigar_bytes)
+            dc.fill_zero()
+            ctx.align_device(dw.ptr, dp.ptr, w.n, w.max_len, dr.ptr, dc.ptr)
+            check(dr.download(ewfa.RESULT_DTYPE, w.n), w.pairs[:w.n], dc.download(np.int8), d, st, order + k)
