@@ -791,7 +791,7 @@ __device__ __forceinline__ float wavefront_cost(float d, bool deep) {
 }
 // Microseconds a wave instruction takes of the whole chip (256 CUs at about
 // 2.3 GHz), and a column of a pair from table to path.
-constexpr float BP_INSTR_US = 1.7e-6f, BP_COLUMN_US = 0.105f;
+constexpr float BP_INSTR_US = 1.7e-6f, BP_COLUMN_US = 0.13f;
 
 // Sum and maximum over the wave, in every lane.
 __device__ __forceinline__ float wave_add(float v) {
@@ -950,22 +950,25 @@ __global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* 
     const uint32_t item = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) / 128u);
     const uint32_t pidx = list ? list[item] : item;
     const ewfa_pair_t pr = a.pairs[pidx];
-    float wfa = 0.f, bp = 0.f, levels = 0.f, columns = 0.f;
+    float edits = 0.f, bases = 0.f, columns = 0.f;
     if (pr.plen <= a.max_len && pr.tlen <= a.max_len && pr.tlen > 0u) {
         const int tl = min((int)pr.tlen, PROBE_BASES), pl = min((int)pr.plen, PROBE_BASES);
         int slope = 0;
-        const uint32_t u = lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl, slope);
+        edits = (float)lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl, slope);
+        bases = (float)tl;
         columns = (float)pr.tlen;
-        levels = (float)u / (float)tl * columns;
-        wfa = wavefront_cost(levels, false);
-        bp = columns * 7.5f + 25.0f * levels;
     }
-    for (int d = 32; d; d >>= 1) {
-        wfa += __shfl_xor(wfa, d);
-        bp += __shfl_xor(bp, d);
-        levels = fmaxf(levels, __shfl_xor(levels, d));
-        columns = fmaxf(columns, __shfl_xor(columns, d));
-    }
+    // the pairs' rates, drawn to their mean by the share of their variance that few
+    // bases explain (the longest chain is that of a true rate, not of a sample's)
+    const float all = fmaxf(wave_add(bases), 1.f), mean = wave_add(edits) / all;
+    const float off = bases > 0.f ? edits / bases - mean : 0.f;
+    const float var = wave_add(off * off), few = 64.f * 64.f * mean / all;
+    const float rate = fminf(mean + off * (var > few ? 1.f - few / var : 0.f), 2.5f * mean);
+    float levels = rate * columns;
+    const float wfa = wave_add(wavefront_cost(levels, false));
+    const float bp = wave_add(columns * 7.5f + 25.0f * levels);
+    levels = wave_most(levels);
+    columns = wave_most(columns);
     // wave instructions a microsecond: 256 CUs at about 2.3 GHz
     const float us = (float)n / 64.0f / 590000.0f;
     const float chain = levels * (1.1f + 0.0005f * levels) * (levels > (float)budget ? 2.0f : 1.0f);
@@ -1051,6 +1054,8 @@ hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t
 
 namespace {
 
+constexpr float LOST_RATE = 0.15f;
+
 // What a pair costs each way: wave instructions of the chip's work, and the us its
 // own chain takes: its levels (about 1.1 us and half a ns a diagonal each, its
 // stream included; twice where the pass's budget of levels defers it), or its
@@ -1059,6 +1064,7 @@ struct BpCost {
     int c;  // class: the narrowest band that holds every path within the bound
             // (BP_CLASSES: no bound, the pair is the wavefront's)
     float wave, bits, wave_us, bits_us;
+    float lost_us;  // a pair without a bound: its levels if it has LOST_RATE edits a base
 };
 
 // A bound beyond the widest band, or above a fifth of the text, mostly comes of a
@@ -1068,15 +1074,21 @@ struct BpCost {
 // lies (if not the pair is deferred); without a guess such pairs stay with the
 // wavefront.
 __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32_t n) {
-    BpCost k{BP_CLASSES, 0.f, 0.f, 0.f, 0.f};
+    BpCost k{BP_CLASSES, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const auto levels_us = [&](float d) { return d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f); };
     const ewfa_pair_t pr = a.pairs[pidx];
     uint32_t u = a.bound[pidx];
-    if (u == BOUND_NONE || pr.plen > a.max_len || pr.tlen > a.max_len || pr.tlen == 0u || pr.plen == 0u) return k;
+    if (pr.plen > a.max_len || pr.tlen > a.max_len || pr.tlen == 0u || pr.plen == 0u) return k;
+    if (u == BOUND_NONE) {
+        k.lost_us = levels_us(LOST_RATE * (float)pr.tlen);
+        return k;
+    }
     const int tk = (int)pr.tlen - (int)pr.plen;
     int S, c = BP_CLASSES - 1;
     while (c > 0 && bp_band(bp_words(c), tk, S) < (int)u) --c;
     const int L = bp_band(bp_words(c), tk, S);
     if (L < (int)u || u > pr.tlen / 5u + 64u) {
+        k.lost_us = levels_us(LOST_RATE * (float)pr.tlen);
         if (!a.guess || n < a.lane_min || L < 0) return k;
         u = a.guess[pidx];
     }
@@ -1084,7 +1096,9 @@ __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32
     k.c = c;
     k.wave = wavefront_cost(d, a.deep);
     k.bits = cols * (bp_column_cost(c) + 2.0f) + 25.0f * d;
-    k.wave_us = d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f);
+    // (few pairs have lost their path, and their guesses are rough: they are no
+    // measure of the list's chains)
+    k.wave_us = k.lost_us > 0.f ? 0.f : levels_us(d);
     k.bits_us = cols * BP_COLUMN_US;
     return k;
 }
@@ -1092,14 +1106,20 @@ __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32
 // The list's way, from its pairs' costs together: every pair by the wavefront
 // (0), each the way with less work (1), or every pair that has a class by the
 // bit-parallel kernel (2).  A way's time is its work and its longest chain, of
-// which few pairs hide nothing (1,500, 5,000 and 15,000 pairs of 10..20 kbp at
+// which they hide about half (1,500, 5,000 and 15,000 pairs of 10..20 kbp at
 // 1..3% edits: 1.8, 3.4 and 9.0 ms by the wavefront, 3.0, 3.4 and 6.4
-// bit-parallel); the two ways of one list run one after the other.
+// bit-parallel); the two ways of one list run one after the other.  A pair without
+// a bound starts first in a wavefront pass, beside the others; without a class it
+// is the wavefront's in any case, after the bit-parallel kernels (3,462 pairs of
+// 12..25 kbp, 61 of them such: 14.0 ms by the wavefront, 15.4 both ways).
 __device__ __forceinline__ int bp_way(const BpWeigh& w) {
-    auto time = [](uint64_t work, uint32_t chain) { return (float)work * BP_INSTR_US + (float)chain; };
-    const float t0 = time(w.wave, w.wave_us);
-    const float t1 = time(w.split_bits, w.split_bits_us) + time(w.split_wave, w.split_wave_us);
-    const float t2 = time(w.bits, w.bits_us);
+    auto time = [](uint64_t work, uint32_t chain) {
+        const float t = (float)work * BP_INSTR_US, l = (float)chain;
+        return fmaxf(t, l) + 0.5f * fminf(t, l);
+    };
+    const float t0 = fmaxf(time(w.wave, w.wave_us), (float)max(w.lost_us, w.rest_us));
+    const float t1 = time(w.split_bits, w.split_bits_us) + time(w.split_wave, w.split_wave_us) + (float)w.rest_us;
+    const float t2 = time(w.bits, w.bits_us) + (float)w.rest_us;
     return t0 <= t1 && t0 <= t2 ? 0 : t1 <= t2 ? 1 : 2;
 }
 
@@ -1126,11 +1146,14 @@ __global__ __launch_bounds__(256) void bp_weigh_kernel(BpArgs a, const uint32_t*
                                                        uint32_t count) {
     const uint32_t n = count_ptr ? *count_ptr : count;
     if (a.flag && *a.flag == 0u) return;
-    float sum[4] = {}, most[4] = {};
+    float sum[4] = {}, most[6] = {};
     for (uint32_t at = blockIdx.x * 256u + threadIdx.x; at < n; at += gridDim.x * 256u) {
         const BpCost k = bp_cost(a, list ? list[at] : at, n);
         const bool bits = k.bits <= k.wave;
-        if (k.c == BP_CLASSES) continue;
+        if (k.c == BP_CLASSES) {
+            most[5] = fmaxf(most[5], k.lost_us);
+            continue;
+        }
         sum[0] += k.wave;
         sum[1] += k.bits;
         sum[2] += bits ? 0.f : k.wave;
@@ -1139,15 +1162,24 @@ __global__ __launch_bounds__(256) void bp_weigh_kernel(BpArgs a, const uint32_t*
         most[1] = fmaxf(most[1], k.bits_us);
         most[2] = fmaxf(most[2], bits ? 0.f : k.wave_us);
         most[3] = fmaxf(most[3], bits ? k.bits_us : 0.f);
+        most[4] = fmaxf(most[4], k.lost_us);
     }
-    uint64_t* const sums = &a.weigh->wave;
-    uint32_t* const mosts = &a.weigh->wave_us;
-    for (int i = 0; i < 4; ++i) {
-        const float v = wave_add(sum[i]), m = wave_most(most[i]);
-        if ((threadIdx.x & 63u) == 0u && v > 0.f) {
-            atomicAdd((unsigned long long*)(sums + i), (unsigned long long)v);
-            atomicMax(mosts + i, (uint32_t)m);
-        }
+    // one wave of the block adds for all (each wave for itself took 0.1 to 0.4 ms of
+    // adds to one line for 80,000 pairs)
+    __shared__ float part[4][10];
+    const int wv = threadIdx.x >> 6;
+    for (int i = 0; i < 10; ++i) {
+        const float v = i < 4 ? wave_add(sum[i]) : wave_most(most[i - 4]);
+        if ((threadIdx.x & 63u) == 0u) part[wv][i] = v;
+    }
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i < 4) {
+        const float v = part[0][i] + part[1][i] + part[2][i] + part[3][i];
+        if (v > 0.f) atomicAdd((unsigned long long*)(&a.weigh->wave + i), (unsigned long long)v);
+    } else if (i < 10) {
+        const float m = fmaxf(fmaxf(part[0][i], part[1][i]), fmaxf(part[2][i], part[3][i]));
+        if (m > 0.f) atomicMax(&a.weigh->wave_us + (i - 4), (uint32_t)m);
     }
 }
 
@@ -1231,7 +1263,7 @@ hipError_t launch_bp_sort(const BpArgs& a, const uint32_t* list, const uint32_t*
                           hipStream_t stream) {
     if (count == 0) return hipSuccess;
     const uint32_t blocks = (count + 255u) / 256u;
-    hipLaunchKernelGGL(bp_weigh_kernel, dim3(blocks < 512u ? blocks : 512u), dim3(256), 0, stream, a, list, count_ptr, count);
+    hipLaunchKernelGGL(bp_weigh_kernel, dim3(blocks < 128u ? blocks : 128u), dim3(256), 0, stream, a, list, count_ptr, count);
     hipLaunchKernelGGL(bp_count_kernel, dim3(blocks), dim3(256), 0, stream, a, list, count_ptr, count);
     hipLaunchKernelGGL(bp_place_kernel, dim3(blocks), dim3(256), 0, stream, a, list, count_ptr, count);
     return hipGetLastError();

@@ -211,6 +211,7 @@ __host__ __device__ inline int bp_band(int N, int tk, int& S) {
 struct BpWeigh {
     uint64_t wave, bits, split_wave, split_bits;          // wave instructions
     uint32_t wave_us, bits_us, split_wave_us, split_bits_us;  // longest chains
+    uint32_t lost_us, rest_us;  // ... of pairs without a bound: with a class, and without
 };
 
 struct BpArgs {
