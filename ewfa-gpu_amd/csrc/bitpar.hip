@@ -1064,8 +1064,13 @@ struct BpCost {
     int c;  // class: the narrowest band that holds every path within the bound
             // (BP_CLASSES: no bound, the pair is the wavefront's)
     float wave, bits, wave_us, bits_us;
+    float edits, bases;
     float lost_us;  // a pair without a bound: its levels if it has LOST_RATE edits a base
 };
+
+__device__ __forceinline__ float bp_levels_us(const BpArgs& a, float d) {
+    return d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f);
+}
 
 // A bound beyond the widest band, or above a fifth of the text, mostly comes of a
 // search whose window lost the path at a long gap: it then says nothing of the
@@ -1074,8 +1079,8 @@ struct BpCost {
 // lies (if not the pair is deferred); without a guess such pairs stay with the
 // wavefront.
 __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32_t n) {
-    BpCost k{BP_CLASSES, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const auto levels_us = [&](float d) { return d * (1.1f + 0.0005f * d) * (d > (float)a.budget ? 2.0f : 1.0f); };
+    BpCost k{BP_CLASSES, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const auto levels_us = [&](float d) { return bp_levels_us(a, d); };
     const ewfa_pair_t pr = a.pairs[pidx];
     uint32_t u = a.bound[pidx];
     if (pr.plen > a.max_len || pr.tlen > a.max_len || pr.tlen == 0u || pr.plen == 0u) return k;
@@ -1100,6 +1105,8 @@ __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32
     // measure of the list's chains)
     k.wave_us = k.lost_us > 0.f ? 0.f : levels_us(d);
     k.bits_us = cols * BP_COLUMN_US;
+    k.edits = d;
+    k.bases = cols;
     return k;
 }
 
@@ -1112,14 +1119,20 @@ __device__ __forceinline__ BpCost bp_cost(const BpArgs& a, uint32_t pidx, uint32
 // a bound starts first in a wavefront pass, beside the others; without a class it
 // is the wavefront's in any case, after the bit-parallel kernels (3,462 pairs of
 // 12..25 kbp, 61 of them such: 14.0 ms by the wavefront, 15.4 both ways).
-__device__ __forceinline__ int bp_way(const BpWeigh& w) {
+__device__ __forceinline__ int bp_way(const BpWeigh& w, const BpArgs& a) {
     auto time = [](uint64_t work, uint32_t chain) {
         const float t = (float)work * BP_INSTR_US, l = (float)chain;
         return fmaxf(t, l) + 0.5f * fminf(t, l);
     };
-    const float t0 = fmaxf(time(w.wave, w.wave_us), (float)max(w.lost_us, w.rest_us));
-    const float t1 = time(w.split_bits, w.split_bits_us) + time(w.split_wave, w.split_wave_us) + (float)w.rest_us;
-    const float t2 = time(w.bits, w.bits_us) + (float)w.rest_us;
+    // (a loose bound is no distance: no chain of more than 2.5 times the mean rate)
+    const float most = bp_levels_us(a, 2.5f * (float)w.edits / (float)max(w.bases, (uint64_t)1) * (float)w.bits_us /
+                                           BP_COLUMN_US);
+    // (wide and narrow classes of a deep bucket run one after the other)
+    const uint32_t twice = a.deep && w.wide_us ? w.wide_us : 0u;
+    const float t0 = fmaxf(time(w.wave, min(w.wave_us, (uint32_t)most)), (float)max(w.lost_us, w.rest_us));
+    const float t1 = time(w.split_bits, w.split_bits_us + twice) +
+                     time(w.split_wave, min(w.split_wave_us, (uint32_t)most)) + (float)w.rest_us;
+    const float t2 = time(w.bits, w.bits_us + twice) + (float)w.rest_us;
     return t0 <= t1 && t0 <= t2 ? 0 : t1 <= t2 ? 1 : 2;
 }
 
@@ -1136,7 +1149,7 @@ __device__ __forceinline__ int bp_bin_of(const BpArgs& a, uint32_t pidx, int way
 
 // The way of a list: what the sample said, else its pairs' sums.
 __device__ __forceinline__ int bp_list_way(const BpArgs& a) {
-    return a.flag && *a.flag == 0u ? 0 : bp_way(*a.weigh);
+    return a.flag && *a.flag == 0u ? 0 : bp_way(*a.weigh, a);
 }
 
 }  // namespace
@@ -1146,7 +1159,7 @@ __global__ __launch_bounds__(256) void bp_weigh_kernel(BpArgs a, const uint32_t*
                                                        uint32_t count) {
     const uint32_t n = count_ptr ? *count_ptr : count;
     if (a.flag && *a.flag == 0u) return;
-    float sum[4] = {}, most[6] = {};
+    float sum[6] = {}, most[7] = {};
     for (uint32_t at = blockIdx.x * 256u + threadIdx.x; at < n; at += gridDim.x * 256u) {
         const BpCost k = bp_cost(a, list ? list[at] : at, n);
         const bool bits = k.bits <= k.wave;
@@ -1162,24 +1175,29 @@ __global__ __launch_bounds__(256) void bp_weigh_kernel(BpArgs a, const uint32_t*
         most[1] = fmaxf(most[1], k.bits_us);
         most[2] = fmaxf(most[2], bits ? 0.f : k.wave_us);
         most[3] = fmaxf(most[3], bits ? k.bits_us : 0.f);
+        sum[4] += k.edits;
+        sum[5] += k.bases;
         most[4] = fmaxf(most[4], k.lost_us);
+        most[6] = fmaxf(most[6], bp_group(k.c, a.spread) >= 32 ? k.bits_us : 0.f);
     }
     // one wave of the block adds for all (each wave for itself took 0.1 to 0.4 ms of
     // adds to one line for 80,000 pairs)
-    __shared__ float part[4][10];
+    constexpr int SUMS = 6, ALL = SUMS + 7;
+    __shared__ float part[4][ALL];
     const int wv = threadIdx.x >> 6;
-    for (int i = 0; i < 10; ++i) {
-        const float v = i < 4 ? wave_add(sum[i]) : wave_most(most[i - 4]);
+#pragma unroll
+    for (int i = 0; i < ALL; ++i) {
+        const float v = i < SUMS ? wave_add(sum[i]) : wave_most(most[i - SUMS]);
         if ((threadIdx.x & 63u) == 0u) part[wv][i] = v;
     }
     __syncthreads();
     const int i = threadIdx.x;
-    if (i < 4) {
+    if (i < SUMS) {
         const float v = part[0][i] + part[1][i] + part[2][i] + part[3][i];
         if (v > 0.f) atomicAdd((unsigned long long*)(&a.weigh->wave + i), (unsigned long long)v);
-    } else if (i < 10) {
+    } else if (i < ALL) {
         const float m = fmaxf(fmaxf(part[0][i], part[1][i]), fmaxf(part[2][i], part[3][i]));
-        if (m > 0.f) atomicMax(&a.weigh->wave_us + (i - 4), (uint32_t)m);
+        if (m > 0.f) atomicMax(&a.weigh->wave_us + (i - SUMS), (uint32_t)m);
     }
 }
 

@@ -209,9 +209,11 @@ __host__ __device__ inline int bp_band(int N, int tk, int& S) {
 // A list's costs each way (bp_cost): all by the wavefront, all bit-parallel,
 // each the way with less work.
 struct BpWeigh {
-    uint64_t wave, bits, split_wave, split_bits;          // wave instructions
+    uint64_t wave, bits, split_wave, split_bits;  // wave instructions
+    uint64_t edits, bases;                        // bounds and columns
     uint32_t wave_us, bits_us, split_wave_us, split_bits_us;  // longest chains
     uint32_t lost_us, rest_us;  // ... of pairs without a bound: with a class, and without
+    uint32_t wide_us;           // ... of the classes of 32 lanes and more
 };
 
 struct BpArgs {
