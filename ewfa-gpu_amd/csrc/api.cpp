@@ -871,12 +871,13 @@ int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len,
          bool deeper = false) {
     // a wave a pair while its lists are short: a lane's steps wait for memory,
     // which takes many more pairs to hide (3,000 pairs of 1..10 kbp at 1..5% edits
-    // 1,098 -> 815 us, 30,000 of 8 kbp at 1.1% 1,630 -> 1,480; but 86,000 of 2.3 kbp
-    // at 2.1% 1,498 by lanes and 1,776 by waves; where both sequences take more than
-    // 12 KB of LDS, few waves: 1,500 pairs of 10..20 kbp 1,926 -> 1,628, none of it
-    // left at 3,000).  Beside a bucket whose narrow slots just fill the LDS (deeper),
+    // 1,098 -> 815 us; but 86,000 of 2.3 kbp at 2.1% 1,498 by lanes and 1,776 by
+    // waves).  Both sequences in LDS leave fewer waves the longer they are: above
+    // 6 KB lanes win earlier (21,442 pairs of 8.7 kbp at 3.9% 3,641 and 3,879), above
+    // 12 KB soon (1,500 pairs of 10..20 kbp 1,926 -> 1,628, none of it left at 3,000).  Beside a bucket whose narrow slots just fill the LDS (deeper),
     // its blocks would keep one of those off every CU.
-    const uint32_t per_cu = deeper ? FEW_PER_CU : (size_t)2 * overlapped_words_for(max_len) * 8 <= 12288 ? 128u : 8u;
+    const size_t lds = (size_t)2 * overlapped_words_for(max_len) * 8;
+    const uint32_t per_cu = deeper ? FEW_PER_CU : lds <= 6144 ? 128u : lds <= 12288 ? 60u : 8u;
     if (staged && items <= (uint32_t)c->num_cus * per_cu) return emit_list(c, e, items, max_len, s);
     const int sw = seq_words_for(max_len);
     if (staged && sw <= ewfa::EMIT_LDS_MAX_SW)
