@@ -354,8 +354,8 @@ constexpr uint32_t BP_SPREAD_BELOW = 32768;
 // Pairs per CU up to which a list counts as few.
 constexpr uint32_t FEW_PER_CU = 4;
 
-// The bit-parallel pass ahead of a block bucket pass: it takes the pairs for
-// which it is the cheaper way (bp_class_of).  Not under a distance cap, whose
+// The bit-parallel pass ahead of a block bucket pass: it takes the pairs, or the
+// lists, for which it is the faster way (bp_way).  Not under a distance cap, whose
 // output is the wavefront's at the capped level.
 void choose_bp(ewfa_ctx* c, Pass& p, uint32_t blen, uint32_t items) {
     p.bp_grid = 0;

@@ -932,14 +932,12 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
 }  // namespace
 
 // Whether a list takes the bit-parallel way at all, from a sample: 64 of its
-// pairs, a lane each, and the edits in the first PROBE_BASES of each.  The
-// wavefront's time is its work, or its longest pair's levels (about 0.4 us and
-// 0.5 ns a diagonal each, and 0.7 us an op for the stream), twice where the pass's
-// budget of levels defers the pair; the bit-parallel one its work, or its longest
-// pair's columns of about 0.35 us (bounds, table and path).  (Short lists of moderate lengths go faster
-// through the wavefront: jobs of 100..5,000 bp at 1..10% edits in batches of
-// 25,000 pairs 5.6 against 7.4 ms, while 15,001 pairs of 3..7 kbp at 8..15%
-// take 3.3 against 5.9.)  The sample takes about 25 us.
+// pairs, a lane each, and the edits in the first PROBE_BASES of each (25 us).  The
+// wavefront's time is its work, or its longest pair's levels (as in bp_way); the
+// bit-parallel one its work, or its longest pair's columns of about 0.35 us (bounds,
+// table and path).  Jobs of 100..5,000 bp at 1..10% edits in batches of 25,000
+// pairs take 5.6 ms by the wavefront and 7.4 bit-parallel, 15,001 pairs of 3..7 kbp
+// at 8..15% 5.9 and 2.9.
 constexpr int PROBE_BASES = 256;
 constexpr float FEW_LEVELS = 512.0f;
 
