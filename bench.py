@@ -5,9 +5,9 @@ Headline workload (the JSON `value`): 1,000,000 pairs of 1,000 bp, uniform
 ACGT, 5% edits split equally between substitution, insertion and deletion
 (seed 2), 2-bit packed uint64 input resident in HBM, the reference's
 per-pair CIGAR buffer of 1,004 bytes.  One step = distances and full CIGAR
-streams for all 1,000,000 pairs on the persistent path (one hipGraph-launched
-persistent kernel over a device work queue, then the emit kernel), under the
-launch policy the autotuner wrote for this workload.
+streams for all 1,000,000 pairs on the persistent path (one persistent kernel
+over a device work queue, which writes the streams, then the emit of the few it
+leaves), under the launch policy the autotuner wrote for this workload.
 
 Beside it, on the same box and run:
   plain      the reference's launch model (batches of 100,000, one workgroup
@@ -17,12 +17,12 @@ Beside it, on the same box and run:
   c3         500,000 pairs, log-uniform 100..10,000 bp, 1..10% edits, one
              launch under the autotuned per-bucket policy
   c4         20,000 pairs of 10..50 kbp at 10..15% edits with indel runs
-             (backtrace spilled to HBM), with the device footprint
+             (the bit-parallel pass, its records in HBM), with the device footprint
   served     Poisson arrivals of jobs of 1..4,096 pairs (lengths and errors as
              c3) into the job server; p50/p99 latency from arrival to results
              in host memory, and alignments/s against the c3 batched rate
   roofline   algorithmic bytes per align launch / its average duration from
-             HIP events recorded (inside the graph) on its launch stream
+             HIP events recorded on its launch stream
   cpu        the oracle (a C restatement of the reference's algorithm with its
              CPU validity check) on a bounded sample, and on c1
 """
@@ -116,7 +116,7 @@ def leg_c2(args, threads):
     r = Resident(w)
     out = {}
 
-    # the value: persistent path, hipGraph replay, timing events in the graph
+    # the value: persistent path, with timing events around its launches
     ctx = ewfa.Context(mode=ewfa.MODE_PERSISTENT, flags=ewfa.FLAG_TIMING, policy_path=POLICY_C2)
     dt, a_ms, e_ms = timed(r.run, ctx, args.steps, args.warmup)
     out["value"] = args.steps * n / dt
@@ -583,7 +583,7 @@ def main():
         return
 
     if args.profile_run:
-        # the bench's own timed loop for one workload (graph replay with the
+        # the bench's own timed loop for one workload (with the
         # timing events, --warmup then --steps calls), so that a profiler's
         # per-kernel averages compare with the bench's kernels_ms
         name = args.profile_run
@@ -675,7 +675,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": "1,000,000 pairs x 1,000 bp, uniform ACGT, 5% edits (sub/ins/del equal), seed 2; "
                                "2-bit packed u64 input resident in HBM, CIGAR stride 1004 B; persistent kernel, "
-                               "hipGraph replay, autotuned policy",
+                               "autotuned policy",
                    "pairs": n, "seq_len": 1000, "error": 0.05, "plain_batch": args.batch,
                    "parallelism": "single GPU"},
         "kernels_ms": {"align": round(c2["align_ms"], 4), "emit": round(c2["emit_ms"], 4)},
