@@ -596,6 +596,21 @@ void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t n, Chain& 
     g_err.clear();
 }
 
+// The levels within which every pair ends in its bucket's pass: the least of
+// the passes' budgets.  A narrow slot and a bit-parallel band hold less than the
+// pass's budget (at 9.5 kbp 9,600 and 8,129 of 9,900 levels), and what they defer
+// needs a pass after them even where the budget exceeds any distance: the chain
+// then ends with one of max_len + 1 levels.
+int plan_reach(const Plan& pl, uint32_t max_len) {
+    int reach = pl.pass[0].dcap;
+    for (int b = 0; b < pl.nb; ++b) {
+        const Pass& p = pl.pass[b];
+        reach = std::min(reach, p.dcap);
+        if (p.band_cap > 0 || p.bp_grid > 0) reach = (int)std::min((uint32_t)reach, max_len);
+    }
+    return reach;
+}
+
 // Longest pairs of a banded pass over a whole list: up to here (5.7 KB of LDS a
 // wave) a CU holds 28 of its waves.
 constexpr uint32_t BANDED_ONE_LEN = 3000;
@@ -614,7 +629,7 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         // where a pair has more (7 pairs of 135..675 bp at 4..15%: 153 -> 105 us)
         if (c->builtin_policy && bp.dcap == 63 && max_len > 420) bp.dcap = REG4_LEVELS;
         CHK(pass_from_bucket(c, bp, max_len, n, pl.pass[0]));
-        plan_chain(c, max_len, pl.pass[0].dcap, n, pl.chain);
+        plan_chain(c, max_len, plan_reach(pl, max_len), n, pl.chain);
         assign_slots(pl);
         return EWFA_OK;
     }
@@ -646,9 +661,7 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         if (max_len <= b.len_hi) break;
     }
     pl.table.nb = pl.nb;
-    int dcap_min = pl.pass[0].dcap;
-    for (int b = 1; b < pl.nb; ++b) dcap_min = std::min(dcap_min, pl.pass[b].dcap);
-    plan_chain(c, max_len, dcap_min, n, pl.chain);
+    plan_chain(c, max_len, plan_reach(pl, max_len), n, pl.chain);
     pl.fanout = std::min(pl.nb, c->fanout);
     assign_slots(pl);
     return EWFA_OK;

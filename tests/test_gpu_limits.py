@@ -1,0 +1,58 @@
+"""Calls at the limits of what their passes hold, against the oracle."""
+import numpy as np
+import pytest
+
+import ewfa
+from test_gpu_bitpar import POLICY
+from test_gpu_bound import check, policy_file
+from test_gpu_stress import oracle_streams
+
+pytestmark = pytest.mark.gpu
+
+BASES = np.frombuffer(b"ACGT", dtype=np.uint8)
+
+
+class OnDevice:
+    """Sequences, descriptors and outputs in device memory."""
+
+    def __init__(self, words, pairs, cigar_bytes, max_len):
+        self.pairs, self.n, self.max_len = pairs, len(pairs), max_len
+        self.dw, self.dp = ewfa.DeviceBuffer.from_array(words), ewfa.DeviceBuffer.from_array(pairs)
+        self.dr, self.dc = ewfa.DeviceBuffer(self.n * 16), ewfa.DeviceBuffer(cigar_bytes)
+        self.dc.fill_zero()
+
+    def align(self, ctx):
+        ctx.align_device(self.dw.ptr, self.dp.ptr, self.n, self.max_len, self.dr.ptr, self.dc.ptr)
+        return self
+
+    def check(self, d, st, label):
+        check(self.dr.download(ewfa.RESULT_DTYPE, self.n), self.pairs, self.dc.download(np.int8), d, st, label)
+
+
+def fill_pairs(count, lo=40, hi=260, seed=3):
+    """Short pairs of a few substitutions, and their oracle outputs."""
+    rng = np.random.default_rng(seed)
+    pool = []
+    for _ in range(200):
+        p = rng.choice(BASES, int(rng.integers(lo, hi)))
+        t = p.copy()
+        t[rng.integers(0, len(t), 3)] = rng.choice(BASES, 3)
+        pool.append((p.tobytes(), t.tobytes()))
+    d, st = oracle_streams([p for p, _ in pool], [t for _, t in pool])
+    take = [i % len(pool) for i in range(count)]
+    return [pool[i][0] for i in take], [pool[i][1] for i in take], [d[i] for i in take], [st[i] for i in take]
+
+
+@pytest.mark.parametrize("count", [300, 8300])
+def test_distances_beyond_the_narrow_slots_and_the_widest_band(tmp_path, count):
+    """One bucket whose budget exceeds any distance: pairs beyond what its
+    narrow slots hold (9,600 levels at this length), and beyond the widest
+    band of the bit-parallel pass (8,129), which defer them."""
+    print(f"case beyond the bands: {count} pairs", flush=True)
+    # nothing in common: as many substitutions as bases
+    P, T = [b"A" * n for n in (9700, 9500, 8200, 9400)], [b"C" * n for n in (9700, 9500, 8200, 9400)]
+    d, st = [len(p) for p in P], [np.full(len(p), ord("X"), dtype=np.int8) for p in P]
+    fp, ft, fd, fst = fill_pairs(count - len(P))
+    case = OnDevice(*ewfa.from_sequences(P + fp, T + ft))
+    with ewfa.Context(policy_path=policy_file(tmp_path, "one", POLICY)) as ctx:
+        case.align(ctx).check(d + fd, st + fst, "beyond the bands")
