@@ -1316,22 +1316,6 @@ int pipeline_upload(ewfa_ctx* c, const Chunk& ch, size_t k, const uint64_t* h_wo
     return EWFA_OK;
 }
 
-// Device address of `bytes` of host memory at p when they are pinned (one
-// allocation, by both ends), else null.
-template <typename T>
-T* mapped_host(T* p, size_t bytes) {
-    hipPointerAttribute_t a{}, b{};
-    char* const last = reinterpret_cast<char*>(p) + (bytes ? bytes - 1 : 0);
-    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&b, last) != hipSuccess) {
-        (void)hipGetLastError();  // ordinary memory
-        return nullptr;
-    }
-    if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || !a.devicePointer || !b.devicePointer ||
-        static_cast<char*>(b.devicePointer) - static_cast<char*>(a.devicePointer) != last - reinterpret_cast<char*>(p))
-        return nullptr;
-    return static_cast<T*>(a.devicePointer);
-}
-
 // The caller's output buffers of a host-pipeline call, and their device
 // addresses where they are pinned: such streams and results go straight to
 // their places, without the stage and the host threads that place it.
@@ -1469,8 +1453,9 @@ int run_pipeline(ewfa_ctx* c, const uint64_t* h_words, size_t n_words, const ewf
     // size the per-chunk scratch for the largest chunk before any chunk
     // computes, so that no buffer is replaced while chunks are in flight
     if (rc == EWFA_OK) rc = reserve_scratch(c, most, max_len);
-    const HostOut out{h_results, h_cigars, mapped_host(h_results, n * sizeof(ewfa_result_t)),
-                      mapped_host(h_cigars, cigar_bytes)};
+    const HostOut out{h_results, h_cigars,
+                      static_cast<ewfa_result_t*>(ewfa::mapped_host(h_results, n * sizeof(ewfa_result_t))),
+                      static_cast<int8_t*>(ewfa::mapped_host(h_cigars, cigar_bytes))};
     size_t enq = 0, done = 0;
     for (size_t k = 0; k < chunks.size() && rc == EWFA_OK; ++k) {
         if (!h_words) rc = words_wait(c, chunks[k].w_hi);
@@ -1500,6 +1485,19 @@ int set_error(int code, const char* fmt, ...) {
     va_end(ap);
     g_err = buf;
     return code;
+}
+
+void* mapped_host(void* p, size_t bytes) {
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost || !a.devicePointer ||
+        hipMemGetAddressRange(&base, &size, a.devicePointer) != hipSuccess) {
+        (void)hipGetLastError();  // ordinary memory
+        return nullptr;
+    }
+    const size_t at = (size_t)(static_cast<char*>(a.devicePointer) - static_cast<char*>(base));
+    return at <= size && bytes <= size - at ? a.devicePointer : nullptr;
 }
 
 size_t op_scratch_bytes(size_t n, uint32_t max_len) { return n * (size_t)ops_words(max_len + 1) * 8; }

@@ -51,6 +51,10 @@ int align_device_with_scratch(ewfa_ctx_t* ctx, const uint64_t* d_words, const ew
                               uint32_t max_len, ewfa_result_t* d_results, int8_t* d_cigars, void* stream,
                               uint64_t* d_ops, size_t ops_bytes);
 
+// Device address of `bytes` of host memory at p when all of them lie in one
+// pinned allocation, else null.
+void* mapped_host(void* p, size_t bytes);
+
 // The context's own stream (its kernels run there).
 hipStream_t context_stream(ewfa_ctx_t* ctx);
 

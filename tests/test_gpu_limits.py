@@ -1,4 +1,6 @@
 """Calls at the limits of what their passes hold, against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -56,3 +58,21 @@ def test_distances_beyond_the_narrow_slots_and_the_widest_band(tmp_path, count):
     case = OnDevice(*ewfa.from_sequences(P + fp, T + ft))
     with ewfa.Context(policy_path=policy_file(tmp_path, "one", POLICY)) as ctx:
         case.align(ctx).check(d + fd, st + fst, "beyond the bands")
+
+
+def test_outputs_are_pinned_only_within_one_allocation():
+    """Buffers the device may write as they are: parts of one pinned
+    allocation, and nothing that reaches past its end into another."""
+    print("case pinned ranges", flush=True)
+    mapped = ewfa.lib()._ZN4ewfa11mapped_hostEPvm
+    mapped.restype, mapped.argtypes = ctypes.c_void_p, [ctypes.c_void_p, ctypes.c_size_t]
+    size = 3 << 20
+    held = [ewfa.PinnedArray(size, np.uint8) for _ in range(2)]
+    a, b = sorted(h.array.ctypes.data for h in held)
+    assert mapped(a, size) and mapped(a + 4096, size - 4096) and mapped(a + size - 4, 4) and mapped(b, 0)
+    assert not mapped(a, b - a + size)  # both ends pinned, and what lies between not known to be
+    assert not mapped(a + 4, size)
+    plain = np.zeros(size, dtype=np.uint8)
+    assert not mapped(plain.ctypes.data, size)
+    dev = ewfa.DeviceBuffer(size)
+    assert not mapped(dev.ptr, size)
