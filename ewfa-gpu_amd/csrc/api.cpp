@@ -1297,7 +1297,9 @@ int pipeline_setup(ewfa_ctx* c, size_t chunks) {
         c->ev_up.push_back(e);
     }
     for (ewfa_ctx::Stage& st : c->stage)
-        if (!st.done) HIPCHK(hipEventCreateWithFlags(&st.done, hipEventDisableTiming));
+        // released to the system: streams placed in a caller's pinned memory by the
+        // device's stores are to be seen by the host, non-coherent memory included
+        if (!st.done) HIPCHK(hipEventCreateWithFlags(&st.done, hipEventDisableTiming | hipEventReleaseToSystem));
     return EWFA_OK;
 }
 

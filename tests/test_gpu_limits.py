@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import ewfa
+import oracle_py as orc
 from test_gpu_bitpar import POLICY
 from test_gpu_bound import check, policy_file
 from test_gpu_stress import oracle_streams
@@ -76,3 +77,35 @@ def test_outputs_are_pinned_only_within_one_allocation():
     assert not mapped(plain.ctypes.data, size)
     dev = ewfa.DeviceBuffer(size)
     assert not mapped(dev.ptr, size)
+
+
+@pytest.mark.parametrize("flags", [0, 0x40000000, 0x80000000])  # default, coherent, non-coherent
+def test_streams_in_pinned_memory_of_every_kind(flags):
+    """Calls one after the other into the same pinned buffers, read by the host
+    after each."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def pinned(nbytes):
+        p = ctypes.c_void_p()
+        assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes), ctypes.c_uint(flags)) == 0
+        return p, np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_int8)), (nbytes,))
+
+    print(f"case pinned memory {flags:#x}", flush=True)
+    ewfa.synchronize()
+    loads = []
+    for seed in range(3):
+        w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=seed, len_lo=100, len_hi=700, err_lo=0.01, err_hi=0.1), 3000,
+                          cigar_cap=160)
+        ok, d, sl, st = orc.batch_workload(w)
+        loads.append((w, d, st))
+    pr, res = pinned(3000 * 16)
+    pc, cig = pinned(3000 * 160)
+    res = res.view(ewfa.RESULT_DTYPE)
+    with ewfa.Context() as ctx:
+        for k in (0, 1, 2, 0, 1, 2):
+            w, d, st = loads[k]
+            cig[:] = 1
+            ctx.align_host(w.words, w.pairs, w.n, w.cigar_bytes, results=res, cigars=cig)
+            check(res, w.pairs[:w.n], cig, d, st, (flags, k))
+    for p in (pr, pc):
+        assert hip.hipHostFree(p) == 0
