@@ -1381,6 +1381,10 @@ int pipeline_complete(ewfa_ctx* c, const Chunk& ch, size_t k, const ewfa_pair_t*
 
 // h_words null: the words of the last ewfa_upload_words are resident.  The
 // descriptors are checked while the chunks are formed.
+// Bytes of a buffer for n_words uploaded words: the kernels read a sequence's pad
+// word, which may lie just past the upload's last.
+size_t words_bytes(size_t n_words) { return (n_words + 1) * 8; }
+
 // Words per piece of an asynchronous upload (16 MiB).
 constexpr size_t WORDS_PIECE = (size_t)2 << 20;
 
@@ -1405,7 +1409,7 @@ int run_pipeline(ewfa_ctx* c, const uint64_t* h_words, size_t n_words, const ewf
                  ewfa_result_t* h_results, int8_t* h_cigars, size_t cigar_bytes) {
     if (h_words) {
         CHK(words_settle(c));
-        CHK(c->h_words.reserve(c, std::max<size_t>(n_words, 1) * 8));
+        CHK(c->h_words.reserve(c, words_bytes(n_words)));
         c->resident_words = 0;  // only the words these pairs read go up
     }
     CHK(c->h_pairs.reserve(c, n * sizeof(ewfa_pair_t)));
@@ -2010,7 +2014,7 @@ int ewfa_upload_words(ewfa_ctx_t* c, const uint64_t* h_words, size_t n_words) {
     if (!h_words && n_words) return fail(EWFA_ERR_ARG, "null buffer");
     CHK(set_device(c));
     CHK(words_settle(c));
-    CHK(c->h_words.reserve(c, std::max<size_t>(n_words, 1) * 8));
+    CHK(c->h_words.reserve(c, words_bytes(n_words)));
     if (n_words) {
         HIPCHK(hipMemcpyAsync(c->h_words.p, h_words, n_words * 8, hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -2026,7 +2030,7 @@ int ewfa_upload_words_async(ewfa_ctx_t* c, const uint64_t* h_words, size_t n_wor
     CHK(words_settle(c));
     // work already queued on the context may still read the old words
     HIPCHK(hipStreamSynchronize(c->stream));
-    CHK(c->h_words.reserve(c, std::max<size_t>(n_words, 1) * 8));
+    CHK(c->h_words.reserve(c, words_bytes(n_words)));
     c->resident_words = n_words;
     if (n_words == 0) return EWFA_OK;
     if (!c->wup) HIPCHK(hipStreamCreateWithFlags(&c->wup, hipStreamNonBlocking));

@@ -47,7 +47,8 @@ public:
 
     int init(int device, size_t bytes) {
         if (hipSetDevice(device) != hipSuccess) return EWFA_ERR_HIP;
-        if (hipMalloc(&base_, bytes) != hipSuccess) {
+        // (a block's last sequence may have its pad word, which kernels read, just past it)
+        if (hipMalloc(&base_, bytes + kAlign) != hipSuccess) {
             base_ = nullptr;
             return EWFA_ERR_NOMEM;
         }

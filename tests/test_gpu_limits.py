@@ -109,3 +109,17 @@ def test_streams_in_pinned_memory_of_every_kind(flags):
             check(res, w.pairs[:w.n], cig, d, st, (flags, k))
     for p in (pr, pc):
         assert hip.hipHostFree(p) == 0
+
+
+@pytest.mark.parametrize("entry", ["ewfa_upload_words", "ewfa_upload_words_async"])
+def test_uploaded_words_have_room_for_the_last_pad_word(entry):
+    """The last sequence's pad word, which kernels read, may lie just past the
+    words given: the context's buffer holds it."""
+    n = 1 << 18  # whole pages of words
+    print(f"case pad word {entry}", flush=True)
+    words = np.zeros(n, dtype=np.uint64)
+    with ewfa.Context() as ctx:
+        before = ctx.memory_bytes()
+        assert getattr(ewfa.lib(), entry)(ctx.handle, ctypes.c_void_p(words.ctypes.data), ctypes.c_size_t(n)) == 0
+        ewfa.synchronize()
+        assert ctx.memory_bytes() - before >= (n + 1) * 8
