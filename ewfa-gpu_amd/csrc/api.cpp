@@ -621,17 +621,22 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
     if (!capped && n <= (uint32_t)c->num_cus && max_len > c->policy.buckets.front().len_hi) {
         // at most a pair per CU: the call lasts as long as its longest pair,
         // so all go through that pair's pass, without bucketing and the fork
-        // over streams (60 pairs of 100..2,000 bp: 175 -> 130 us)
-        pl.nb = 1;
+        // over streams (60 pairs of 100..2,000 bp: 175 -> 130 us).  Not through one
+        // with its slots in HBM, of which there may be a single one (60 pairs of
+        // 10 kbp beside one of 400 kbp: 15.2 ms so, 6.6 ms by their buckets)
         pl.blen[0] = max_len;
         ewfa::BucketPolicy bp = c->policy.bucket_for(max_len);
         // nothing to gain from 63 levels alone here, and a second pass to lose
         // where a pair has more (7 pairs of 135..675 bp at 4..15%: 153 -> 105 us)
         if (c->builtin_policy && bp.dcap == 63 && max_len > 420) bp.dcap = REG4_LEVELS;
         CHK(pass_from_bucket(c, bp, max_len, n, pl.pass[0]));
-        plan_chain(c, max_len, plan_reach(pl, max_len), n, pl.chain);
-        assign_slots(pl);
-        return EWFA_OK;
+        if (!pl.pass[0].gslot) {
+            pl.nb = 1;
+            plan_chain(c, max_len, plan_reach(pl, max_len), n, pl.chain);
+            assign_slots(pl);
+            return EWFA_OK;
+        }
+        pl = Plan{};
     }
     // Under a cap of at most 64 every search ends within 63 levels, which the
     // banded register pass holds whatever the length: one such pass without

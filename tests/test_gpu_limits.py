@@ -1,5 +1,6 @@
 """Calls at the limits of what their passes hold, against the oracle."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -123,3 +124,29 @@ def test_uploaded_words_have_room_for_the_last_pad_word(entry):
         assert getattr(ewfa.lib(), entry)(ctx.handle, ctypes.c_void_p(words.ctypes.data), ctypes.c_size_t(n)) == 0
         ewfa.synchronize()
         assert ctx.memory_bytes() - before >= (n + 1) * 8
+
+
+def test_short_pairs_beside_one_beyond_lds_are_not_served_in_turn():
+    """A call of few pairs, one of which needs its slot in HBM: the others run
+    beside it, so that the call takes little longer than that pair alone."""
+    print("case 60 pairs of 10 kbp and one of 400 kbp", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=5, len_lo=9000, len_hi=10000, err_lo=0.01, err_hi=0.02), 60)
+    P, T = [bytes(w.pattern(i)) for i in range(60)], [bytes(w.text(i)) for i in range(60)]
+    rng = np.random.default_rng(4)
+    p = rng.choice(BASES, 400_000)
+    t = p.copy()
+    at = rng.choice(400_000, 300, replace=False)
+    t[at] = BASES[(np.searchsorted(BASES, t[at]) + 1) % 4]
+    d, st = oracle_streams(P + [p.tobytes()], T + [t.tobytes()])
+    took = []
+    for a, b, dd, ss in (([], [], [], []), (P, T, list(d[:60]), list(st[:60]))):
+        case = OnDevice(*ewfa.from_sequences(a + [p.tobytes()], b + [t.tobytes()]))
+        with ewfa.Context() as ctx:
+            case.align(ctx).check(dd + [d[60]], ss + [st[60]], "beside 400 kbp")
+            times = []
+            for _ in range(7):
+                t0 = time.perf_counter()
+                case.align(ctx)
+                times.append(time.perf_counter() - t0)
+        took.append(sorted(times)[3])
+    assert took[1] < 1.6 * took[0], took
