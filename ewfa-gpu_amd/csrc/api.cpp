@@ -235,6 +235,7 @@ struct Pass {
     int seq_words;
     int reg;  // register-wavefront chunks (0: offsets staged in LDS)
     int off16;  // 16-bit LDS offsets (block kernel, backtrace in HBM, no bounds)
+    uint32_t defer_len;  // register pass: longer pairs are deferred untried (0: none)
     int band_cap;  // bounded pass with narrow slots: the largest bound they hold (0: none)
     size_t lds;
     uint32_t grid;
@@ -559,13 +560,18 @@ constexpr size_t REG4_CHAIN_LDS = 10240;
 // The longest pairs of the built-in policy's register passes.
 constexpr uint32_t REG_LEN = 1200;
 
-void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t n, Chain& ch) {
+// reg_len: the longest pairs that passes of fewer levels than it defer (0: none).
+void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t reg_len, uint32_t n, Chain& ch) {
     ch = Chain{};
     int dcap = dcap_min;
     // what a banded pass defers (63 levels) mostly ends within 127, which a wave
     // holds in registers: 100,000 pairs of 521 bp at 14.5% edits, all deferred,
-    // took 10,154 us through the block passes below alone, 1,570 so
-    if (dcap < REG4_LEVELS) {
+    // took 10,154 us through the block passes below alone, 1,570 so.  Pairs that
+    // passes of as many levels deferred go on untried, and the passes after this
+    // one are those there would be without it: 2,210 pairs of 4.8 kbp at 12.6%
+    // (600 edits, beyond their bucket's 512) took 7.3 ms where 127, 508 and 4,761
+    // levels followed each other in place of 256 and 1,024 (2.5 ms).
+    if (reg_len > 0) {
         const int ow = overlapped_words_for(max_len);
         if (ewfa::lds_bytes_reg(ow, REG4_LEVELS, 4) <= REG4_CHAIN_LDS) {
             Pass p{};
@@ -576,10 +582,8 @@ void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t n, Chain& 
             p.grab = 4;
             p.reg = 4;
             p.dcap = REG4_LEVELS;
-            if (finish_pass(c, p, n) == EWFA_OK) {
-                ch.pass[ch.np++] = p;
-                dcap = p.dcap;
-            }
+            p.defer_len = reg_len;
+            if (finish_pass(c, p, n) == EWFA_OK) ch.pass[ch.np++] = p;
         }
     }
     while (ch.np < MAX_CHAIN) {
@@ -611,6 +615,14 @@ int plan_reach(const Plan& pl, uint32_t max_len) {
     return reach;
 }
 
+// The longest pairs of the passes below the four-chunk register pass's levels.
+uint32_t plan_reg_len(const Plan& pl) {
+    uint32_t len = 0;
+    for (int b = 0; b < pl.nb; ++b)
+        if (pl.pass[b].dcap < REG4_LEVELS) len = std::max(len, pl.blen[b]);
+    return len;
+}
+
 // Longest pairs of a banded pass over a whole list: up to here (5.7 KB of LDS a
 // wave) a CU holds 28 of its waves.
 constexpr uint32_t BANDED_ONE_LEN = 3000;
@@ -632,7 +644,7 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         CHK(pass_from_bucket(c, bp, max_len, n, pl.pass[0]));
         if (!pl.pass[0].gslot) {
             pl.nb = 1;
-            plan_chain(c, max_len, plan_reach(pl, max_len), n, pl.chain);
+            plan_chain(c, max_len, plan_reach(pl, max_len), plan_reg_len(pl), n, pl.chain);
             assign_slots(pl);
             return EWFA_OK;
         }
@@ -666,7 +678,7 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         if (max_len <= b.len_hi) break;
     }
     pl.table.nb = pl.nb;
-    plan_chain(c, max_len, plan_reach(pl, max_len), n, pl.chain);
+    plan_chain(c, max_len, plan_reach(pl, max_len), plan_reg_len(pl), n, pl.chain);
     pl.fanout = std::min(pl.nb, c->fanout);
     assign_slots(pl);
     return EWFA_OK;
@@ -846,6 +858,7 @@ void fill_pass_args(ewfa::AlignArgs& a, const Pass& p, ewfa_ctx* c) {
     a.bt_slot_words = 2u * (uint64_t)ewfa::bt_chunks((uint32_t)p.dcap);
     a.off16 = p.off16;
     a.band_cap = p.band_cap;
+    a.defer_len = p.defer_len;
     a.gslot = p.gslot ? sx.gslot + p.gslot_off / 8 : nullptr;
     a.gslot_words = p.gslot ? p.gslot_bytes / 8 : 0;
 }

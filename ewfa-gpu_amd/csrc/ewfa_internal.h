@@ -103,6 +103,7 @@ struct AlignArgs {
     // 64-bit addresses.
     uint64_t* gslot;
     uint64_t gslot_words;
+    uint32_t defer_len;  // four-chunk register pass: longer pairs are deferred untried (0: none)
     uint32_t below;  // bound search: lists of this many pairs or more have another (0: none have)
 };
 

@@ -1255,6 +1255,8 @@ template <int NC>
 __device__ __forceinline__ bool align_pair_reg(const AlignArgs& a, uint32_t pidx, const PairPrefetch& f, uint64_t* slot, int lane) {
     if constexpr (NC == 1) return align_pair_band(a, pidx, f, slot, lane);
     const ewfa_pair_t& pr = f.pr;
+    // (its status says so since an earlier pass)
+    if (NC == 4 && a.defer_len && max(pr.plen, pr.tlen) > a.defer_len) return true;
     const int plen = (int)pr.plen, tlen = (int)pr.tlen;
     const int sw = a.seq_words;
     const int nwp = (plen + 31) >> 5, nwt = (tlen + 31) >> 5;

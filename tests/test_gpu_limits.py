@@ -150,3 +150,35 @@ def test_short_pairs_beside_one_beyond_lds_are_not_served_in_turn():
                 times.append(time.perf_counter() - t0)
         took.append(sorted(times)[3])
     assert took[1] < 1.6 * took[0], took
+
+
+def median_us(call, reps=7):
+    call()
+    times = []
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        call()
+        times.append(time.perf_counter() - t0)
+    return sorted(times)[reps // 2] * 1e6
+
+
+def test_a_list_beyond_its_budget_goes_on_to_the_next(tmp_path):
+    """2,210 pairs of 4,760 bp at 12.6%: 540 to 600 edits, beyond their bucket's
+    512 levels and within the 1,024 that follow, which hold them at twice the
+    occupancy of a budget of the whole length."""
+    print("case 2210 pairs of 4760 bp, all deferred", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=0, seed=5, len=4760, err=0.126), 2210)
+    few = ewfa.Workload(ewfa.synth_spec(kind=0, seed=5, len=4760, err=0.126), 24)
+    ok, d, sl, st = orc.batch_workload(few)
+    case = OnDevice(w.words, w.pairs[:w.n].copy(), w.cigar_bytes, w.max_len)
+    out, took = [], []
+    for path in (policy_file(tmp_path, "enough", "4000000000 2 1024 0 1\n"), None):
+        with ewfa.Context(policy_path=path) as ctx:
+            case.dc.fill_zero()
+            took.append(median_us(lambda: case.align(ctx)))
+        res, cig = case.dr.download(ewfa.RESULT_DTYPE, case.n), case.dc.download(np.int8)
+        check(res[:24], case.pairs[:24], cig, d, st, path)
+        assert (res["status"] == ewfa.PAIR_OK).all() and res["distance"].max() > 512
+        out.append((res, cig))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert took[1] < 2.2 * took[0], took
