@@ -1551,8 +1551,14 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
     if (!d_words || !d_pairs || !d_results || !d_cigars || !scratch) return fail(EWFA_ERR_ARG, "null buffer");
     if (n > 0xFFFFFFF0u) return fail(EWFA_ERR_RANGE, "too many pairs in one call");
     CHK(set_device(c));
+    // per-pair buffers first, then one region for the passes' slots
+    const auto r256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t ops_bytes = op_scratch_bytes(n, max_len);
+    const size_t list = r256(n * 4);
+    size_t fixed = r256(ops_bytes) + r256(CTRL_BP * 4) + 4 * list;
     Plan pl;
     CHK(plan_persistent(c, max_len, (uint32_t)n, pl));
+    if (pl.nb > 1) fixed += r256((size_t)pl.nb * n * 4);
     // one stream: every pass's slots share the region.  The static scratch
     // has no room for slots in HBM: the deferral chain stops before the first
     // such pass (its pairs come back TOO_DISTANT), and sequences too long for
@@ -1569,11 +1575,6 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
     pl.fanout = 1;
     for (int b = 0; b < pl.nb; ++b) pl.pass[b].bp_grid = pl.free_pass[b].grid = 0;  // nor for bit-parallel slots
     assign_slots(pl);
-    // per-pair buffers first, then one region for the passes' slots
-    const auto r256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t ops_bytes = op_scratch_bytes(n, max_len);
-    const size_t list = r256(n * 4);
-    const size_t fixed = r256(ops_bytes) + r256(CTRL_BP * 4) + 4 * list + (pl.nb > 1 ? r256((size_t)pl.nb * n * 4) : 0);
     if (fixed > bytes)
         return fail(EWFA_ERR_RANGE, "%zu pairs of up to %u bases need %zu bytes of scratch before any pass; the "
                     "allocation-free call holds %zu", n, max_len, fixed, bytes);
@@ -1605,6 +1606,14 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
         if (p.grid > most) p.grid = (uint32_t)most;
         return EWFA_OK;
     };
+    // the chain's register pass where its run rows have room for a wave per SIMD:
+    // the passes after it do without
+    Chain& ch = pl.chain;
+    if (ch.np && ch.pass[0].reg &&
+        x.region / runs_slot_of(ch.pass[0]) < std::min<size_t>(ch.pass[0].grid, 4u * (size_t)c->num_cus)) {
+        std::copy(ch.pass + 1, ch.pass + ch.np, ch.pass);
+        --ch.np;
+    }
     for (int k = 0; k < pl.nb; ++k) CHK(fit(pl.pass[k]));
     for (int k = 0; k < pl.chain.np; ++k) CHK(fit(pl.chain.pass[k]));
     hipStream_t s = c->stream;

@@ -182,3 +182,34 @@ def test_a_list_beyond_its_budget_goes_on_to_the_next(tmp_path):
         out.append((res, cig))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert took[1] < 2.2 * took[0], took
+
+
+def test_the_allocation_free_call_takes_what_its_per_pair_buffers_hold():
+    """Short pairs fill its scratch to the last pair: no pass refuses what is
+    left of it."""
+    print("case allocation-free, scratch full of 150 bp pairs", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=0, seed=5, len=150, err=0.02), 1000)
+    ok, d, sl, st = orc.batch_workload(w)
+    n = 1_400_000
+    pairs = np.resize(w.pairs[:w.n], n)
+    pairs["cigar_off"] = np.arange(n, dtype=np.uint64) * 64
+    pairs["cigar_cap"] = 64
+    case = OnDevice(w.words, pairs, 64 * n, w.max_len)
+
+    def call(m):
+        ctx.align_device_noalloc(case.dw.ptr, case.dp.ptr, m, case.max_len, case.dr.ptr, case.dc.ptr, None)
+
+    with ewfa.Context() as ctx:
+        lo, hi = 1_000_000, n
+        while lo < hi:
+            m = (lo + hi + 1) // 2
+            try:
+                call(m)
+                lo = m
+            except ewfa.EwfaError as e:
+                hi, why = m - 1, str(e)
+        call(lo)
+        res, cig = case.dr.download(ewfa.RESULT_DTYPE, n), case.dc.download(np.int8)
+        assert "before any pass" in why, (lo, why)
+        check(res[lo - 1000:lo], pairs[lo - 1000:lo], cig, [d[i % 1000] for i in range(lo - 1000, lo)],
+              [st[i % 1000] for i in range(lo - 1000, lo)], lo)
