@@ -627,7 +627,8 @@ uint32_t plan_reg_len(const Plan& pl) {
 // wave) a CU holds 28 of its waves.
 constexpr uint32_t BANDED_ONE_LEN = 3000;
 
-int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
+// slots: the bytes there are for the passes' slots.
+int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl, size_t slots = SIZE_MAX) {
     pl = Plan{};
     const bool capped = c->opts.max_distance > 0 && c->opts.max_distance <= 64;
     if (!capped && n <= (uint32_t)c->num_cus && max_len > c->policy.buckets.front().len_hi) {
@@ -635,14 +636,15 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
         // so all go through that pair's pass, without bucketing and the fork
         // over streams (60 pairs of 100..2,000 bp: 175 -> 130 us).  Not through one
         // with its slots in HBM, of which there may be a single one (60 pairs of
-        // 10 kbp beside one of 400 kbp: 15.2 ms so, 6.6 ms by their buckets)
+        // 10 kbp beside one of 400 kbp: 15.2 ms so, 6.6 ms by their buckets), nor
+        // where the slots' bytes leave it fewer blocks than pairs
         pl.blen[0] = max_len;
         ewfa::BucketPolicy bp = c->policy.bucket_for(max_len);
         // nothing to gain from 63 levels alone here, and a second pass to lose
         // where a pair has more (7 pairs of 135..675 bp at 4..15%: 153 -> 105 us)
         if (c->builtin_policy && bp.dcap == 63 && max_len > 420) bp.dcap = REG4_LEVELS;
         CHK(pass_from_bucket(c, bp, max_len, n, pl.pass[0]));
-        if (!pl.pass[0].gslot) {
+        if (!pl.pass[0].gslot && slot_bytes(pl.pass[0]) * pl.pass[0].grid <= slots) {
             pl.nb = 1;
             plan_chain(c, max_len, plan_reach(pl, max_len), plan_reg_len(pl), n, pl.chain);
             assign_slots(pl);
@@ -1557,7 +1559,7 @@ int align_device_in(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t* d
     const size_t list = r256(n * 4);
     size_t fixed = r256(ops_bytes) + r256(CTRL_BP * 4) + 4 * list;
     Plan pl;
-    CHK(plan_persistent(c, max_len, (uint32_t)n, pl));
+    CHK(plan_persistent(c, max_len, (uint32_t)n, pl, bytes > fixed ? bytes - fixed : 0));
     if (pl.nb > 1) fixed += r256((size_t)pl.nb * n * 4);
     // one stream: every pass's slots share the region.  The static scratch
     // has no room for slots in HBM: the deferral chain stops before the first

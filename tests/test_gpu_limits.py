@@ -213,3 +213,19 @@ def test_the_allocation_free_call_takes_what_its_per_pair_buffers_hold():
         assert "before any pass" in why, (lo, why)
         check(res[lo - 1000:lo], pairs[lo - 1000:lo], cig, [d[i % 1000] for i in range(lo - 1000, lo)],
               [st[i % 1000] for i in range(lo - 1000, lo)], lo)
+
+
+def test_the_allocation_free_call_over_few_long_pairs():
+    """200 pairs, whose longest have room for a few blocks only, take no longer
+    than 300 of the same lengths."""
+    took = []
+    for n in (200, 300):
+        print(f"case allocation-free, {n} pairs of 1..12 kbp", flush=True)
+        w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=5, len_lo=1000, len_hi=12000, err_lo=0.025, err_hi=0.05), n)
+        ok, d, sl, st = orc.batch_workload(w)
+        case = OnDevice(w.words, w.pairs[:w.n].copy(), w.cigar_bytes, w.max_len)
+        with ewfa.Context() as ctx:
+            took.append(median_us(lambda: ctx.align_device_noalloc(case.dw.ptr, case.dp.ptr, n, case.max_len,
+                                                                   case.dr.ptr, case.dc.ptr, None)))
+        case.check(d, st, "allocation-free")
+    assert took[0] < 1.2 * took[1], took
