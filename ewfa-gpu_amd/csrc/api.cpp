@@ -56,6 +56,7 @@ struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
     int reserve(ewfa_ctx* c, size_t n);
+    void retire(ewfa_ctx* c);
     void release() {
         if (p) (void)hipFree(p);
         p = nullptr;
@@ -183,6 +184,16 @@ void release_retired(ewfa_ctx* c) {
     c->retired_bytes = 0;
 }
 
+// Work already queued may still use it: freed by release_retired.
+void DevBuf::retire(ewfa_ctx* c) {
+    if (!p) return;
+    c->retired.push_back(p);
+    c->retired_bytes += bytes;
+    ++c->buffer_gen;
+    p = nullptr;
+    bytes = 0;
+}
+
 int DevBuf::reserve(ewfa_ctx* c, size_t n) {
     if (n <= bytes) return EWFA_OK;
     size_t want = p ? std::max(n, bytes + bytes / 2) : n;
@@ -193,16 +204,15 @@ int DevBuf::reserve(ewfa_ctx* c, size_t n) {
         want = n;
         e = hipMalloc(&q, want);
     }
-    if (e != hipSuccess && !c->retired.empty()) {
+    if (e != hipSuccess && (!c->retired.empty() || (this != &c->bt && c->bt.p))) {
         (void)hipGetLastError();
+        // the backtrace region too, which a plan reserves last
+        if (this != &c->bt) c->bt.retire(c);
         release_retired(c);
         e = hipMalloc(&q, want);
     }
     if (e != hipSuccess) return fail(EWFA_ERR_NOMEM, "hipMalloc(%zu): %s", want, hipGetErrorString(e));
-    if (p) {
-        c->retired.push_back(p);
-        c->retired_bytes += bytes;
-    }
+    retire(c);
     p = q;
     bytes = want;
     ++c->buffer_gen;
@@ -778,19 +788,6 @@ int reserve_bt(ewfa_ctx* c, const Pass& p) {
 }
 
 int reserve_plan(ewfa_ctx* c, Plan& pl, size_t n) {
-    // where the device has no room for all slots, fewer for the bit-parallel
-    // passes (every later plan of the context then asks for fewer)
-    for (;;) {
-        const int rc = c->bt.reserve(c, pl.bt_bytes);
-        if (rc == EWFA_OK) break;
-        if (!pl.bp) return rc;
-        (void)hipGetLastError();
-        g_err.clear();
-        c->bp_budget = std::min(c->bp_budget, BP_BUDGET) / 4;
-        ++c->policy_gen;
-        for (int b = 0; b < pl.nb; ++b) choose_bp(c, pl.pass[b], pl.blen[b], (uint32_t)n);
-        assign_slots(pl);
-    }
     CHK(c->runs.reserve(c, pl.runs_bytes));
     CHK(c->gslot.reserve(c, pl.gslot_bytes));
     if (pl.nb > 1) CHK(c->buckets.reserve(c, (size_t)pl.nb * std::max<size_t>(n, 1) * 4));
@@ -803,7 +800,29 @@ int reserve_plan(ewfa_ctx* c, Plan& pl, size_t n) {
     bool narrow = false;
     for (int b = 0; b < pl.nb; ++b) narrow = narrow || pl.pass[b].band_cap > 0;
     if (narrow) CHK(c->order.reserve(c, (size_t)std::max(pl.nb, 1) * std::max<size_t>(n, 1) * 4));
-    return EWFA_OK;
+    // the backtrace region last.  Where the device has no room for all slots, or
+    // those of the bit-parallel passes would take more than half of what is free,
+    // fewer of these (every later plan of the context then asks for fewer)
+    const auto fewer = [&]() {
+        c->bp_budget = std::min(c->bp_budget, BP_BUDGET) / 2;
+        ++c->policy_gen;
+        for (int b = 0; b < pl.nb; ++b) choose_bp(c, pl.pass[b], pl.blen[b], (uint32_t)n);
+        assign_slots(pl);
+    };
+    size_t room = 0, total = 0;
+    if (pl.bp && pl.bt_bytes > c->bt.bytes && hipMemGetInfo(&room, &total) == hipSuccess) {
+        Plan rest = pl;
+        for (int b = 0; b < pl.nb; ++b) rest.pass[b].bp_grid = 0;
+        assign_slots(rest);
+        while (pl.bp && pl.bt_bytes > std::max({c->bt.bytes, rest.bt_bytes, room / 2})) fewer();
+    }
+    for (;;) {
+        const int rc = c->bt.reserve(c, pl.bt_bytes);
+        if (rc == EWFA_OK || !pl.bp) return rc;
+        (void)hipGetLastError();
+        g_err.clear();
+        fewer();
+    }
 }
 
 int launch_pass(const ewfa::AlignArgs& a, const Pass& p, hipStream_t s) {

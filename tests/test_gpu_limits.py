@@ -229,3 +229,33 @@ def test_the_allocation_free_call_over_few_long_pairs():
                                                                    case.dr.ptr, case.dc.ptr, None)))
         case.check(d, st, "allocation-free")
     assert took[0] < 1.2 * took[1], took
+
+
+def test_bit_parallel_slots_leave_others_room():
+    """With 44 GiB of the device free, a call whose bit-parallel slots could
+    take 40 (its wavefront's own take 21) holds about half of them."""
+    gib = 44
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    fp, ft, fd, fst = fill_pairs(5000)
+    rng = np.random.default_rng(gib)
+    P = [rng.choice(BASES, n).tobytes() for n in (24_000, 49_000)]
+    T = [bytes(BASES[(np.searchsorted(BASES, np.frombuffer(p, np.uint8)) + (np.arange(len(p)) % 25 == 7)) % 4]) for p in P]
+    d, st = oracle_streams(P, T)
+    case = OnDevice(*ewfa.from_sequences(P + fp, T + ft))
+    ewfa.synchronize()
+    print(f"case {gib} GiB free", flush=True)
+    held = ewfa.DeviceBuffer(free_bytes() - (gib << 30))
+    try:
+        with ewfa.Context() as ctx:
+            for _ in range(2):
+                case.align(ctx).check(list(d) + fd, list(st) + fst, gib)
+            assert ctx.memory_bytes() < 0.6 * (gib << 30)
+            assert free_bytes() > 0.35 * (gib << 30)
+    finally:
+        held.free()
