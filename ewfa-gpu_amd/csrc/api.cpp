@@ -245,7 +245,7 @@ struct Pass {
     int seq_words;
     int reg;  // register-wavefront chunks (0: offsets staged in LDS)
     int off16;  // 16-bit LDS offsets (block kernel, backtrace in HBM, no bounds)
-    uint32_t defer_len;  // register pass: longer pairs are deferred untried (0: none)
+    uint32_t defer_len;  // chain: longer pairs are deferred untried (0: none)
     int band_cap;  // bounded pass with narrow slots: the largest bound they hold (0: none)
     size_t lds;
     uint32_t grid;
@@ -563,6 +563,8 @@ void assign_slots(Plan& pl) {
 
 int next_pass(ewfa_ctx* c, uint32_t max_len, int prev_dcap, uint32_t items, Pass& p);
 
+// Edits that the widest bit-parallel band holds on every target diagonal.
+constexpr int BP_REACH = 64 * (ewfa::BP_WIDEST - 2) / 2;
 // Levels of the four-chunk register pass, and the LDS a wave of it may take ahead
 // of the deferral chain (four waves a SIMD).
 constexpr int REG4_LEVELS = 127;
@@ -570,17 +572,44 @@ constexpr size_t REG4_CHAIN_LDS = 10240;
 // The longest pairs of the built-in policy's register passes.
 constexpr uint32_t REG_LEN = 1200;
 
-// reg_len: the longest pairs that passes of fewer levels than it defer (0: none).
-void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t reg_len, uint32_t n, Chain& ch) {
+// Distances that every pair of a pass within them ends at: its budget, or what
+// its narrow slots or the bit-parallel band ahead of it hold.
+int reach_of(const Pass& p) {
+    int reach = p.dcap;
+    if (p.band_cap > 0) reach = std::min(reach, p.band_cap);
+    if (p.bp_grid > 0) reach = std::min(reach, BP_REACH);
+    return reach;
+}
+
+// The longest pairs that a pass within `levels` may defer at fewer.
+uint32_t deferred_len(const Plan& pl, int levels) {
+    uint32_t len = 0;
+    for (int b = 0; b < pl.nb; ++b)
+        if (reach_of(pl.pass[b]) < levels) len = std::max(len, pl.blen[b]);
+    return len;
+}
+
+void plan_chain(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl) {
+    Chain& ch = pl.chain;
     ch = Chain{};
-    int dcap = dcap_min;
-    // what a banded pass defers (63 levels) mostly ends within 127, which a wave
+    // the levels within which every pair ends in its bucket's pass.  What narrow
+    // slots and bit-parallel bands defer needs a pass after theirs even where the
+    // budget exceeds any distance: the chain then ends with one of max_len + 1 levels.
+    int dcap = pl.pass[0].dcap;
+    for (int b = 0; b < pl.nb; ++b) {
+        const Pass& p = pl.pass[b];
+        dcap = std::min(dcap, p.dcap);
+        if (reach_of(p) < p.dcap) dcap = (int)std::min((uint32_t)dcap, max_len);
+    }
+    // Pairs of a bucket whose pass held as many levels as a chain's go on untried
+    // (defer_len).
+    // What a banded pass defers (63 levels) mostly ends within 127, which a wave
     // holds in registers: 100,000 pairs of 521 bp at 14.5% edits, all deferred,
-    // took 10,154 us through the block passes below alone, 1,570 so.  Pairs that
-    // passes of as many levels deferred go on untried, and the passes after this
-    // one are those there would be without it: 2,210 pairs of 4.8 kbp at 12.6%
-    // (600 edits, beyond their bucket's 512) took 7.3 ms where 127, 508 and 4,761
-    // levels followed each other in place of 256 and 1,024 (2.5 ms).
+    // took 10,154 us through the block passes below alone, 1,570 so.  The passes
+    // after this one are those there would be without it: 2,210 pairs of 4.8 kbp at
+    // 12.6% (600 edits, beyond their bucket's 512) took 7.3 ms where 127, 508 and
+    // 4,761 levels followed each other, 2.2 with 127, 256 and 1,024.
+    const uint32_t reg_len = deferred_len(pl, REG4_LEVELS);
     if (reg_len > 0) {
         const int ow = overlapped_words_for(max_len);
         if (ewfa::lds_bytes_reg(ow, REG4_LEVELS, 4) <= REG4_CHAIN_LDS) {
@@ -604,33 +633,11 @@ void plan_chain(ewfa_ctx* c, uint32_t max_len, int dcap_min, uint32_t reg_len, u
             const size_t most = std::max<size_t>(CHAIN_BT_BUDGET / slot, 1);
             if (p.grid > most) p.grid = (uint32_t)most;
         }
+        p.defer_len = deferred_len(pl, p.dcap);
         ch.pass[ch.np++] = p;
         dcap = p.dcap;
     }
     g_err.clear();
-}
-
-// The levels within which every pair ends in its bucket's pass: the least of
-// the passes' budgets.  A narrow slot and a bit-parallel band hold less than the
-// pass's budget (at 9.5 kbp 9,600 and 8,129 of 9,900 levels), and what they defer
-// needs a pass after them even where the budget exceeds any distance: the chain
-// then ends with one of max_len + 1 levels.
-int plan_reach(const Plan& pl, uint32_t max_len) {
-    int reach = pl.pass[0].dcap;
-    for (int b = 0; b < pl.nb; ++b) {
-        const Pass& p = pl.pass[b];
-        reach = std::min(reach, p.dcap);
-        if (p.band_cap > 0 || p.bp_grid > 0) reach = (int)std::min((uint32_t)reach, max_len);
-    }
-    return reach;
-}
-
-// The longest pairs of the passes below the four-chunk register pass's levels.
-uint32_t plan_reg_len(const Plan& pl) {
-    uint32_t len = 0;
-    for (int b = 0; b < pl.nb; ++b)
-        if (pl.pass[b].dcap < REG4_LEVELS) len = std::max(len, pl.blen[b]);
-    return len;
 }
 
 // Longest pairs of a banded pass over a whole list: up to here (5.7 KB of LDS a
@@ -656,7 +663,7 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl, size_t 
         CHK(pass_from_bucket(c, bp, max_len, n, pl.pass[0]));
         if (!pl.pass[0].gslot && slot_bytes(pl.pass[0]) * pl.pass[0].grid <= slots) {
             pl.nb = 1;
-            plan_chain(c, max_len, plan_reach(pl, max_len), plan_reg_len(pl), n, pl.chain);
+            plan_chain(c, max_len, n, pl);
             assign_slots(pl);
             return EWFA_OK;
         }
@@ -690,7 +697,7 @@ int plan_persistent(ewfa_ctx* c, uint32_t max_len, uint32_t n, Plan& pl, size_t 
         if (max_len <= b.len_hi) break;
     }
     pl.table.nb = pl.nb;
-    plan_chain(c, max_len, plan_reach(pl, max_len), plan_reg_len(pl), n, pl.chain);
+    plan_chain(c, max_len, n, pl);
     pl.fanout = std::min(pl.nb, c->fanout);
     assign_slots(pl);
     return EWFA_OK;

@@ -103,7 +103,7 @@ struct AlignArgs {
     // 64-bit addresses.
     uint64_t* gslot;
     uint64_t gslot_words;
-    uint32_t defer_len;  // four-chunk register pass: longer pairs are deferred untried (0: none)
+    uint32_t defer_len;  // block and four-chunk register passes: longer pairs are deferred untried (0: none)
     uint32_t below;  // bound search: lists of this many pairs or more have another (0: none have)
 };
 
@@ -175,8 +175,9 @@ inline int reg_chunks_for(int dcap) {
 // Classes of pairs by the words of 32 diagonals their band starts with, widest
 // first.
 constexpr int BP_CLASSES = 10;
+constexpr int BP_WIDEST = 256;
 __host__ __device__ inline int bp_words(int c) {
-    return c == 0 ? 256 : c == 1 ? 192 : c == 2 ? 128 : c == 3 ? 96 : c == 4 ? 64 : c == 5 ? 48 : c == 6 ? 32 : c == 7 ? 24 : c == 8 ? 16 : 8;
+    return c == 0 ? BP_WIDEST : c == 1 ? 192 : c == 2 ? 128 : c == 3 ? 96 : c == 4 ? 64 : c == 5 ? 48 : c == 6 ? 32 : c == 7 ? 24 : c == 8 ? 16 : 8;
 }
 // Lanes per pair: 64 for 129..256 words, 32 for 65..128, 16 for 33..64, 8 below,
 // four words a lane at most; `spread` doubles them (for short lists, where more

@@ -1410,7 +1410,12 @@ __global__ __launch_bounds__(64 * G) void align_kernel(AlignArgs a, int persiste
     };
     const auto run = [&](uint32_t base, uint32_t end) {
         for (uint32_t it = base; it < end; ++it) {
-            align_pair<G, BT_LDS, BOUNDED, Off, GSLOT>(a, a.list ? a.list[it] : it, slot, btg, tid);
+            const uint32_t pidx = a.list ? a.list[it] : it;
+            if (a.defer_len && (a.pairs[pidx].plen > a.defer_len || a.pairs[pidx].tlen > a.defer_len)) {
+                if (tid == 0) a.defer_list[atomicAdd(a.defer_count, 1u)] = pidx;
+                continue;
+            }
+            align_pair<G, BT_LDS, BOUNDED, Off, GSLOT>(a, pidx, slot, btg, tid);
             group_sync<G>();  // the slot is reused by the next pair
         }
     };

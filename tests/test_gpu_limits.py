@@ -7,7 +7,7 @@ import pytest
 
 import ewfa
 import oracle_py as orc
-from test_gpu_bitpar import POLICY
+from test_gpu_bitpar import POLICY, mutate
 from test_gpu_bound import check, policy_file
 from test_gpu_stress import oracle_streams
 
@@ -259,3 +259,29 @@ def test_bit_parallel_slots_leave_others_room():
             assert free_bytes() > 0.35 * (gib << 30)
     finally:
         held.free()
+
+
+@pytest.mark.parametrize("policy", [None, "500 1 200 1 2\n1500 1 40 1 2\n4000000000 4 300 0 1\n"])
+def test_deferred_pairs_of_every_bucket(tmp_path, policy):
+    """A list in which every bucket defers pairs: each goes untried through the
+    deferral passes that hold no more than its bucket's did, and ends in a
+    later one.  Also where a shorter bucket has the larger budget."""
+    print("case deferred from every bucket", flush=True)
+    rng = np.random.default_rng(8)
+    P, T = [], []
+    for n, rate in ((250, .40), (480, .30), (650, .25), (690, .12), (1100, .14), (1400, .08), (2400, .40), (3000, .14),
+                    (4900, .16), (9000, .15), (10400, .13)):
+        for _ in range(4):
+            p = rng.choice(BASES, n).tobytes()
+            P.append(p)
+            T.append(mutate(rng, p, rate))
+    d, st = oracle_streams(P, T)
+    fp, ft, fd, fst = fill_pairs(600)
+    order = rng.permutation(len(P) + 600)
+    P, T, d, st = P + fp, T + ft, list(d) + fd, list(st) + fst
+    P, T, d, st = ([x[i] for i in order] for x in (P, T, d, st))
+    case = OnDevice(*ewfa.from_sequences(P, T))
+    with ewfa.Context(policy_path=policy_file(tmp_path, "some", policy) if policy else None) as ctx:
+        for _ in range(2):
+            case.dc.fill_zero()
+            case.align(ctx).check(d, st, policy)
