@@ -76,6 +76,7 @@ enum : int {
     CTRL_BQUEUE = 8,    // queue heads of the bucket passes (MAX_BUCKETS)
     CTRL_BCOUNT = 16,   // pairs per bucket (MAX_BUCKETS)
     CTRL_BOUNDQ = 24,   // work counters of the bucket passes' distance bounds (MAX_BUCKETS)
+    CTRL_EMIT = 32,     // a bucket's counts by wave and by lane emit (2 x MAX_BUCKETS)
     CTRL_XQ = 64,       // per-XCD work counters of the bucket passes (MAX_BUCKETS x XCDS, strided)
     // per bucket: the bit-parallel sort's bins and cursors, the classes' places,
     // the count of pairs left to the wavefront and the pass's work counter
@@ -361,6 +362,10 @@ constexpr uint64_t BP_PROBE_MIN = 60000000000ull;
 // SIMDs with less than two waves (15,001 pairs of 3..7 kbp: 4.0 -> 3.5 ms; 500,000
 // pairs of up to 10 kbp 17.5 -> 20.8 ms, so large lists keep the narrow groups).
 constexpr uint32_t BP_SPREAD_BELOW = 32768;
+
+// Pairs per CU up to which a list's streams are written by a wave a pair whatever its
+// edits (8,000 pairs of 1.5 kbp at 10% 509 us by lanes and 505 by waves, 11,000 616 and 675).
+constexpr uint32_t EMIT_WAVE_PER_CU = 40;
 
 // Pairs per CU up to which a list counts as few.
 constexpr uint32_t FEW_PER_CU = 4;
@@ -926,23 +931,35 @@ int emit_list(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max
     return EWFA_OK;
 }
 
+// counts: two words for the list's count as the wave and as the lane emit's (null:
+// lists above EMIT_WAVE_PER_CU pairs per CU go by lanes).
 int emit(ewfa_ctx* c, const ewfa::EmitArgs& e, uint32_t items, uint32_t max_len, bool staged, hipStream_t s,
-         bool deeper = false) {
+         uint32_t* counts = nullptr, bool deeper = false) {
     // a wave a pair while its lists are short: a lane's steps wait for memory,
     // which takes many more pairs to hide (3,000 pairs of 1..10 kbp at 1..5% edits
-    // 1,098 -> 815 us; but 86,000 of 2.3 kbp at 2.1% 1,498 by lanes and 1,776 by
-    // waves).  Both sequences in LDS leave fewer waves the longer they are: above
-    // 6 KB lanes win earlier (21,442 pairs of 8.7 kbp at 3.9% 3,641 and 3,879), above
-    // 12 KB soon (1,500 pairs of 10..20 kbp 1,926 -> 1,628, none of it left at 3,000).  Beside a bucket whose narrow slots just fill the LDS (deeper),
-    // its blocks would keep one of those off every CU.
+    // 1,098 -> 815 us).  Longer lists as their edits say (emit_pick_kernel).
+    // Both sequences in LDS leave fewer waves the longer they are: above 6 KB lanes
+    // win earlier (21,442 pairs of 8.7 kbp at 3.9% 3,641 and 3,879), above 12 KB soon
+    // (1,500 pairs of 10..20 kbp 1,926 -> 1,628, none of it left at 3,000).  Beside a
+    // bucket whose narrow slots just fill the LDS (deeper), its blocks would keep one
+    // of those off every CU.
     const size_t lds = (size_t)2 * overlapped_words_for(max_len) * 8;
+    const uint32_t cus = (uint32_t)c->num_cus;
     const uint32_t per_cu = deeper ? FEW_PER_CU : lds <= 6144 ? 128u : lds <= 12288 ? 60u : 8u;
-    if (staged && items <= (uint32_t)c->num_cus * per_cu) return emit_list(c, e, items, max_len, s);
+    if (staged && items <= cus * std::min(per_cu, EMIT_WAVE_PER_CU)) return emit_list(c, e, items, max_len, s);
+    ewfa::EmitArgs lanes = e;
+    if (staged && counts && items <= cus * per_cu) {
+        HIPCHK(ewfa::launch_emit_pick(e, (lds <= 6144 ? 2.5f : 1.6f) * (float)cus, counts, s));
+        ewfa::EmitArgs waves = e;
+        waves.count_ptr = counts;
+        lanes.count_ptr = counts + 1;
+        CHK(emit_list(c, waves, items, max_len, s));
+    }
     const int sw = seq_words_for(max_len);
     if (staged && sw <= ewfa::EMIT_LDS_MAX_SW)
-        HIPCHK(ewfa::launch_emit_lds(e, items, sw, s));
+        HIPCHK(ewfa::launch_emit_lds(lanes, items, sw, s));
     else
-        HIPCHK(ewfa::launch_emit(e, items, emit_per_wave(c, items), s));
+        HIPCHK(ewfa::launch_emit(lanes, items, emit_per_wave(c, items), s));
     return EWFA_OK;
 }
 
@@ -1201,7 +1218,8 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 e.list = emit_items;
                 e.count = n;
                 e.count_ptr = emit_count;
-                CHK(emit(c, e, n, pl.blen[b], true, q, b < pl.nb - 1 && pl.pass[pl.nb - 1].band_cap > 0));
+                CHK(emit(c, e, n, pl.blen[b], true, q, ctrl + CTRL_EMIT + 2 * b,
+                         b < pl.nb - 1 && pl.pass[pl.nb - 1].band_cap > 0));
             }
         }
         for (int i = 1; i < F; ++i) {

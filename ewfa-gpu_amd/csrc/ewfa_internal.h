@@ -319,6 +319,9 @@ constexpr int EMIT_PER_WAVE = 16;
 // copies of sw words (2 * sw * 8 bytes per block, at most EMIT_WAVE_MAX_LDS);
 // at most max_grid blocks, grid-stride.
 hipError_t launch_emit_wave(const EmitArgs& a, uint32_t grid_items, int sw, uint32_t max_grid, hipStream_t stream);
+// counts[0], counts[1]: a list's count as the wave and as the lane emit's, one of them
+// 0: the waves' while a sample's edits a base times the count stay within `most`.
+hipError_t launch_emit_pick(const EmitArgs& a, float most, uint32_t* counts, hipStream_t stream);
 constexpr size_t EMIT_WAVE_MAX_LDS = 65536;
 // Marks the pairs of list[0..*count_ptr) EWFA_PAIR_TOO_DISTANT.
 hipError_t launch_mark_too_distant(const uint32_t* list, const uint32_t* count_ptr, ewfa_result_t* results,

@@ -1907,6 +1907,42 @@ __device__ __forceinline__ int wave_lcp(const uint64_t* P, const uint64_t* T, in
     return rem > 0 ? rem : 0;
 }
 
+// Which of the two writes a list's streams, from 256 of its pairs.  A
+// wave's time goes with its ops, a lane's mostly with the longest path: they meet
+// where the pairs per CU times the edits a base come to about 2.5 (1.5 to 5 kbp:
+// 15,000 pairs at 4.5%, 22,000 at 3%, 32,000 at 2%; 32,000 of 5 kbp take 1,139 us by
+// lanes and 853 by waves at 1%, 3,816 and 4,540 at 6%), above 6 KB of LDS a pair 1.6.
+__global__ __launch_bounds__(256) void emit_pick_kernel(EmitArgs a, float most, uint32_t* counts) {
+    __shared__ float part[4][2];
+    const uint32_t n = a.count_ptr ? *a.count_ptr : a.count;
+    float edits = 0.f, bases = 0.f;
+    if (n) {
+        const uint32_t at = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) >> 9);
+        const uint32_t i = a.list ? a.list[at] : at;
+        const ewfa_result_t r = a.results[i];
+        const uint32_t tlen = a.pairs[i].tlen;
+        if (r.status == EWFA_PAIR_OK || r.status == EWFA_PAIR_CAPPED) {
+            edits = (float)r.distance;
+            bases = (float)tlen;
+        }
+    }
+    for (int d = 32; d; d >>= 1) {
+        edits += __shfl_xor(edits, d);
+        bases += __shfl_xor(bases, d);
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        part[threadIdx.x >> 6][0] = edits;
+        part[threadIdx.x >> 6][1] = bases;
+    }
+    __syncthreads();
+    if (threadIdx.x) return;
+    edits = part[0][0] + part[1][0] + part[2][0] + part[3][0];
+    bases = part[0][1] + part[1][1] + part[2][1] + part[3][1];
+    const bool waves = (float)n * edits <= most * bases;
+    counts[0] = waves ? n : 0u;
+    counts[1] = waves ? 0u : n;
+}
+
 // Emit with one wave per pair: the wave stages its pair's sequences
 // (little-endian overlapped copies, sw words each) and finds every match run
 // with wave_lcp.  A run depends on the one before, so the walk is a chain; what
@@ -2350,6 +2386,11 @@ hipError_t launch_emit_wave(const EmitArgs& a, uint32_t grid_items, int sw, uint
     const size_t lds = (size_t)2 * (size_t)sw * 8;
     const uint32_t blocks = grid_items < max_grid ? grid_items : max_grid;
     hipLaunchKernelGGL(emit_wave_kernel, dim3(blocks), dim3(64), lds, stream, a, sw);
+    return hipGetLastError();
+}
+
+hipError_t launch_emit_pick(const EmitArgs& a, float most, uint32_t* counts, hipStream_t stream) {
+    hipLaunchKernelGGL(emit_pick_kernel, dim3(1), dim3(256), 0, stream, a, most, counts);
     return hipGetLastError();
 }
 

@@ -285,3 +285,47 @@ def test_deferred_pairs_of_every_bucket(tmp_path, policy):
         for _ in range(2):
             case.dc.fill_zero()
             case.align(ctx).check(d, st, policy)
+
+
+@pytest.mark.parametrize("err", [0.01, 0.12])
+@pytest.mark.parametrize("count", [10_240, 10_241, 32_768, 32_769])
+def test_streams_by_wave_and_by_lane(tmp_path, count, err):
+    """Lists on either side of 40 and 128 pairs per CU: a wave a pair, as a
+    sample of the results says, and a lane a pair."""
+    print(f"case streams {count} pairs {err}", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=2, seed=count, len_lo=100, len_hi=200, err_lo=err / 2, err_hi=err), count)
+    ok, d, sl, st = orc.batch_workload(w)
+    case = OnDevice(w.words, w.pairs[:w.n].copy(), w.cigar_bytes, w.max_len)
+    with ewfa.Context(policy_path=policy_file(tmp_path, "block", "4000000000 2 256 0 1\n")) as ctx:
+        for _ in range(2):
+            case.dc.fill_zero()
+            case.align(ctx).check(d, st, (count, err))
+
+
+class EmitArgs(ctypes.Structure):
+    _fields_ = [(k, ctypes.c_void_p) for k in ("words", "pairs", "results", "ops")] + [
+        ("ops_stride", ctypes.c_uint32), ("cigars", ctypes.c_void_p), ("list", ctypes.c_void_p),
+        ("count", ctypes.c_uint32), ("count_ptr", ctypes.c_void_p), ("per_wave", ctypes.c_uint32)]
+
+
+@pytest.mark.parametrize("count,distance,waves", [(15_000, 50, True), (15_000, 80, False), (30_000, 30, True),
+                                                  (30_000, 40, False), (300, 900, True), (1, 1000, True), (0, 0, True)])
+def test_a_sample_of_the_results_picks_the_emit(count, distance, waves):
+    """At 256 CUs a list of 1,500 bp pairs goes by waves while its pairs per CU
+    times its edits a base stay within 2.5."""
+    print(f"case pick {count} pairs of {distance} edits", flush=True)
+    n = max(count, 1)
+    pairs, res = np.zeros(2 * n, dtype=ewfa.PAIR_DTYPE), np.zeros(2 * n, dtype=ewfa.RESULT_DTYPE)
+    pairs["tlen"] = 1500
+    res["distance"], res["status"] = distance, ewfa.PAIR_OK
+    res["distance"][::2], res["status"][1::14] = 1500, ewfa.PAIR_BADARG  # not of the list, and not aligned
+    lst = np.arange(n, dtype=np.uint32) * 2 + 1
+    bufs = [ewfa.DeviceBuffer.from_array(x) for x in (pairs, res, lst, np.array([count, 7, 7], dtype=np.uint32))]
+    args = EmitArgs(pairs=bufs[0].ptr, results=bufs[1].ptr, list=bufs[2].ptr, count=3 * n, count_ptr=bufs[3].ptr)
+    pick = ewfa.lib()._ZN4ewfa16launch_emit_pickERKNS_8EmitArgsEfPjP12ihipStream_t
+    pick.argtypes = [ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_void_p]
+    at = bufs[3].ptr.value if isinstance(bufs[3].ptr, ctypes.c_void_p) else bufs[3].ptr
+    assert pick(ctypes.byref(args), 2.5 * 256, at + 4, None) == 0
+    ewfa.synchronize()
+    got = bufs[3].download(np.uint32, 3)
+    assert got.tolist() == [count, count if waves else 0, 0 if waves else count]
