@@ -1162,7 +1162,12 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
                 x.tok_bytes = ewfa::bp_tok_bytes();
                 const bool probe = p.dcap < BOUND_MIN_DCAP;
                 if (probe) {
-                    HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, p.dcap, ctl + BP_FLAG, q));
+                    ewfa::BpBeside y{};
+                    y.counts = ctrl + CTRL_BCOUNT;
+                    y.nb = F > 1 ? pl.nb : 0;
+                    y.self = b;
+                    for (int i = 0; i < pl.nb; ++i) y.len[i] = pl.pass[i].reg ? 0u : pl.blen[i];
+                    HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, p.dcap, y, ctl + BP_FLAG, q));
                     x.flag = ctl + BP_FLAG;
                 }
                 // a part of a long call may be a short list: both searches are

@@ -854,8 +854,13 @@ __device__ __forceinline__ uint32_t sign_mask(uint32_t planes, int i) { return (
 // The bound, and in `slope` the least growth of the window's middle value over
 // SLOPE_BLOCKS column blocks (the edit rate while the window was on the path;
 // unchanged when the text has fewer).
+// SAMPLE: the edits of the text's first tlen bases against whatever part of the
+// pattern suits them, the least value of the last column (that of row tlen counts
+// the path's distance from the diagonal as edits: half as many again for pairs of
+// 4.5% in runs), and in `slope` the same of the first half of them.
 constexpr int SLOPE_BLOCKS = 32;
 
+template <bool SAMPLE = false>
 __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen, int tlen, int& slope) {
     const int nwp = (plen + 31) >> 5;
     int mid0 = 0;
@@ -878,8 +883,19 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
         const uint32_t q[2] = {__builtin_amdgcn_alignbit(c[1], c[0], (uint32_t)i), __builtin_amdgcn_alignbit(c[2], c[1], (uint32_t)i)};
         return band_column(vp, vn, p, q, sign_mask(t0, i), sign_mask(t1, i));
     };
+    // least value of the column over the pattern's rows
+    const auto least = [&]() -> int {
+        int v = b.sc, m = v;
+        const int rows = min(plen - b.r0, 64);
+        for (int i = 0; i < rows; ++i) {
+            v += (int)((b.vp >> i) & 1u) - (int)((b.vn >> i) & 1u);
+            m = min(m, v);
+        }
+        return m;
+    };
     const int full = tlen >> 5;
     for (int j = 0; j < full; ++j) {
+        if (SAMPLE && j == full / 2) slope = least();
         uint32_t t0, t1;
         load();
         planes_of(gt[j], t0, t1);
@@ -922,6 +938,7 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
         b.vn = (uint64_t)vn[1] << 32 | vn[0];
         b.r0 += rest;
     }
+    if constexpr (SAMPLE) return (uint32_t)least();
     // row plen - 1 of the last column
     const int idx = plen - b.r0;
     if (idx <= 0) return (uint32_t)(b.sc - idx);
@@ -931,46 +948,93 @@ __device__ uint32_t lane_bound(const uint64_t* gp, const uint64_t* gt, int plen,
 
 }  // namespace
 
-// Whether a list takes the bit-parallel way at all, from a sample: 64 of its
-// pairs, a lane each, and the edits in the first PROBE_BASES of each (25 us).  The
-// wavefront's time is its work, or its longest pair's levels (as in bp_way); the
-// bit-parallel one its work, or its longest pair's columns of about 0.35 us (bounds,
-// table and path).  Jobs of 100..5,000 bp at 1..10% edits in batches of 25,000
-// pairs take 5.6 ms by the wavefront and 7.4 bit-parallel, 15,001 pairs of 3..7 kbp
-// at 8..15% 5.9 and 2.9.
+// Whether a list takes the bit-parallel way at all, from a sample: 256 of its
+// pairs, a lane each, and the edits in the first PROBE_BASES of each (35 us).  The
+// wavefront's time is the longer of its work and its longest pair's levels and three
+// quarters of the other, and the levels once more and 2 us each for pairs beyond its
+// budget; the bit-parallel one its work and its longest pair's columns and levels.
+// Over 146 drawn lists of one bucket (1,030..60,000 pairs of 1.3..10.4 kbp at 0.2..15%
+// edits) the median of the time by the estimate is 1.00 and 0.99, and of 210 lists 7
+// went a way more than 6% behind the other.  The ways of 35,000 pairs of 5 kbp at 4%
+// take 2.73 ms (wavefront) and 3.23, 2,500 of 4.3..8.7 kbp at 3..6% in runs
+// 0.86 and 2.36; the other way round 35,000 of 5 kbp at 9% 7.32 and 3.71.
 constexpr int PROBE_BASES = 256;
+constexpr int PROBE_PAIRS = 256;
 constexpr float FEW_LEVELS = 512.0f;
 
-__global__ __launch_bounds__(64) void bp_probe_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
-                                                      uint32_t count, int budget, uint32_t* flag) {
+__global__ __launch_bounds__(PROBE_PAIRS) void bp_probe_kernel(BpArgs a, const uint32_t* list, const uint32_t* count_ptr,
+                                                               uint32_t count, int budget, BpBeside beside,
+                                                               uint32_t* flag) {
     const uint32_t n = count_ptr ? *count_ptr : count;
     if (n == 0) return;
-    const uint32_t item = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) / 128u);
+    __shared__ float part[PROBE_PAIRS / 64][5];
+    // over the block, in every thread: the sums of the first `sums` values, the
+    // greatest of the others
+    const auto join = [&](auto& v, int sums) {
+        constexpr int N = (int)(sizeof v / sizeof v[0]);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            v[i] = i < sums ? wave_add(v[i]) : wave_most(v[i]);
+            if ((threadIdx.x & 63u) == 0u) part[threadIdx.x >> 6][i] = v[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            v[i] = part[0][i];
+            for (int w = 1; w < PROBE_PAIRS / 64; ++w) v[i] = i < sums ? v[i] + part[w][i] : fmaxf(v[i], part[w][i]);
+        }
+    };
+    const uint32_t item = (uint32_t)(((uint64_t)n * (2u * threadIdx.x + 1u)) / (2u * PROBE_PAIRS));
     const uint32_t pidx = list ? list[item] : item;
     const ewfa_pair_t pr = a.pairs[pidx];
-    float edits = 0.f, bases = 0.f, columns = 0.f;
+    float edits = 0.f, second = 0.f, bases = 0.f, columns = 0.f;
     if (pr.plen <= a.max_len && pr.tlen <= a.max_len && pr.tlen > 0u) {
-        const int tl = min((int)pr.tlen, PROBE_BASES), pl = min((int)pr.plen, PROBE_BASES);
-        int slope = 0;
-        edits = (float)lane_bound(a.words + pr.pattern_off, a.words + pr.text_off, pl, tl, slope);
+        const int tl = min((int)pr.tlen, PROBE_BASES);
+        int half = 0;
+        edits = (float)lane_bound<true>(a.words + pr.pattern_off, a.words + pr.text_off, (int)pr.plen, tl, half);
+        second = edits - (float)half;
         bases = (float)tl;
         columns = (float)pr.tlen;
     }
-    // the pairs' rates, drawn to their mean by the share of their variance that few
-    // bases explain (the longest chain is that of a true rate, not of a sample's)
-    const float all = fmaxf(wave_add(bases), 1.f), mean = wave_add(edits) / all;
-    const float off = bases > 0.f ? edits / bases - mean : 0.f;
-    const float var = wave_add(off * off), few = 64.f * 64.f * mean / all;
-    const float rate = fminf(mean + off * (var > few ? 1.f - few / var : 0.f), 2.5f * mean);
-    float levels = rate * columns;
-    const float wfa = wave_add(wavefront_cost(levels, false));
-    const float bp = wave_add(columns * 7.5f + 25.0f * levels);
-    levels = wave_most(levels);
-    columns = wave_most(columns);
+    // the list's rate from the samples' second halves, since an end that is free
+    // to choose saves an edit or two, the first half's as the whole's
+    float s1[3] = {bases, edits, second};
+    join(s1, 3);
+    const float all = fmaxf(s1[0], 1.f), sum = fmaxf(s1[1], 1.f), mean = 2.f * s1[2] / all;
+    // the pairs' rates, drawn to their mean by what the two halves of a sample show
+    // to be the sample's own variance (edits come in runs): each to the likeliest
+    // rate, and for the share of pairs beyond the budget only until the variance is
+    // that of the rates
+    const float off = bases > 0.f ? edits * all / (bases * sum) - 1.f : 0.f;
+    const float diff = bases > 0.f ? (2.f * second - edits) * all / (bases * sum) : 0.f;
+    float s2[2] = {off * off, diff * diff};
+    join(s2, 2);
+    const float keep = s2[0] > s2[1] ? 1.f - s2[1] / s2[0] : 0.f;
+    const float levels = mean * fminf(1.f + off * keep, 2.5f) * columns;
+    const bool beyond = mean * fminf(1.f + off * sqrtf(keep), 2.5f) * columns > (float)budget;
+    // wave instructions of both ways: a two-wave search with its staging and stream
+    // (35,000 pairs of 1.5, 2.4, 3.5 and 5 kbp at 2, 4 and 9% edits within 10%, from 493
+    // us at 1.5 kbp and 2% to 7,322 at 5 kbp and 9%), and bounds, table and path
+    float s3[5] = {levels * (95.0f + 0.29f * levels) + 2.9f * columns, columns * 7.5f + 25.0f * levels,
+                   beyond ? 1.f : 0.f, levels, columns};
+    join(s3, 3);
+    const float most = s3[3], longest = s3[4];
     // wave instructions a microsecond: 256 CUs at about 2.3 GHz
-    const float us = (float)n / 64.0f / 590000.0f;
-    const float chain = levels * (1.1f + 0.0005f * levels) * (levels > (float)budget ? 2.0f : 1.0f);
-    if (threadIdx.x == 0) *flag = fmaxf(bp * us, columns * 0.35f) < fmaxf(wfa * us, chain) ? 1u : 0u;
+    const float share = (float)n / (float)PROBE_PAIRS, us = share / 590000.0f;
+    const float wfa = s3[0] * us, bp = s3[1] * us, deferred = s3[2] >= 3.f ? s3[2] * share : 0.f;
+    const float chain = most * (1.1f + 0.0005f * most) * (deferred > 0.f ? 2.0f : 1.0f);
+    const float wave_us = 1.1f * (fmaxf(wfa, chain) + 0.75f * fminf(wfa, chain)) + 2.0f * deferred;
+    // other buckets' passes of twice this one's bases fill what its columns' chains
+    // leave idle (500,000 pairs of 100..10,000 bp at 1..10%: 15.6 ms with the 80,000 of
+    // 1.2..2.5 kbp by the wavefront, 15.0 without)
+    const float columns_us = 0.2f * longest + 0.5f * most;
+    float others = 0.f;
+    for (int b = 0; b < beside.nb; ++b)
+        if (b != beside.self) others += (float)beside.counts[b] * (float)beside.len[b];
+    const bool hidden = beside.nb > 1 && others >= 2.f * (float)n * (float)beside.len[beside.self];
+    const float bits_us = fmaxf(bp, columns_us) + (hidden ? 0.25f : 1.0f) * fminf(bp, columns_us);
+    if (threadIdx.x == 0) *flag = bits_us < wave_us ? 1u : 0u;
 }
 
 // Splits a list of few long pairs between two passes, by the same sample: all of
@@ -1043,8 +1107,8 @@ hipError_t launch_few_probe(const uint64_t* words, const ewfa_pair_t* pairs, uin
 }
 
 hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
-                           int budget, uint32_t* flag, hipStream_t stream) {
-    hipLaunchKernelGGL(bp_probe_kernel, dim3(1), dim3(64), 0, stream, a, list, count_ptr, count, budget, flag);
+                           int budget, const BpBeside& beside, uint32_t* flag, hipStream_t stream) {
+    hipLaunchKernelGGL(bp_probe_kernel, dim3(1), dim3(PROBE_PAIRS), 0, stream, a, list, count_ptr, count, budget, beside, flag);
     return hipGetLastError();
 }
 

@@ -253,10 +253,17 @@ struct BpArgs {
 // records, per block of 32 columns up to four words a lane of 16 bytes.
 inline size_t bp_tok_bytes() { return 4u * 8u * (size_t)BP_TOK_STRIDE(64) / 4u; }
 inline size_t bp_slot_bytes(uint32_t max_len) { return bp_tok_bytes() + (size_t)(max_len / 32u + 1u) * 64u * 4u * 16u; }
+// The block buckets of a call whose passes run beside each other: their pairs and
+// longest texts (0 of other passes), and the list's own (nb 0: alone).
+struct BpBeside {
+    const uint32_t* counts;
+    uint32_t len[MAX_BUCKETS];
+    int nb, self;
+};
 // *flag = 1 when a sample of the list says the bit-parallel way is the faster
 // (budget: the levels of the wavefront pass).
 hipError_t launch_bp_probe(const BpArgs& a, const uint32_t* list, const uint32_t* count_ptr, uint32_t count,
-                           int budget, uint32_t* flag, hipStream_t stream);
+                           int budget, const BpBeside& beside, uint32_t* flag, hipStream_t stream);
 // counts[0], counts[1]: the list's count for the pass without and the one within
 // distance bounds, one of them 0.
 hipError_t launch_few_probe(const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len, const uint32_t* list,

@@ -329,3 +329,27 @@ def test_a_sample_of_the_results_picks_the_emit(count, distance, waves):
     ewfa.synchronize()
     got = bufs[3].download(np.uint32, 3)
     assert got.tolist() == [count, count if waves else 0, 0 if waves else count]
+
+
+@pytest.mark.parametrize("count,kind,lo,hi,err,bits", [
+    (2500, 2, 4350, 8700, 0.06, False),   # 0.86 ms by the wavefront, 2.36 bit-parallel
+    (2500, 2, 2500, 5000, 0.09, False),   # 0.71 and 1.49
+    (6000, 0, 8700, 8700, 0.13, True),    # 92 (beyond its budget) and 4.1
+    (15000, 0, 5000, 5000, 0.13, True),   # 36 and 3.0
+])
+def test_a_sample_sends_a_list_the_faster_way(count, kind, lo, hi, err, bits):
+    """Lists whose two ways are far apart, beside the same call with a distance
+    cap beyond any distance, which only has the wavefront."""
+    print(f"case sampled {count} pairs of {lo}..{hi} at {err}", flush=True)
+    w = ewfa.Workload(ewfa.synth_spec(kind=kind, seed=5, len=hi, err=err, len_lo=lo, len_hi=hi, err_lo=err / 2,
+                                      err_hi=err), count)
+    case = OnDevice(w.words, w.pairs[:w.n].copy(), w.cigar_bytes, w.max_len)
+    out, took = [], []
+    for cap in (0, 1 << 20):
+        with ewfa.Context(max_distance=cap) as ctx:
+            case.dc.fill_zero()
+            took.append(median_us(lambda: case.align(ctx), 5))
+        out.append((case.dr.download(ewfa.RESULT_DTYPE, count), case.dc.download(np.int8)))
+    assert (out[0][0]["status"] == ewfa.PAIR_OK).all()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert took[0] < (0.5 if bits else 1.35) * took[1], took
