@@ -334,6 +334,7 @@ def test_a_sample_of_the_results_picks_the_emit(count, distance, waves):
 @pytest.mark.parametrize("count,kind,lo,hi,err,bits", [
     (2500, 2, 4350, 8700, 0.06, False),   # 0.86 ms by the wavefront, 2.36 bit-parallel
     (2500, 2, 2500, 5000, 0.09, False),   # 0.71 and 1.49
+    (1450, 2, 4832, 24162, 0.06, False),  # 3.6 and 8.6: weighed by its bounds
     (6000, 0, 8700, 8700, 0.13, True),    # 92 (beyond its budget) and 4.1
     (15000, 0, 5000, 5000, 0.13, True),   # 36 and 3.0
 ])
