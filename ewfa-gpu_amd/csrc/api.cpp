@@ -90,6 +90,8 @@ enum : int {
     CTRL_WORDS = CTRL_BP + ewfa::MAX_BUCKETS * BP_CTRL,
     PLAIN_CTRL = CTRL_XQ + ewfa::XCDS * ewfa::XQ_STRIDE  // words of a plan of one pass
 };
+// the counts of the deferral chain's lists
+constexpr int CHAIN_COUNT[2] = {CTRL_DEFER_A, CTRL_DEFER_B};
 
 }  // namespace
 
@@ -1007,67 +1009,102 @@ int enqueue_main(ewfa_ctx* c, const Pass& p, const uint64_t* words, const ewfa_p
     return EWFA_OK;
 }
 
-// Enqueues a persistent plan: bucketing, one align pass per bucket (longest
-// first), the emit per bucket, and the deferred count's copy to the host.
-// The deferral chain of a plan, then the marking of pairs no pass could
-// resolve.
-// n bounds the deferred pairs.
-int enqueue_chain(ewfa_ctx* c, const Chain& ch, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t n,
-                  uint32_t max_len, ewfa_result_t* results, int8_t* cigars, hipStream_t s) {
+// Pass k of a plan's deferral chain: over the pairs that the pass before deferred
+// (list k & 1), of which n are the most.
+int enqueue_chain_pass(ewfa_ctx* c, const Chain& ch, int k, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t n,
+                       uint32_t max_len, ewfa_result_t* results, int8_t* cigars, hipStream_t s) {
     const ewfa::Scratch sx = scratch_of(c);
     uint32_t* ctrl = sx.ctrl;
     uint32_t* lists[2] = {sx.list_a, sx.list_b};
-    const int ctr[2] = {CTRL_DEFER_A, CTRL_DEFER_B};
-    int cur = 0;
-    for (int k = 0; k < ch.np; ++k) {
-        Pass p = ch.pass[k];
-        p.grid = std::min(p.grid, n);
-        // the pass's queue head, the count of the list it defers into and
-        // its bounds' work counter start at zero (one launch)
-        HIPCHK(ewfa::launch_clear_words(
-            ctrl, (1ull << CTRL_QUEUE) | (1ull << ctr[1 - cur]) | (1ull << CTRL_CHAIN_BQ), s));
-        ewfa::AlignArgs a = base_args(c, words, pairs, results, max_len);
-        fill_pass_args(a, p, c);
-        a.list = lists[cur];
-        a.count = n;
-        a.count_ptr = ctrl + ctr[cur];
-        a.queue = ctrl + CTRL_QUEUE;
-        a.defer_list = lists[1 - cur];
-        a.defer_count = ctrl + ctr[1 - cur];
-        if (p.reg) {
-            HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_XQ, 0u, (size_t)ewfa::XCDS * ewfa::XQ_STRIDE, s));
-            a.xqueue = ctrl + CTRL_XQ;  // (the first bucket's, whose pass has ended)
-            reg_args(a, p, cigars, c);
-            CHK(launch_pass(a, p, s));
-            cur = 1 - cur;
-            continue;
-        }
-        CHK(enqueue_bound(c, a, p, ctrl + CTRL_CHAIN_BQ, n, s));
-        CHK(launch_pass(a, p, s));
-        ewfa::EmitArgs e{};
-        e.words = words;
-        e.pairs = pairs;
-        e.results = results;
-        e.ops = ops_base(c);
-        e.ops_stride = ewfa::ops_words(max_len + 1);
-        e.cigars = cigars;
-        e.list = lists[cur];
-        e.count = n;
-        e.count_ptr = ctrl + ctr[cur];
-        CHK(emit_list(c, e, n, max_len, s));
-        cur = 1 - cur;
+    const int cur = k & 1;
+    Pass p = ch.pass[k];
+    p.grid = std::min(p.grid, n);
+    // the pass's queue head, the count of the list it defers into and
+    // its bounds' work counter start at zero (one launch)
+    HIPCHK(ewfa::launch_clear_words(
+        ctrl, (1ull << CTRL_QUEUE) | (1ull << CHAIN_COUNT[1 - cur]) | (1ull << CTRL_CHAIN_BQ), s));
+    ewfa::AlignArgs a = base_args(c, words, pairs, results, max_len);
+    fill_pass_args(a, p, c);
+    a.list = lists[cur];
+    a.count = n;
+    a.count_ptr = ctrl + CHAIN_COUNT[cur];
+    a.queue = ctrl + CTRL_QUEUE;
+    a.defer_list = lists[1 - cur];
+    a.defer_count = ctrl + CHAIN_COUNT[1 - cur];
+    if (p.reg) {
+        HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_XQ, 0u, (size_t)ewfa::XCDS * ewfa::XQ_STRIDE, s));
+        a.xqueue = ctrl + CTRL_XQ;  // (the first bucket's, whose pass has ended)
+        reg_args(a, p, cigars, c);
+        return launch_pass(a, p, s);
     }
-    HIPCHK(ewfa::launch_mark_too_distant(lists[cur], ctrl + ctr[cur], results, n, s));
+    CHK(enqueue_bound(c, a, p, ctrl + CTRL_CHAIN_BQ, n, s));
+    CHK(launch_pass(a, p, s));
+    ewfa::EmitArgs e{};
+    e.words = words;
+    e.pairs = pairs;
+    e.results = results;
+    e.ops = ops_base(c);
+    e.ops_stride = ewfa::ops_words(max_len + 1);
+    e.cigars = cigars;
+    e.list = lists[cur];
+    e.count = n;
+    e.count_ptr = ctrl + CHAIN_COUNT[cur];
+    return emit_list(c, e, n, max_len, s);
+}
+
+// Marks the pairs that the whole chain deferred: no pass could resolve them.
+int enqueue_chain_end(ewfa_ctx* c, const Chain& ch, uint32_t n, ewfa_result_t* results, hipStream_t s) {
+    const ewfa::Scratch sx = scratch_of(c);
+    HIPCHK(ewfa::launch_mark_too_distant(ch.np & 1 ? sx.list_b : sx.list_a, sx.ctrl + CHAIN_COUNT[ch.np & 1], results, n,
+                                         s));
     return EWFA_OK;
 }
 
-// phase: PLAN_ALL, or PLAN_ALIGN (bucketing, the bucket passes and the emits
-// of the block buckets), after which a call that waits for its results reads
-// whether anything is left for PLAN_EMIT (the fused passes' fallback emit and
-// the deferral chain): most calls defer nothing, and the chain's empty
-// launches (2 to 17 of them, about 4.5 us each) were up to half of a small
-// call.
-enum { PLAN_ALL = 3, PLAN_ALIGN = 1, PLAN_EMIT = 2 };
+// Paths of register passes with a match run of 255 bases or more go through the
+// emit kernel: n at most.
+int enqueue_fallbacks(ewfa_ctx* c, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t n, uint32_t max_len,
+                      ewfa_result_t* results, int8_t* cigars, hipStream_t s) {
+    const ewfa::Scratch sx = scratch_of(c);
+    ewfa::EmitArgs e{};
+    e.words = words;
+    e.pairs = pairs;
+    e.results = results;
+    e.ops = ops_base(c);
+    e.ops_stride = ewfa::ops_words(max_len + 1);
+    e.cigars = cigars;
+    e.list = sx.list_fb;
+    e.count = n;
+    e.count_ptr = sx.ctrl + CTRL_FALLBACK;
+    return emit_list(c, e, n, max_len, s);
+}
+
+// What the bucket passes of a call that waits for its results left over, by the
+// counts they published: the deferral chain a pass at a time, as long as a count
+// says that pairs remain (whole it was up to 17 launches of about 4.5 us, though
+// most deferred pairs end in its first pass), then the fallback emit.
+int finish_call(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t max_len,
+                ewfa_result_t* results, int8_t* cigars, hipStream_t s) {
+    const ewfa::Scratch sx = scratch_of(c);
+    uint32_t deferred = c->host_ctrl[CTRL_DEFER_A];
+    for (int k = 0; k < pl.chain.np && deferred > 0; ++k) {
+        CHK(enqueue_chain_pass(c, pl.chain, k, words, pairs, deferred, max_len, results, cigars, s));
+        const int left = CHAIN_COUNT[(k + 1) & 1];
+        HIPCHK(ewfa::launch_publish_counts(sx.ctrl, left, CTRL_FALLBACK, 0u, c->host_ctrl + left,
+                                           c->host_ctrl + CTRL_FALLBACK, s));
+        HIPCHK(hipStreamSynchronize(s));
+        deferred = c->host_ctrl[left];
+    }
+    if (deferred > 0) CHK(enqueue_chain_end(c, pl.chain, deferred, results, s));
+    if (c->host_ctrl[CTRL_FALLBACK] > 0)
+        CHK(enqueue_fallbacks(c, words, pairs, c->host_ctrl[CTRL_FALLBACK], max_len, results, cigars, s));
+    return EWFA_OK;
+}
+
+// phase: PLAN_ALL, or PLAN_ALIGN (bucketing, the bucket passes, the emits of the
+// block buckets, and the counts of what they left over), after which a call that
+// waits for its results goes on as the counts say (finish_call): most calls
+// defer nothing, and the chain's empty launches were up to half of a small call.
+enum { PLAN_ALL, PLAN_ALIGN };
 
 // The streams (and join events) a plan's bucket passes fan out over beyond
 // the context's own, created on the first plan that has more than one
@@ -1087,9 +1124,11 @@ int ensure_aux(ewfa_ctx* c, int F) {
     return EWFA_OK;
 }
 
+// Enqueues a persistent plan: bucketing, one align pass per bucket (longest
+// first) with its emit, and by phase what follows.
 int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_pair_t* pairs, uint32_t n,
                  uint32_t max_len, ewfa_result_t* results, int8_t* cigars, hipStream_t s, bool timing,
-                 int phase = PLAN_ALL, uint32_t fallbacks = 0xFFFFFFFFu, uint32_t deferred = 0xFFFFFFFFu) {
+                 int phase = PLAN_ALL) {
     const ewfa::Scratch sx = scratch_of(c);
     uint32_t* ctrl = sx.ctrl;
     uint32_t* lists = sx.buckets;
@@ -1097,163 +1136,149 @@ int enqueue_plan(ewfa_ctx* c, const Plan& pl, const uint64_t* words, const ewfa_
     const bool clean = c->ctrl_clean && !c->ext;
     c->ctrl_clean = false;
     const int F = std::max(1, std::min(pl.fanout, ewfa_ctx::MAX_FANOUT));
-    if (phase & PLAN_ALIGN) CHK(ensure_aux(c, F));
+    CHK(ensure_aux(c, F));
     hipStream_t st[ewfa_ctx::MAX_FANOUT] = {s};
     for (int i = 1; i < F; ++i) st[i] = c->aux[i - 1];
     bool fused = false;
     for (int b = 0; b < pl.nb; ++b) fused = fused || pl.pass[b].reg;
-    if (phase & PLAN_ALIGN) {
-        // (still 0 from the call before where that one deferred nothing: one pair
-        // 23.1 -> 20.2 us)
-        if (bucketed || !clean)
-            HIPCHK(ewfa::launch_fill_u32(ctrl, 0u, CTRL_XQ + (size_t)pl.nb * ewfa::XCDS * ewfa::XQ_STRIDE, s));
-        if (pl.bp) HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_BP, 0u, (size_t)pl.nb * BP_CTRL, s));
-        if (bucketed) HIPCHK(ewfa::launch_bucketize(pairs, n, pl.table, lists, ctrl + CTRL_BCOUNT, s));
-        if (timing) HIPCHK(hipEventRecord(c->ev_a0, s));
-        if (F > 1) {
-            HIPCHK(hipEventRecord(c->ev_fork, s));
-            for (int i = 1; i < F; ++i) HIPCHK(hipStreamWaitEvent(st[i], c->ev_fork, 0));
-        }
-        // longest bucket first, the passes dealt over the streams in turn;
-        // each block bucket's emit follows its pass on the same stream
-        int k = 0;
-        for (int b = pl.nb - 1; b >= 0; --b, ++k) {
-            const Pass& p = pl.pass[b];
-            hipStream_t q = st[k % F];
-            ewfa::AlignArgs a = base_args(c, words, pairs, results, max_len);
-            fill_pass_args(a, p, c);
-            a.list = bucketed ? lists + (size_t)b * n : nullptr;
-            a.count = n;
-            a.count_ptr = bucketed ? ctrl + CTRL_BCOUNT + b : nullptr;
-            a.queue = ctrl + CTRL_BQUEUE + b;
-            a.xqueue = ctrl + CTRL_XQ + (size_t)b * ewfa::XCDS * ewfa::XQ_STRIDE;
-            a.defer_list = sx.list_a;
-            a.defer_count = ctrl + CTRL_DEFER_A;
-            a.max_len = pl.blen[b];
-            if (p.reg) reg_args(a, p, cigars, c);
-            const uint32_t* emit_count = nullptr;
-            if (p.bp_grid) {
-                // the bit-parallel pass takes its pairs, the rest stay
-                uint32_t* ctl = ctrl + CTRL_BP + (size_t)b * BP_CTRL;
-                ewfa::BpArgs x{};
-                x.words = words;
-                x.pairs = pairs;
-                x.results = results;
-                x.cigars = cigars;
-                x.max_len = pl.blen[b];
-                x.bound = sx.bound;
-                x.bins = ctl;
-                x.cursors = ctl + ewfa::BP_BINS;
-                x.seg = ctl + BP_SEG;
-                static_assert(CTRL_BP % 2 == 0 && BP_WEIGH % 2 == 0, "64-bit sums");
-                x.weigh = reinterpret_cast<ewfa::BpWeigh*>(ctl + BP_WEIGH);
-                x.list_out = c->bp_list.as<uint32_t>() + (size_t)b * n;
-                x.list = x.list_out;
-                x.rest = c->bp_rest.as<uint32_t>() + (size_t)b * n;
-                x.rest_count = ctl + BP_REST;
-                x.queue = ctl + BP_QUEUE;
-                x.spread = p.bp_spread;
-                x.budget = p.dcap;
-                x.deep = p.dcap >= BOUND_MIN_DCAP;
-                x.defer_list = sx.list_a;
-                x.defer_count = ctrl + CTRL_DEFER_A;
-                x.slots = c->bt.as<uint8_t>() + p.slot_off;  // the pass's own, which runs after
-                x.slot_bytes = p.bp_slot_bytes;
-                x.tok_bytes = ewfa::bp_tok_bytes();
-                const bool probe = p.dcap < BOUND_MIN_DCAP;
-                if (probe) {
-                    ewfa::BpBeside y{};
-                    y.counts = ctrl + CTRL_BCOUNT;
-                    y.nb = F > 1 ? pl.nb : 0;
-                    y.self = b;
-                    for (int i = 0; i < pl.nb; ++i) y.len[i] = pl.pass[i].reg ? 0u : pl.blen[i];
-                    HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, p.dcap, y, ctl + BP_FLAG, q));
-                    x.flag = ctl + BP_FLAG;
-                }
-                // a part of a long call may be a short list: both searches are
-                // launched, and the list's count picks one (20,000 pairs of
-                // 200..20,000 bp at 1..4% edits 5,151 -> 3,964 us; at half the
-                // calls' limit, since lanes give guesses for lost paths too:
-                // 20,000 of 10..50 kbp, 7,500 of them up to 25 kbp, 51.8 -> 44.2 ms)
-                x.lane_min = probe ? 0u : LANE_BOUND_MIN / 2u;
-                a.below = n < LANE_BOUND_MIN ? 0u : LANE_BOUND_MIN / 2u;
-                if (!probe) CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
-                if (probe || n >= LANE_BOUND_MIN) {
-                    x.guess = c->bp_guess.as<uint32_t>();
-                    HIPCHK(ewfa::launch_bp_bound(x, sx.bound, a.list, a.count_ptr, n, (uint32_t)c->num_cus * 16u, q));
-                }
-                HIPCHK(ewfa::launch_bp_sort(x, a.list, a.count_ptr, n, q));
-                for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW})
-                    HIPCHK(ewfa::launch_bp(x, part, p.bp_part[part], q));
-                a.list = x.rest;
-                a.count_ptr = x.rest_count;
-            } else if (pl.free_pass[b].grid) {
-                // a sample sends the list to one of the two passes
-                uint32_t* counts = ctrl + CTRL_BP + (size_t)b * BP_CTRL + BP_QUEUE;
-                HIPCHK(ewfa::launch_few_probe(words, pairs, pl.blen[b], a.list, a.count_ptr, n, counts, q));
-                ewfa::AlignArgs f = a;
-                fill_pass_args(f, pl.free_pass[b], c);
-                f.count_ptr = counts;
-                CHK(launch_pass(f, pl.free_pass[b], q));
-                emit_count = a.count_ptr;
-                a.count_ptr = counts + 1;
-                CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
-            } else {
-                CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
-            }
-            const uint32_t* const emit_items = a.list;
-            if (!pl.free_pass[b].grid) emit_count = a.count_ptr;
-            if (p.band_cap > 0 && a.bound && sx.order) {
-                // the pass takes its pairs by decreasing bound, share by share
-                uint32_t* ord = sx.order + (size_t)b * n;
-                int shift = 0;
-                while ((p.band_cap >> shift) >= ewfa::ORDER_BINS) ++shift;
-                HIPCHK(ewfa::launch_order_by_bound(a.list, a.count_ptr, a.count, a.bound, ord, shift, q));
-                a.list = ord;
-            }
-            CHK(launch_pass(a, p, q));
-            if (!p.reg) {
-                ewfa::EmitArgs e{};
-                e.words = words;
-                e.pairs = pairs;
-                e.results = results;
-                e.ops = ops_base(c);
-                e.ops_stride = ewfa::ops_words(max_len + 1);
-                e.cigars = cigars;
-                e.list = emit_items;
-                e.count = n;
-                e.count_ptr = emit_count;
-                CHK(emit(c, e, n, pl.blen[b], true, q, ctrl + CTRL_EMIT + 2 * b,
-                         b < pl.nb - 1 && pl.pass[pl.nb - 1].band_cap > 0));
-            }
-        }
-        for (int i = 1; i < F; ++i) {
-            HIPCHK(hipEventRecord(c->ev_join[i - 1], st[i]));
-            HIPCHK(hipStreamWaitEvent(s, c->ev_join[i - 1], 0));
-        }
-        if (timing) HIPCHK(hipEventRecord(c->ev_a1, s));
+    // (still 0 from the call before where that one deferred nothing: one pair
+    // 23.1 -> 20.2 us)
+    if (bucketed || !clean)
+        HIPCHK(ewfa::launch_fill_u32(ctrl, 0u, CTRL_XQ + (size_t)pl.nb * ewfa::XCDS * ewfa::XQ_STRIDE, s));
+    if (pl.bp) HIPCHK(ewfa::launch_fill_u32(ctrl + CTRL_BP, 0u, (size_t)pl.nb * BP_CTRL, s));
+    if (bucketed) HIPCHK(ewfa::launch_bucketize(pairs, n, pl.table, lists, ctrl + CTRL_BCOUNT, s));
+    if (timing) HIPCHK(hipEventRecord(c->ev_a0, s));
+    if (F > 1) {
+        HIPCHK(hipEventRecord(c->ev_fork, s));
+        for (int i = 1; i < F; ++i) HIPCHK(hipStreamWaitEvent(st[i], c->ev_fork, 0));
     }
-    if (phase == PLAN_ALIGN)
+    // longest bucket first, the passes dealt over the streams in turn;
+    // each block bucket's emit follows its pass on the same stream
+    int k = 0;
+    for (int b = pl.nb - 1; b >= 0; --b, ++k) {
+        const Pass& p = pl.pass[b];
+        hipStream_t q = st[k % F];
+        ewfa::AlignArgs a = base_args(c, words, pairs, results, max_len);
+        fill_pass_args(a, p, c);
+        a.list = bucketed ? lists + (size_t)b * n : nullptr;
+        a.count = n;
+        a.count_ptr = bucketed ? ctrl + CTRL_BCOUNT + b : nullptr;
+        a.queue = ctrl + CTRL_BQUEUE + b;
+        a.xqueue = ctrl + CTRL_XQ + (size_t)b * ewfa::XCDS * ewfa::XQ_STRIDE;
+        a.defer_list = sx.list_a;
+        a.defer_count = ctrl + CTRL_DEFER_A;
+        a.max_len = pl.blen[b];
+        if (p.reg) reg_args(a, p, cigars, c);
+        const uint32_t* emit_count = nullptr;
+        if (p.bp_grid) {
+            // the bit-parallel pass takes its pairs, the rest stay
+            uint32_t* ctl = ctrl + CTRL_BP + (size_t)b * BP_CTRL;
+            ewfa::BpArgs x{};
+            x.words = words;
+            x.pairs = pairs;
+            x.results = results;
+            x.cigars = cigars;
+            x.max_len = pl.blen[b];
+            x.bound = sx.bound;
+            x.bins = ctl;
+            x.cursors = ctl + ewfa::BP_BINS;
+            x.seg = ctl + BP_SEG;
+            static_assert(CTRL_BP % 2 == 0 && BP_WEIGH % 2 == 0, "64-bit sums");
+            x.weigh = reinterpret_cast<ewfa::BpWeigh*>(ctl + BP_WEIGH);
+            x.list_out = c->bp_list.as<uint32_t>() + (size_t)b * n;
+            x.list = x.list_out;
+            x.rest = c->bp_rest.as<uint32_t>() + (size_t)b * n;
+            x.rest_count = ctl + BP_REST;
+            x.queue = ctl + BP_QUEUE;
+            x.spread = p.bp_spread;
+            x.budget = p.dcap;
+            x.deep = p.dcap >= BOUND_MIN_DCAP;
+            x.defer_list = sx.list_a;
+            x.defer_count = ctrl + CTRL_DEFER_A;
+            x.slots = c->bt.as<uint8_t>() + p.slot_off;  // the pass's own, which runs after
+            x.slot_bytes = p.bp_slot_bytes;
+            x.tok_bytes = ewfa::bp_tok_bytes();
+            const bool probe = p.dcap < BOUND_MIN_DCAP;
+            if (probe) {
+                ewfa::BpBeside y{};
+                y.counts = ctrl + CTRL_BCOUNT;
+                y.nb = F > 1 ? pl.nb : 0;
+                y.self = b;
+                for (int i = 0; i < pl.nb; ++i) y.len[i] = pl.pass[i].reg ? 0u : pl.blen[i];
+                HIPCHK(ewfa::launch_bp_probe(x, a.list, a.count_ptr, n, p.dcap, y, ctl + BP_FLAG, q));
+                x.flag = ctl + BP_FLAG;
+            }
+            // a part of a long call may be a short list: both searches are
+            // launched, and the list's count picks one (20,000 pairs of
+            // 200..20,000 bp at 1..4% edits 5,151 -> 3,964 us; at half the
+            // calls' limit, since lanes give guesses for lost paths too:
+            // 20,000 of 10..50 kbp, 7,500 of them up to 25 kbp, 51.8 -> 44.2 ms)
+            x.lane_min = probe ? 0u : LANE_BOUND_MIN / 2u;
+            a.below = n < LANE_BOUND_MIN ? 0u : LANE_BOUND_MIN / 2u;
+            if (!probe) CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
+            if (probe || n >= LANE_BOUND_MIN) {
+                x.guess = c->bp_guess.as<uint32_t>();
+                HIPCHK(ewfa::launch_bp_bound(x, sx.bound, a.list, a.count_ptr, n, (uint32_t)c->num_cus * 16u, q));
+            }
+            HIPCHK(ewfa::launch_bp_sort(x, a.list, a.count_ptr, n, q));
+            for (int part : {ewfa::BP_ALL, ewfa::BP_WIDE, ewfa::BP_NARROW})
+                HIPCHK(ewfa::launch_bp(x, part, p.bp_part[part], q));
+            a.list = x.rest;
+            a.count_ptr = x.rest_count;
+        } else if (pl.free_pass[b].grid) {
+            // a sample sends the list to one of the two passes
+            uint32_t* counts = ctrl + CTRL_BP + (size_t)b * BP_CTRL + BP_QUEUE;
+            HIPCHK(ewfa::launch_few_probe(words, pairs, pl.blen[b], a.list, a.count_ptr, n, counts, q));
+            ewfa::AlignArgs f = a;
+            fill_pass_args(f, pl.free_pass[b], c);
+            f.count_ptr = counts;
+            CHK(launch_pass(f, pl.free_pass[b], q));
+            emit_count = a.count_ptr;
+            a.count_ptr = counts + 1;
+            CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
+        } else {
+            CHK(enqueue_bound(c, a, p, ctrl + CTRL_BOUNDQ + b, n, q));
+        }
+        const uint32_t* const emit_items = a.list;
+        if (!pl.free_pass[b].grid) emit_count = a.count_ptr;
+        if (p.band_cap > 0 && a.bound && sx.order) {
+            // the pass takes its pairs by decreasing bound, share by share
+            uint32_t* ord = sx.order + (size_t)b * n;
+            int shift = 0;
+            while ((p.band_cap >> shift) >= ewfa::ORDER_BINS) ++shift;
+            HIPCHK(ewfa::launch_order_by_bound(a.list, a.count_ptr, a.count, a.bound, ord, shift, q));
+            a.list = ord;
+        }
+        CHK(launch_pass(a, p, q));
+        if (!p.reg) {
+            ewfa::EmitArgs e{};
+            e.words = words;
+            e.pairs = pairs;
+            e.results = results;
+            e.ops = ops_base(c);
+            e.ops_stride = ewfa::ops_words(max_len + 1);
+            e.cigars = cigars;
+            e.list = emit_items;
+            e.count = n;
+            e.count_ptr = emit_count;
+            CHK(emit(c, e, n, pl.blen[b], true, q, ctrl + CTRL_EMIT + 2 * b,
+                     b < pl.nb - 1 && pl.pass[pl.nb - 1].band_cap > 0));
+        }
+    }
+    for (int i = 1; i < F; ++i) {
+        HIPCHK(hipEventRecord(c->ev_join[i - 1], st[i]));
+        HIPCHK(hipStreamWaitEvent(s, c->ev_join[i - 1], 0));
+    }
+    if (timing) HIPCHK(hipEventRecord(c->ev_a1, s));
+    if (phase == PLAN_ALIGN) {
         HIPCHK(ewfa::launch_publish_counts(ctrl, CTRL_DEFER_A, CTRL_FALLBACK, bucketed ? 0u : PLAIN_CTRL,
                                            c->host_ctrl + CTRL_DEFER_A, c->host_ctrl + CTRL_FALLBACK, s));
-    if (!(phase & PLAN_EMIT)) return EWFA_OK;
-    if (deferred > 0)
-        CHK(enqueue_chain(c, pl.chain, words, pairs, std::min(n, deferred), max_len, results, cigars, s));
-    const bool chain_reg = deferred > 0 && pl.chain.np > 0 && pl.chain.pass[0].reg;
-    if ((fused && fallbacks > 0) || chain_reg) {
-        // paths with a match run of 255 bases or more go through the emit kernel
-        ewfa::EmitArgs e{};
-        e.words = words;
-        e.pairs = pairs;
-        e.results = results;
-        e.ops = ops_base(c);
-        e.ops_stride = ewfa::ops_words(max_len + 1);
-        e.cigars = cigars;
-        e.list = sx.list_fb;
-        e.count = chain_reg ? n : std::min(n, fallbacks);
-        e.count_ptr = ctrl + CTRL_FALLBACK;
-        CHK(emit_list(c, e, e.count, max_len, s));
+        return EWFA_OK;
     }
+    const Chain& ch = pl.chain;
+    for (int k = 0; k < ch.np; ++k) CHK(enqueue_chain_pass(c, ch, k, words, pairs, n, max_len, results, cigars, s));
+    CHK(enqueue_chain_end(c, ch, n, results, s));
+    if (fused || (ch.np > 0 && ch.pass[0].reg)) CHK(enqueue_fallbacks(c, words, pairs, n, max_len, results, cigars, s));
     if (timing) HIPCHK(hipEventRecord(c->ev_e1, s));
     return EWFA_OK;
 }
@@ -2055,9 +2080,7 @@ int ewfa_align_device(ewfa_ctx_t* c, const uint64_t* d_words, const ewfa_pair_t*
         const uint32_t deferred = c->host_ctrl[CTRL_DEFER_A], fallbacks = c->host_ctrl[CTRL_FALLBACK];
         // the counts were published and the control words set back
         if (pl.nb == 1 && !deferred && !fallbacks) c->ctrl_clean = true;
-        if (deferred || fallbacks)
-            CHK(enqueue_plan(c, pl, d_words, d_pairs, (uint32_t)n, max_len, d_results, d_cigars, s, false, PLAN_EMIT,
-                             fallbacks, deferred));
+        if (deferred || fallbacks) CHK(finish_call(c, pl, d_words, d_pairs, max_len, d_results, d_cigars, s));
         if (timing) HIPCHK(hipEventRecord(c->ev_e1, s));
         if (deferred || fallbacks || timing) HIPCHK(hipStreamSynchronize(s));
         if (timing) {
