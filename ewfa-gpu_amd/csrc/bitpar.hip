@@ -108,12 +108,12 @@ struct BpPair {
     int S;               // band: words j + S .. at column block j
 };
 
-// The band's widths over the column blocks: segment k of `n` starts at block
+// The band's widths over the column blocks: segment k starts at block
 // from[k], with w[k] words a lane, its records from row at[k] on (a row: 64
 // lanes of Pv, Mv, then 64 lanes of the horizontal deltas below the word).
 // Uniform over the wave; S[k] is each pair's own.
 struct BpSegs {
-    int n, from[4], w[4], at[4], S[4];
+    int from[4], w[4], at[4], S[4];
 };
 
 __device__ __forceinline__ BpPair bp_load(const BpArgs& a, uint32_t pidx, const ewfa_pair_t& pr, int N) {
@@ -378,7 +378,6 @@ __device__ __forceinline__ void bp_forward(BpPair p, int W, int nblk, uint2* rec
                                            int lane) {
     int sc = -32 * p.S, j = 0, w = W, n_prev = 0, first = 0;
     const uint2* const rec0 = rec;
-    sg.n = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         sg.from[k] = 0x7FFFFFFF;
@@ -390,7 +389,6 @@ __device__ __forceinline__ void bp_forward(BpPair p, int W, int nblk, uint2* rec
         sg.w[k] = w;
         sg.at[k] = (int)((rec - rec0) >> 7);
         sg.S[k] = p.S;
-        sg.n = k + 1;
         int wn = w;
         if (w == 4) j = bp_segment<GL, 4>(p, j, nblk, n_prev, first, sc, rec, wn, lds, lane);
         else if (w == 3) j = bp_segment<GL, 3>(p, j, nblk, n_prev, first, sc, rec, wn, lds, lane);
@@ -715,11 +713,11 @@ __device__ __forceinline__ void bp_item(const BpArgs& a, uint32_t first, uint32_
     bp_forward<GL>(p, W, nblk, rec, sg, reinterpret_cast<uint32_t*>(tiles), lane);
     __threadfence_block();  // the records are read back by other lanes
     int run = 0, cnt = 0;
-    if constexpr (GL < 32) cnt = bp_walk<GL>(p, first + g < end, sg, rec, tok + g * BP_TOK_STRIDE(GL), tiles, run, lane);
+    if constexpr (GL < 32) cnt = bp_walk<GL>(p, first + g < end, sg, rec, tok + g * bp_tok_stride(GL), tiles, run, lane);
     for (uint32_t q = 0; q < 64u / GL && first + q < end; ++q) {
         const int src = (int)q * GL;
         const uint32_t mine = (uint32_t)__builtin_amdgcn_readlane((int)pidx, src);
-        uint32_t* const t = tok + q * BP_TOK_STRIDE(GL);
+        uint32_t* const t = tok + q * bp_tok_stride(GL);
         if constexpr (GL < 32) {
             __threadfence_block();  // the tokens are read back by other lanes
             bp_emit(a, mine, __builtin_amdgcn_readlane(cnt, src), __builtin_amdgcn_readlane(run, src), t, lane);

@@ -248,10 +248,14 @@ struct BpArgs {
 
 // Tokens a pair of a group of gl lanes may have: its band's most edits (below
 // 32 * 4 * gl) and room for a flush.
-#define BP_TOK_STRIDE(gl) (128u * (unsigned)(gl) + 64u)
-// A slot for texts up to max_len bases: the tokens of 64 / gl pairs, then the
-// records, per block of 32 columns up to four words a lane of 16 bytes.
-inline size_t bp_tok_bytes() { return 4u * 8u * (size_t)BP_TOK_STRIDE(64) / 4u; }
+__host__ __device__ constexpr uint32_t bp_tok_stride(int gl) { return 128u * (uint32_t)gl + 64u; }
+// A slot for texts up to max_len bases: the tokens of a wave's 64 / gl pairs, most
+// of them in groups of 8, then the records, per block of 32 columns up to four words
+// a lane of 16 bytes.
+constexpr size_t bp_tok_bytes() { return 4u * 8u * (size_t)bp_tok_stride(8); }
+static_assert(64 / 8 * bp_tok_stride(8) >= 64 / 16 * bp_tok_stride(16) &&
+              64 / 16 * bp_tok_stride(16) >= 64 / 32 * bp_tok_stride(32) &&
+              64 / 32 * bp_tok_stride(32) >= bp_tok_stride(64) && bp_tok_bytes() % 256 == 0, "a wave's tokens");
 inline size_t bp_slot_bytes(uint32_t max_len) { return bp_tok_bytes() + (size_t)(max_len / 32u + 1u) * 64u * 4u * 16u; }
 // The block buckets of a call whose passes run beside each other: their pairs and
 // longest texts (0 of other passes), and the list's own (nb 0: alone).

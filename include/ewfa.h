@@ -196,7 +196,10 @@ int ewfa_align_resident(ewfa_ctx_t *ctx, const ewfa_pair_t *h_pairs, size_t n,
 
 /* Kernel timing of the last ewfa_align_device call on this context, from HIP
  * events recorded on the launch stream: milliseconds in the align kernel(s)
- * and in the CIGAR-emit kernel. */
+ * and in the CIGAR-emit kernel.  On the persistent path the align part holds the
+ * bucket passes with their streams, the emit part what they left over: the
+ * deferral passes and the fallback emit, with the host's look at their counts
+ * (some 10 us where nothing is left). */
 int ewfa_last_timing(ewfa_ctx_t *ctx, float *align_ms, float *emit_ms);
 
 /* Context flags (ewfa_set_flags).  Default: 0 (hipGraph replay of the
